@@ -413,6 +413,7 @@ int advance_stack(Ctx* c, const StepArgs& a, hipStream_t s) {
     ReduceArgs r{};
     r.n = n;
     r.slots = c->grid;
+    r.keep = generic_capture_overwrites(n) ? 1 : 0;
     r.partials_in = static_cast<const double*>(c->d_partials.p);
     r.partials = static_cast<double*>(c->d_partials.p);
     r.obs = static_cast<double*>(c->d_obs.p) + (size_t)a.frame * kQ * n;
@@ -558,6 +559,7 @@ int advance_generic_fft(Ctx* c, const StepArgs& a, hipStream_t s) {
     ReduceArgs r{};
     r.n = n;
     r.slots = c->grid;
+    r.keep = generic_capture_overwrites(n) ? 1 : 0;
     r.partials_in = static_cast<const double*>(c->d_partials.p);
     r.partials = static_cast<double*>(c->d_partials.p);
     r.obs = static_cast<double*>(c->d_obs.p) + (size_t)a.frame * kQ * n;
@@ -923,7 +925,13 @@ int twmc_batch_begin(twmc_ctx* ctx, const twmc_batch_desc* d) {
   const int slots = std::max({c->grid, c->cap_grid, site_sum_chunks(B, kSiteSumChunks, &ss_chunk)});
   size_t part_bytes = (size_t)slots * kQ * n * sizeof(double);
   HIPCHK(c, c->d_partials.ensure(part_bytes));
-  HIPCHK(c, hipMemsetAsync(c->d_partials.p, 0, part_bytes, s));
+  // only the launches that add to their rows need them cleared (168 MB for the
+  // 64x64 ensemble's 1024 slots): the capture inside a step launch, and the
+  // LDS kernel's capture of a lattice above generic_capture_overwrites
+  const bool adds = c->kernel == TWMC_KERNEL_FUSED64 || c->kernel == TWMC_KERNEL_MFMA ||
+                    (c->kernel == TWMC_KERNEL_GENERIC && c->p.hopping == TWMC_HOP_MATRIX) ||
+                    ((c->kernel == TWMC_KERNEL_GENERIC || c->kernel == TWMC_KERNEL_STACK) && !generic_capture_overwrites(n));
+  if (adds) HIPCHK(c, hipMemsetAsync(c->d_partials.p, 0, part_bytes, s));
   size_t nf = std::max<uint64_t>(c->n_frames, 1);
   HIPCHK(c, c->d_obs.ensure(nf * kQ * n * sizeof(double)));
   HIPCHK(c, hipMemsetAsync(c->d_obs.p, 0, nf * kQ * n * sizeof(double), s));

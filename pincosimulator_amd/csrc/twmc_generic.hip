@@ -546,9 +546,9 @@ __global__ void __launch_bounds__(BLOCK) generic_step_kernel(StepArgs g) {
 // |beta|^2 and |beta|^4, the frame dump and, with FFT hopping, |DFT beta|^2.
 // The per-site sums over the workgroup's trajectories stay in registers (each
 // thread owns fixed sites: the pairs tid + BLOCK j and the k-space sites
-// tid + BLOCK j) and are added to the workgroup's partial row once at the
-// end, so every sum takes the same trajectory order as a per-trajectory update
-// of that row; the state is read and not written back.
+// tid + BLOCK j) and become the workgroup's partial row at the end (every
+// entry is written, so nothing clears the rows beforehand); the state is read
+// and not written back.
 // LDS bytes before the state in the capture kernel: two doubles per wave
 constexpr int capture_red_bytes(int block) { return block > 256 ? block / 4 : 64; }
 
@@ -637,19 +637,17 @@ __global__ void __launch_bounds__(BLOCK) generic_capture_kernel(StepArgs g) {
     for (int h = 0; h < 2; ++h) {
       const int i = 2 * p + h;
       if (p < npairs && i < n) {
-        part[i] += accr[2 * j + h][0];
-        part[n + i] += accr[2 * j + h][1];
-        part[3 * n + i] += accr[2 * j + h][2];
-        part[4 * n + i] += accr[2 * j + h][3];
+        part[i] = accr[2 * j + h][0];
+        part[n + i] = accr[2 * j + h][1];
+        part[3 * n + i] = accr[2 * j + h][2];
+        part[4 * n + i] = accr[2 * j + h][3];
       }
     }
   }
-  if (g.hopping == 0) {
 #pragma unroll
-    for (int j = 0; j < 2 * PPT; ++j) {
-      const int i = tid + BLOCK * j;
-      if (i < n) part[2 * n + i] += acck[j];
-    }
+  for (int j = 0; j < 2 * PPT; ++j) {
+    const int i = tid + BLOCK * j;
+    if (i < n) part[2 * n + i] = acck[j];  // zero with matrix hopping
   }
 }
 
@@ -791,34 +789,47 @@ __global__ void __launch_bounds__(256) site_sums_kernel(SiteSumArgs a) {
   if (a.zero_k) part[2 * a.n + i] = 0.0;
 }
 
-__global__ void reduce_kernel(ReduceArgs a) {
+// Folds the slots' partial rows into one frame's sums.  Bound by the latency of
+// its loads: a few hundred outputs (small lattices) of up to ~1000 slots each.
+// A workgroup therefore takes 16 neighbouring outputs and splits their slots
+// over 16 groups of threads (group g sums slots g, g + 16, ... in that order,
+// 16 loads in flight, 128-byte segments), then adds the 16 group sums in order
+// through LDS: every sum has a fixed order, so repeated runs agree bit for bit.
+// One thread per output, all its slots in one chain that also cleared them,
+// took 61 us for 256 slots of a 64-site chain and 189 us for 1000 slots of a
+// 72-site one, against 4.4 and 5.8 us here (64x64, 1024 + 128 slots: 43 against
+// 12 us, 50 MB).
+constexpr int kRedOut = 16, kRedGroups = 16;
+__global__ void __launch_bounds__(kRedOut* kRedGroups) reduce_kernel(ReduceArgs a) {
+  __shared__ double sums[kRedGroups][kRedOut + 1];
   const int total = kQ * a.n;
-  for (int idx = blockIdx.x * blockDim.x + threadIdx.x; idx < total; idx += gridDim.x * blockDim.x) {
-    const int q = idx / a.n, j = idx - q * a.n;
-    const int ns = (q == 2 && a.slots_k > 0) ? a.slots_k : a.slots;
-    double s = 0.0;
-    if (a.keep) {
-      // read-only: 16 loads in flight per thread, the sum still in slot order
-      const double* in = a.partials_in + idx;
-      int sl = 0;
-      for (; sl + 16 <= ns; sl += 16) {
-        double v[16];
+  const int o = threadIdx.x % kRedOut, g = threadIdx.x / kRedOut;
+  const int idx = blockIdx.x * kRedOut + o;
+  double s = 0.0;
+  if (idx < total) {
+    const int ns = (idx / a.n == 2 && a.slots_k > 0) ? a.slots_k : a.slots;
+    const double* in = a.partials_in + idx;
+    int sl = g;
+    for (; sl + 15 * kRedGroups < ns; sl += 16 * kRedGroups) {
+      double v[16];
 #pragma unroll
-        for (int u = 0; u < 16; ++u) v[u] = in[(size_t)(sl + u) * total];
+      for (int u = 0; u < 16; ++u) v[u] = in[(size_t)(sl + u * kRedGroups) * total];
 #pragma unroll
-        for (int u = 0; u < 16; ++u) s += v[u];
-      }
-      for (; sl < ns; ++sl) s += in[(size_t)sl * total];
-    } else {
-      for (int sl = 0; sl < ns; ++sl) {
-        size_t o = (size_t)sl * total + idx;
-        s += a.partials_in[o];
-        a.partials[o] = 0.0;
-      }
+      for (int u = 0; u < 16; ++u) s += v[u];
     }
+    for (; sl < ns; sl += kRedGroups) s += in[(size_t)sl * total];
+    if (!a.keep)
+      for (sl = g; sl < ns; sl += kRedGroups) a.partials[(size_t)sl * total + idx] = 0.0;
+  }
+  sums[g][o] = s;
+  __syncthreads();
+  if (g == 0 && idx < total) {
+    s = 0.0;
+#pragma unroll
+    for (int u = 0; u < kRedGroups; ++u) s += sums[u][o];
+    const int q = idx / a.n, j = idx - q * a.n;
     const int* perm = (q == 2) ? a.perm_k : a.perm_site;
-    int dst = perm ? perm[j] : j;
-    a.obs[q * a.n + dst] = s;
+    a.obs[q * a.n + (perm ? perm[j] : j)] = s;
   }
 }
 
@@ -846,7 +857,7 @@ template <typename T>
 hipError_t launch_generic_p(const StepArgs& a, int grid, int block, size_t lds, hipStream_t s) {
   int ppt = generic_pairs_per_thread(a.n, block);
   // a capture without steps: the capture kernel, its sums in registers
-  if (a.n_steps == 0 && a.capture && block == kBlock && a.n <= 4096) {
+  if (a.n_steps == 0 && a.capture && block == kBlock && generic_capture_overwrites(a.n)) {
     if (a.n > 2048) return launch_generic_capture_t<T, 2, 1024>(a, grid, lds, s);
     if (a.n > 1024) return launch_generic_capture_t<T, 1, 1024>(a, grid, lds, s);
     return ppt == 1 ? launch_generic_capture_t<T, 1, kBlock>(a, grid, lds, s)
@@ -941,6 +952,8 @@ size_t generic_nn_lds_bytes(int nx, int ny, int precision, bool site_uniform) {
 }
 
 int generic_nn_traj_per_block(int n) { return nn_tpb(n); }
+
+bool generic_capture_overwrites(int n) { return n <= 4096; }
 
 hipError_t generic_nn_occupancy(int precision, int nx, int ny, size_t lds, bool site_uniform,
                                 int* blocks_per_cu) {
@@ -1043,10 +1056,8 @@ hipError_t launch_gauss_init(const GaussArgs& a, int precision, int grid, hipStr
 }
 
 hipError_t launch_reduce(const ReduceArgs& a, hipStream_t s) {
-  int total = kQ * a.n;
-  int block = 64;  // one output per thread: small blocks spread the few waves over every CU
-  int grid = (total + block - 1) / block;
-  hipLaunchKernelGGL(reduce_kernel, dim3(grid), dim3(block), 0, s, a);
+  const int grid = (kQ * a.n + kRedOut - 1) / kRedOut;
+  hipLaunchKernelGGL(reduce_kernel, dim3(grid), dim3(kRedOut * kRedGroups), 0, s, a);
   return hipGetLastError();
 }
 

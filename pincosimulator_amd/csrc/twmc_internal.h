@@ -175,6 +175,9 @@ hipError_t launch_generic(const StepArgs& a, int precision, int grid, int block,
                           hipStream_t s);
 size_t generic_lds_bytes(int nx, int ny, int precision);
 int generic_pairs_per_thread(int n, int block);
+// true: a capture-only launch of launch_generic writes every entry of its
+// workgroups' partial rows; false (larger lattices): it adds to them
+bool generic_capture_overwrites(int n);
 // the LDS kernel as a step launch with the hopping in its nearest-neighbour
 // form and no capture (FFT hopping): one LDS copy of the state
 size_t generic_nn_lds_bytes(int nx, int ny, int precision, bool site_uniform);

@@ -80,11 +80,13 @@ struct Ctx {
   int noise[5] = {0, 0, 0, 0, 0};
   // device-resident constants
   DevBuf d_base[5], d_amp[5], d_twx, d_twy, d_kcx, d_kcy, d_cscp, d_cscr, d_cscv, d_perm_site,
-      d_perm_k, d_ahi, d_alo, d_kamp, d_ft_times, d_ft_vals, d_ft_slopes, d_band;
+      d_perm_k, d_ahi, d_alo, d_kamp, d_ft_times, d_ft_vals, d_ft_slopes, d_band,
+      d_ell_coef, d_ell_row;
   int ft_n = 0;  // F(t) table times (0: static F)
   int np = 0;  // padded site count of the MFMA kernel
   int band_w = -1;  // half-width of the coupling matrix (matrix hopping), -1: not banded
   int band_lieb = 0;  // the banded coupling has the Lieb chain's pattern
+  int ell_m = 0;      // TWMC_KERNEL_GENERIC, matrix hopping: entries per column of the sparse kernel, 0: not used
   StackPlan stack;  // TWMC_KERNEL_STACK: the batch's point and work items on the sweep kernel
   // per-batch buffers
   DevBuf d_ids, d_beta, d_rsl, d_U, d_F, d_partials, d_obs, d_m2, d_m4, d_traj, d_prev;
@@ -109,6 +111,7 @@ struct Ctx {
   mutable size_t seg_completed = 0;
   int grid = 0, block = 256;
   int cap_grid = 0;  // stencil64: grid of the capture launch (the 64x64 FFT kernel's)
+  SparsePlan sparse;  // LDS kernel, matrix hopping: its steps on the sparse kernel
   int grid_nn = 0;   // LDS kernel, FFT hopping: grid of the nearest-neighbour step launch
   size_t lds_nn = 0;
   size_t lds = 0;
@@ -429,6 +432,38 @@ int advance_stack(Ctx* c, const StepArgs& a, hipStream_t s) {
   return TWMC_OK;
 }
 
+// matrix hopping with the steps on the sparse kernel: a frame is the LDS
+// kernel's capture-only launch and the reduction, as advance_generic_fft's
+int advance_sparse(Ctx* c, const StepArgs& a, hipStream_t s) {
+  const int n = c->n;
+  if (a.capture) {
+    StepArgs ca = a;
+    ca.n_steps = 0;
+    hipEvent_t r0 = nullptr;
+    HIPCHK(c, timed(c, c->ev_red, s, true, r0));
+    HIPCHK(c, launch_generic(ca, c->precision, c->grid, c->block, c->lds, s));
+    ReduceArgs r{};
+    r.n = n;
+    r.slots = c->grid;
+    r.keep = 1;
+    r.partials_in = static_cast<const double*>(c->d_partials.p);
+    r.partials = static_cast<double*>(c->d_partials.p);
+    r.obs = static_cast<double*>(c->d_obs.p) + (size_t)a.frame * kQ * n;
+    HIPCHK(c, launch_reduce(r, s));
+    HIPCHK(c, timed(c, c->ev_red, s, false, r0));
+  }
+  if (a.n_steps > 0) {
+    StepArgs sa = a;
+    sa.capture = 0;
+    hipEvent_t e0 = nullptr;
+    HIPCHK(c, timed(c, c->ev_step, s, true, e0));
+    HIPCHK(c, launch_sparse(sa, c->precision, c->sparse, s));
+    HIPCHK(c, timed(c, c->ev_step, s, false, e0));
+    c->stats.site_steps += (uint64_t)a.n_steps * (uint64_t)n * c->n_traj;
+  }
+  return TWMC_OK;
+}
+
 // The address of this device's copy of `scratch`, looked up once per device
 // (the device must be current).
 hipError_t scratch_setup(int device) {
@@ -454,6 +489,7 @@ struct Geometry {
   size_t lds = 0;
   int grid_nn = 0;  // LDS kernel with FFT hopping: the step launch without the FFT's second buffer
   size_t lds_nn = 0;
+  SparsePlan sparse;  // LDS kernel with matrix hopping: the step launch on the sparse kernel
 };
 
 int step_geometry(Ctx* c, size_t B, Geometry& geo) {
@@ -486,6 +522,7 @@ int step_geometry(Ctx* c, size_t B, Geometry& geo) {
     geo.block = 256;
     geo.lds = generic_lds_bytes(c->p.nx, c->p.ny, c->precision);
     HIPCHK(c, generic_occupancy(c->precision, c->n, geo.block, geo.lds, &per_cu));
+    if (c->ell_m > 0) HIPCHK(c, sparse_plan(c->n, c->precision, c->ell_m, B, cus, &geo.sparse));
     if (c->p.hopping == TWMC_HOP_FFT) {
       int per_cu_nn = 0;
       geo.lds_nn = generic_nn_lds_bytes(c->p.nx, c->p.ny, c->precision, site_uniform(c));
@@ -541,6 +578,9 @@ StepArgs shared_step_args(const Ctx* c) {
   a.band_coef = static_cast<const float*>(c->d_band.p);
   a.band_w = c->band_w;
   a.band_lieb = c->band_lieb;
+  a.ell_coef = c->d_ell_coef.p;
+  a.ell_row = static_cast<const int*>(c->d_ell_row.p);
+  a.ell_m = c->ell_m;
   return a;
 }
 
@@ -743,6 +783,25 @@ int twmc_create(const twmc_params* p, int device, twmc_ctx** ctx_out) {
     if (ee == hipSuccess) ee = upload(c->d_cscr, row.data(), row.size() * sizeof(int), s);
     if (ee == hipSuccess) (void)up(c->d_cscv, val, false);
     if (ee != hipSuccess) fail_rc = hip_fail(c, ee, "upload coupling");
+    // the LDS kernel's steps on the sparse kernel: FP64, or FP32 with drawn
+    // parameters (with shared ones it stays the LDS product, the banded and
+    // MFMA kernels' independent counterpart), at most six nonzeros a column
+    int most = 0;
+    for (int j = 0; j < c->n; ++j) most = std::max(most, ptr[j + 1] - ptr[j]);
+    if (fail_rc == TWMC_OK && c->kernel == TWMC_KERNEL_GENERIC && (c->precision == 64 || c->noisy_params) &&
+        sparse_supported(c->n, p->hopping, most)) {
+      const int M = c->ell_m = sparse_entries(most);
+      std::vector<int> erow((size_t)c->n * M, -1);
+      std::vector<double> ecoef((size_t)c->n * M, 0.0);
+      for (int j = 0; j < c->n; ++j)
+        for (int e = ptr[j]; e < ptr[j + 1]; ++e) {
+          erow[(size_t)j * M + (e - ptr[j])] = row[e];
+          ecoef[(size_t)j * M + (e - ptr[j])] = (c->precision == 32 ? p->dt : 1.0) * val[e];
+        }
+      ee = upload(c->d_ell_row, erow.data(), erow.size() * sizeof(int), s);
+      if (ee == hipSuccess) ee = up(c->d_ell_coef, ecoef, false);
+      if (ee != hipSuccess && fail_rc == TWMC_OK) fail_rc = hip_fail(c, ee, "upload coupling");
+    }
   }
   if (fail_rc == TWMC_OK && c->ft_n > 0) {
     // F(t) values and per-interval slopes (NoisyMatrix.cpp:228-239); the
@@ -824,6 +883,7 @@ void twmc_destroy(twmc_ctx* ctx) {
   DevBuf* bufs[] = {&c->d_twx,       &c->d_twy,      &c->d_kcx,       &c->d_kcy,  &c->d_cscp, &c->d_cscr,
                     &c->d_cscv,      &c->d_perm_site, &c->d_perm_k,   &c->d_ahi,  &c->d_alo,  &c->d_kamp,
                     &c->d_ft_times,  &c->d_ft_vals,  &c->d_ft_slopes, &c->d_band, &c->d_ids,  &c->d_beta,
+                    &c->d_ell_coef,  &c->d_ell_row,
                     &c->d_rsl,       &c->d_U,        &c->d_F,         &c->d_partials, &c->d_obs, &c->d_m2,
                     &c->d_m4,        &c->d_traj,     &c->d_prev};
   for (DevBuf* b : bufs) b->release();
@@ -893,6 +953,7 @@ int twmc_batch_begin(twmc_ctx* ctx, const twmc_batch_desc* d) {
     c->block = geo.block;
     c->lds = geo.lds;
     c->cap_grid = geo.cap_grid;
+    c->sparse = geo.sparse;
     c->grid_nn = geo.grid_nn;
     c->lds_nn = geo.lds_nn;
   }
@@ -929,7 +990,7 @@ int twmc_batch_begin(twmc_ctx* ctx, const twmc_batch_desc* d) {
   // 64x64 ensemble's 1024 slots): the capture inside a step launch, and the
   // LDS kernel's capture of a lattice above generic_capture_overwrites
   const bool adds = c->kernel == TWMC_KERNEL_FUSED64 || c->kernel == TWMC_KERNEL_MFMA ||
-                    (c->kernel == TWMC_KERNEL_GENERIC && c->p.hopping == TWMC_HOP_MATRIX) ||
+                    (c->kernel == TWMC_KERNEL_GENERIC && c->p.hopping == TWMC_HOP_MATRIX && c->ell_m == 0) ||
                     ((c->kernel == TWMC_KERNEL_GENERIC || c->kernel == TWMC_KERNEL_STACK) && !generic_capture_overwrites(n));
   if (adds) HIPCHK(c, hipMemsetAsync(c->d_partials.p, 0, part_bytes, s));
   size_t nf = std::max<uint64_t>(c->n_frames, 1);
@@ -1046,6 +1107,9 @@ int twmc_batch_advance(twmc_ctx* ctx, uint64_t n_segments) {
         if (rc != TWMC_OK) return rc;
       } else if (c->kernel == TWMC_KERNEL_GENERIC && c->p.hopping == TWMC_HOP_FFT) {
         int rc = advance_generic_fft(c, a, s);
+        if (rc != TWMC_OK) return rc;
+      } else if (c->kernel == TWMC_KERNEL_GENERIC && c->ell_m > 0) {
+        int rc = advance_sparse(c, a, s);
         if (rc != TWMC_OK) return rc;
       } else if (a.n_steps > 0 || a.capture) {
         hipEvent_t e0 = nullptr, e1 = nullptr;
@@ -1309,6 +1373,8 @@ int twmc_advance_noalloc(twmc_ctx* ctx, const uint64_t* d_traj_ids, uint64_t n_t
       HIPCHK(c, launch_mfma(a, geo.grid, s));
     } else if (c->p.hopping == TWMC_HOP_FFT) {
       HIPCHK(c, launch_generic_nn(a, c->precision, geo.grid_nn, geo.lds_nn, s));
+    } else if (c->ell_m > 0) {
+      HIPCHK(c, launch_sparse(a, c->precision, geo.sparse, s));
     } else {
       HIPCHK(c, launch_generic(a, c->precision, geo.grid, geo.block, geo.lds, s));
     }

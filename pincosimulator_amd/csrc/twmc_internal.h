@@ -87,6 +87,11 @@ struct StepArgs {
   int site_uniform;          // 1: rsl, U and F are the same at every site and in every trajectory, F static
   const float* band_coef;    // banded kernel: [64 S][2W + 1] dt C_(j+d) j
   int band_w;                // banded kernel: half-width W
+  // sparse kernel: the first ell_m >= count nonzeros of each column, [n][ell_m],
+  // as C_ij (FP64) or dt C_ij (FP32) and row i (-1: none)
+  const void* ell_coef;
+  const int* ell_row;
+  int ell_m;
   int band_lieb;             // banded kernel: the coupling has the Lieb chain's pattern (S = 6, W = 2)
   // time-dependent drive: F(t) = ft_vals[id] + (t - ft_times[id]) ft_slopes[id]
   // with id the last table time below t (F = ft_vals[0] up to ft_times[0]);
@@ -232,6 +237,20 @@ void band_coefficients(const double* coupling, int n, int w, double dt, float* o
 bool band_lieb_pattern(const float* coef, int n, int w);
 hipError_t launch_band(const StepArgs& a, int grid, hipStream_t s);
 hipError_t band_occupancy(int n, int w, int lieb, int* blocks_per_cu);
+
+// matrix hopping with at most six nonzeros per column (`most`), up to 512 sites:
+// whole trajectories in a wave's registers, FP64 or FP32
+constexpr int kSparseMaxSites = 512;
+struct SparsePlan {
+  int s = 0;  // sites per lane, 0: not planned
+  int grid = 0;
+  size_t lds = 0;
+};
+int sparse_entries(int most);  // entries per column of the kernel's table, 0: too many
+bool sparse_supported(int n, int hopping, int most);
+hipError_t sparse_plan(int n, int precision, int most, size_t n_traj, int cus, SparsePlan* plan);
+hipError_t launch_sparse(const StepArgs& a, int precision, const SparsePlan& plan, hipStream_t s);
+
 hipError_t mfma_occupancy(int np, int* blocks_per_cu);
 // splits A (row-major np x np, FP64) into BF16 hi and lo parts (raw 16-bit)
 void mfma_split(const double* a, size_t count, uint16_t* hi, uint16_t* lo);

@@ -502,7 +502,7 @@ int step_geometry(Ctx* c, size_t B, Geometry& geo) {
     geo.lds = 0;
     HIPCHK(c, fused64_occupancy(&per_cu));
   } else if (c->kernel == TWMC_KERNEL_STENCIL64) {
-    geo.block = 64;
+    geo.block = stencil64_block();
     geo.lds = 0;
     int cap_per_cu = 0;
     HIPCHK(c, capture64_occupancy(&cap_per_cu));
@@ -533,7 +533,7 @@ int step_geometry(Ctx* c, size_t B, Geometry& geo) {
     }
   }
   if (per_cu < 1) return fail(c, TWMC_ERR_UNSUPPORTED, "step kernel does not fit on a CU");
-  if (c->kernel == TWMC_KERNEL_STENCIL64 || c->kernel == TWMC_KERNEL_FUSED64 || c->kernel == TWMC_KERNEL_BAND)
+  if (c->kernel == TWMC_KERNEL_FUSED64 || c->kernel == TWMC_KERNEL_BAND)
     geo.grid = balanced_wave_grid(B, per_cu, cus);
   else
     geo.grid = (int)std::min<size_t>(units, (size_t)per_cu * cus);

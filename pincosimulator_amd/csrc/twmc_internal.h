@@ -202,6 +202,7 @@ hipError_t fused64_occupancy(int* blocks_per_cu);
 void fused64_perms(int* perm_site, int* perm_k);  // [4096] each
 bool stencil64_supported(int nx, int ny, int hopping, int precision, int param_stride);
 hipError_t launch_stencil64(const StepArgs& a, int grid, hipStream_t s);
+int stencil64_block();  // threads per workgroup (one trajectory)
 hipError_t stencil64_occupancy(int* blocks_per_cu);
 
 // matrix hopping on MFMA (FP32 state, BF16 x 3 products, FP32 accumulation)

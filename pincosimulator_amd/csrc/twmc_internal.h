@@ -218,6 +218,7 @@ struct StackPlan {
   void* d_items = nullptr;
   void* d_counter = nullptr;
   int n_items = 0, grid = 0, tb = 1;
+  bool u_real = false;  // Im U = 0
 };
 bool stack_supported(int nx, int ny);
 hipError_t stack_prepare(StackPlan& sp, int nx, int ny, int n_traj, const double rsl[2], const double u[2],

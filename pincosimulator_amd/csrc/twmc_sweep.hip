@@ -40,9 +40,12 @@ namespace twmc {
 
 namespace {
 
-constexpr int kSweepBlock = 256;
+constexpr int kSweepBlock = 256;  // the capture launch
 constexpr int kSweepMaxSites = 4096;  // sites per work item (LDS and registers)
 constexpr int kPPT = kSweepMaxSites / 2 / kSweepBlock;
+constexpr int kStepBlock = 1024;  // the step launch
+constexpr int kStepPairs = kSweepMaxSites / 2;
+constexpr int kStepPPT = kStepPairs / kStepBlock;
 constexpr int kBins = 32;  // radial |k| bins: 0 is k = 0, 1..31 split (0, pi sqrt 2]
 constexpr int kMaxRows = 256;  // stacked trajectories per work item
 constexpr int kMaxNx = 64;     // rows of a 2D point
@@ -94,34 +97,51 @@ __global__ void sweep_reset_kernel(unsigned int* counter) {
 // The item is ntr trajectories of nxt rows each, stacked: 2D points have
 // nxt = nx lattice rows and x-hopping (XHOP), chains one row each and no
 // x-hopping; MULTI = false is the single-trajectory case (one trajectory id
-// for the whole item).  Thread t owns the site pairs p = t + 256 j, sites 2p
+// for the whole item).  Thread t owns the site pairs p = t + 1024 j, sites 2p
 // and 2p + 1 of one row (rows have even length), so the pair's two values are
-// each other's y-neighbours; the other y-neighbours, and the x-neighbours as
-// the 16-byte pairs of the rows above and below in the same trajectory, come
-// from the LDS copy of the state.  The hopping h = -i J S, S the sum over the
+// each other's y-neighbours; the other y-neighbours and the x-neighbours come
+// from the LDS copy of the state: even and odd sites in separate halves, 8 bytes
+// from lane to lane, one copy read and the other written per step (one
+// barrier), two steps per loop pass so that both copies' addresses are a
+// register plus a constant.  The hopping h = -i J S, S the sum over the
 // periodic nearest neighbours, is the exact real-space form of the reference's
 // IDFT(K DFT(beta)) / N (TWMCBaseSolver.cpp:80-88, :235-242); a length-2
 // dimension gives the one neighbour twice, as the FFT form does.
-template <bool XHOP, bool MULTI>
+// UI0: Im U = 0 in every point, so the per-site FMA of the drift's real part
+// drops out.
+template <bool UI0, bool XHOP, bool MULTI>
 __device__ __forceinline__ void step_item(const SweepArgs& g, const SweepPointDev& P, const SweepItemDev& item,
-                                          cpx<float>* bufA, cpx<float> (&beta)[2 * kPPT], int nxt, int ny,
-                                          int npairs) {
+                                          cpx<float>* st, float4* gbeta, int nxt, int ny, int npairs) {
   // neighbour offsets and Philox counters of the owned pairs, fixed for the item
-  int lft[kPPT], rgt[kPPT], up[kPPT], dn[kPPT];
-  uint32_t pid[kPPT];
-  uint64_t trj[kPPT];
-  const uint64_t traj0 = P.traj_id0 + (uint64_t)item.t0;
+  int lft[kStepPPT], rgt[kStepPPT], up[kStepPPT], dn[kStepPPT];
+  uint32_t pid[kStepPPT];
+  uint64_t trj[kStepPPT];
+  cpx<float> beta[2 * kStepPPT];
+  const uint64_t traj0 = g.traj_ids ? g.traj_ids[item.t0] : P.traj_id0 + (uint64_t)item.t0;  // wave-uniform
+  const int yh = ny / 2;
+  const int wave_p = __builtin_amdgcn_readfirstlane(threadIdx.x & ~63);  // first pair of the wave
 #pragma unroll
-  for (int j = 0; j < kPPT; ++j) {
-    const int p = threadIdx.x + kSweepBlock * j;
-    const int row = (2 * p) / ny, col = 2 * p - row * ny;
+  for (int j = 0; j < kStepPPT; ++j) {
+    const int p = threadIdx.x + kStepBlock * j;
+    const int row = p / yh, q = p - row * yh;
     const int tr = MULTI ? row / nxt : 0, r0 = tr * nxt, r = row - r0;
-    lft[j] = row * ny + (col == 0 ? ny - 1 : col - 1);
-    rgt[j] = row * ny + (col + 2 == ny ? 0 : col + 2);
-    up[j] = ((r0 + (r == 0 ? nxt - 1 : r - 1)) * ny + col) / 2;  // pair index
-    dn[j] = ((r0 + (r + 1 == nxt ? 0 : r + 1)) * ny + col) / 2;
-    pid[j] = (uint32_t)(p - tr * (nxt * ny / 2));
-    trj[j] = g.traj_ids ? g.traj_ids[item.t0 + tr] : traj0 + (uint64_t)tr;
+    lft[j] = kStepPairs + row * yh + (q == 0 ? yh - 1 : q - 1);  // an odd site
+    rgt[j] = row * yh + (q + 1 == yh ? 0 : q + 1);               // an even site
+    up[j] = (r0 + (r == 0 ? nxt - 1 : r - 1)) * yh + q;
+    dn[j] = (r0 + (r + 1 == nxt ? 0 : r + 1)) * yh + q;
+    pid[j] = (uint32_t)(p - tr * (nxt * yh));
+    trj[j] = traj0;
+    if (p < npairs) {
+      if (MULTI) trj[j] = g.traj_ids ? g.traj_ids[item.t0 + tr] : traj0 + (uint64_t)tr;
+      const float4 v = gbeta[p];
+      st[p] = beta[2 * j] = mk(v.x, v.y);
+      st[kStepPairs + p] = beta[2 * j + 1] = mk(v.z, v.w);
+    } else {
+      // lanes past the item's end compute along in a wave that has some of it, on
+      // slot 0, and store nothing
+      lft[j] = rgt[j] = up[j] = dn[j] = 0;
+      beta[2 * j] = beta[2 * j + 1] = mk(0.f, 0.f);
+    }
   }
   // step constants: dt (rsl + i U (|b|^2 - 1)) = (A0 - Ui |b|^2) + i (B0 + Ur |b|^2),
   // dt iF = (fr, fi), dt h = -i jdt S, sigma^2 folded into the Box-Muller log multiplier
@@ -131,43 +151,52 @@ __device__ __forceinline__ void step_item(const SweepArgs& g, const SweepPointDe
   const float fr = -dt * P.f_im, fi = dt * P.f_re;
   const float jdt = dt * (-0.5f * P.kscale);  // dt J
   const float nl = -1.3862943611198906f * P.dt4 * P.dt4;
-  float4* pairs = reinterpret_cast<float4*>(bufA);
+  __syncthreads();
 
-  for (int s = 0; s < g.n_steps; ++s) {
+  // one step from copy C of the state to the other
+  auto step_from = [&](auto copy, uint32_t step) __attribute__((always_inline)) {
+    constexpr int C = decltype(copy)::value;
+    const cpx<float>* cur = st + 2 * kStepPairs * C;
+    cpx<float>* nxt_st = st + 2 * kStepPairs * (1 - C);
 #pragma unroll
-    for (int j = 0; j < kPPT; ++j) {
-      const int p = threadIdx.x + kSweepBlock * j;
-      if (p < npairs) pairs[p] = make_float4(beta[2 * j].re, beta[2 * j].im, beta[2 * j + 1].re, beta[2 * j + 1].im);
-    }
-    __syncthreads();
-    const uint32_t step = uint32_t(g.step0 + (uint64_t)s);
+    for (int j = 0; j < kStepPPT; ++j) {
+      const int p = threadIdx.x + kStepBlock * j;
+      if (wave_p + kStepBlock * j < npairs) {
+        const cpx<float> L = cur[lft[j]], R = cur[rgt[j]];
+        cpx<float> u[2], d[2];
+        if (XHOP) {
 #pragma unroll
-    for (int j = 0; j < kPPT; ++j) {
-      const int p = threadIdx.x + kSweepBlock * j;
-      if (p < npairs) {
-        const u32x4 w = philox4x32_10(make_counter(trj[j], TAG_WIENER, step, pid[j]), g.key0, g.key1);
+          for (int h = 0; h < 2; ++h) {
+            u[h] = cur[kStepPairs * h + up[j]];
+            d[h] = cur[kStepPairs * h + dn[j]];
+          }
+        }
+        // opaque per step, so that no Philox round is hoisted out of the loop
+        uint32_t pair = pid[j];
+        asm volatile("" : "+v"(pair));
+        const u32x4 w = MULTI ? philox4x32_10(make_counter(trj[j], TAG_WIENER, step, pair), g.key0, g.key1)
+                              : philox4x32_10_wave(make_counter(traj0, TAG_WIENER, step, pair), g.key0, g.key1);
         float rs[2], cs[2], sn[2];
         box_muller_f32_scaled(w.x, w.y, nl, rs[0], cs[0], sn[0]);
         box_muller_f32_scaled(w.z, w.w, nl, rs[1], cs[1], sn[1]);
         const cpx<float> z0 = beta[2 * j], z1 = beta[2 * j + 1];
-        const cpx<float> L = bufA[lft[j]], R = bufA[rgt[j]];
         float sr[2], si[2];
         sr[0] = z1.re + L.re;
         si[0] = z1.im + L.im;
         sr[1] = R.re + z0.re;
         si[1] = R.im + z0.im;
         if (XHOP) {
-          const float4 u = pairs[up[j]], d = pairs[dn[j]];
-          sr[0] += d.x + u.x;
-          si[0] += d.y + u.y;
-          sr[1] += d.z + u.z;
-          si[1] += d.w + u.w;
+#pragma unroll
+          for (int h = 0; h < 2; ++h) {
+            sr[h] += d[h].re + u[h].re;
+            si[h] += d[h].im + u[h].im;
+          }
         }
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
           const cpx<float> z = h ? z1 : z0;
           const float mq = fmaf(z.im, z.im, z.re * z.re);
-          const float cr = fmaf(-Ui, mq, A0), ci = fmaf(Ur, mq, B0);
+          const float cr = UI0 ? A0 : fmaf(-Ui, mq, A0), ci = fmaf(Ur, mq, B0);
           // increment = noise + dt iF + drift + hopping, all small, added to beta once
           float dr = fmaf(rs[h], cs[h], fr);
           dr = fmaf(cr, z.re, dr);
@@ -179,25 +208,70 @@ __device__ __forceinline__ void step_item(const SweepArgs& g, const SweepPointDe
           di = fmaf(-jdt, sr[h], di);
           beta[2 * j + h] = mk(z.re + dr, z.im + di);
         }
+        if (p < npairs) {
+          nxt_st[p] = beta[2 * j];
+          nxt_st[kStepPairs + p] = beta[2 * j + 1];
+        }
       }
     }
     __syncthreads();
+  };
+  int s = 0;
+  for (; s + 2 <= g.n_steps; s += 2) {
+    step_from(std::integral_constant<int, 0>{}, uint32_t(g.step0 + (uint64_t)s));
+    step_from(std::integral_constant<int, 1>{}, uint32_t(g.step0 + (uint64_t)s + 1));
+  }
+  if (s < g.n_steps) step_from(std::integral_constant<int, 0>{}, uint32_t(g.step0 + (uint64_t)s));
+#pragma unroll
+  for (int j = 0; j < kStepPPT; ++j) {
+    const int p = threadIdx.x + kStepBlock * j;
+    if (p < npairs) gbeta[p] = make_float4(beta[2 * j].re, beta[2 * j].im, beta[2 * j + 1].re, beta[2 * j + 1].im);
   }
 }
 
-// Built for three waves per SIMD (three 256-thread workgroups per CU, at most
-// 168 VGPRs; a 512-point sweep frame 42.5 -> 34.8 ms against two workgroups
-// per CU at 204 VGPRs; four per CU spill and lose on stacked 2D items).
-template <bool CAPTURE_ONLY>
-__global__ void __launch_bounds__(kSweepBlock, 3) sweep_step_kernel(SweepArgs g) {
+// The step launch: 1024-thread workgroups, up to two site pairs per thread, 64
+// registers for eight waves per SIMD (the transcendental instructions then run
+// beside the others, as in the 64x64 kernel).
+// Bound by VALU issue: 45.6 instructions per site-step (2D; chains 43.5), four of
+// them transcendental.  A 512-point sweep frame 35.8 -> 32.3 ms against 256-thread
+// workgroups of up to eight pairs per thread (168 registers, three waves per
+// SIMD); one-system batches of 16384 trajectories, us per step: 16x16 6.55 -> 5.15,
+// 36x50 39.2 -> 33.1, 48x48 45.7 -> 41.1, 1x512 10.2 -> 8.8 (9.5e11 site-steps/s),
+// and of 32: 16x16 1.27 -> 0.41, 48x48 1.70 -> 0.84.
+template <bool UI0>
+__global__ void __launch_bounds__(kStepBlock, 8) sweep_step_kernel(SweepArgs g) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  int& s_item = *reinterpret_cast<int*>(smem);
+  cpx<float>* st = reinterpret_cast<cpx<float>*>(smem + 64);  // [2 copies][even, odd][pairs]
+  for (;;) {
+    __syncthreads();
+    if (threadIdx.x == 0) s_item = (int)atomicAdd(g.counter, 1u);
+    __syncthreads();
+    const int it = __builtin_amdgcn_readfirstlane(s_item);
+    if (it >= g.n_items) break;  // every workgroup reaches this once the queue is drained
+    const SweepItemDev item = g.items[it];
+    const SweepPointDev& P = g.points[item.point];
+    const int ntr = min(P.tb, P.n_traj - item.t0);
+    const int nxt = P.fft_x ? P.nx : 1, ny = P.ny;  // rows per trajectory
+    const int npairs = ntr * nxt * ny / 2;          // ny is even for every supported size
+    float4* gbeta = reinterpret_cast<float4*>(g.beta + P.state_off + (size_t)item.t0 * nxt * ny);
+    if (!P.fft_x)
+      step_item<UI0, false, true>(g, P, item, st, gbeta, 1, ny, npairs);
+    else if (ntr == 1)
+      step_item<UI0, true, false>(g, P, item, st, gbeta, nxt, ny, npairs);
+    else
+      step_item<UI0, true, true>(g, P, item, st, gbeta, nxt, ny, npairs);
+  }
+}
+
+// The frame's capture launch: per-trajectory means, mean field and k-space bins.
+__global__ void __launch_bounds__(kSweepBlock) sweep_capture_kernel(SweepArgs g) {
   extern __shared__ __align__(16) unsigned char smem[];
   double* red = reinterpret_cast<double*>(smem);  // [8]
   cpx<float>* bufA = reinterpret_cast<cpx<float>*>(smem + 64);
   cpx<float>* bufB = bufA + kSweepMaxSites;
   cpx<float>* twx = bufB + kSweepMaxSites;    // [kMaxNx]
   cpx<float>* twy = twx + kMaxNx;             // [kMaxNy]
-  float* kcx = reinterpret_cast<float*>(twy + kMaxNy);  // [kMaxNx]
-  float* kcy = kcx + kMaxNx;                  // [kMaxNy]
   __shared__ int s_item;
   __shared__ double s_bins[kBins + 2];
 
@@ -209,26 +283,17 @@ __global__ void __launch_bounds__(kSweepBlock, 3) sweep_step_kernel(SweepArgs g)
     if (it >= g.n_items) break;  // every workgroup reaches this once the queue is drained
     const SweepItemDev item = g.items[it];
     const SweepPointDev P = g.points[item.point];
-    // trajectories in the item: the step launch stacks P.tb of every point,
-    // the capture launch takes 2D points one trajectory at a time
-    const int ntr = (CAPTURE_ONLY && P.fft_x) ? 1 : min(P.tb, P.n_traj - item.t0);
+    // trajectories in the item: 2D points one at a time, chains stacked as rows
+    const int ntr = P.fft_x ? 1 : min(P.tb, P.n_traj - item.t0);
     const int nxt = P.fft_x ? P.nx : 1;        // rows per trajectory
     const int rows_traj = P.fft_x ? 1 : ntr;  // chains: one trajectory per row
     const int nx = nxt * ntr;                  // rows of the item array
     const int ny = P.ny;
     const int m = nx * ny;
     const int npairs = m / 2;  // ny is even for every supported size
-    if (CAPTURE_ONLY) {  // FFT tables, for the frame's k-space sums only
-      for (int i = threadIdx.x; i < ny; i += blockDim.x) {
-        twy[i] = g.tw_pool[P.tw_y + i];
-        kcy[i] = g.kc_pool[P.kc_y + i];
-      }
-      if (P.fft_x)
-        for (int i = threadIdx.x; i < P.nx; i += blockDim.x) {
-          twx[i] = g.tw_pool[P.tw_x + i];
-          kcx[i] = g.kc_pool[P.kc_x + i];
-        }
-    }
+    for (int i = threadIdx.x; i < ny; i += blockDim.x) twy[i] = g.tw_pool[P.tw_y + i];
+    if (P.fft_x)
+      for (int i = threadIdx.x; i < P.nx; i += blockDim.x) twx[i] = g.tw_pool[P.tw_x + i];
     __syncthreads();
 
     // the item's state: this thread's pairs p = t + 256 j in registers
@@ -244,31 +309,7 @@ __global__ void __launch_bounds__(kSweepBlock, 3) sweep_step_kernel(SweepArgs g)
       }
     };
 
-    if constexpr (!CAPTURE_ONLY) {
-      // the step launch: no capture, neither bufB nor the FFT tables.  Each
-      // kind of item loads, steps and stores its own copy of the state, so no
-      // register array is live across the three bodies (one shared copy made
-      // the register allocator spill ~26 values per lane at this occupancy)
-      auto run = [&](auto xhop, auto multi, int rows) __attribute__((always_inline)) {
-        cpx<float> beta[2 * kPPT];
-        load_state(beta);
-        step_item<decltype(xhop)::value, decltype(multi)::value>(g, P, item, bufA, beta, rows, ny, npairs);
-#pragma unroll
-        for (int j = 0; j < kPPT; ++j) {
-          const int p = threadIdx.x + kSweepBlock * j;
-          if (p < npairs) {
-            gbeta[2 * p] = beta[2 * j];
-            gbeta[2 * p + 1] = beta[2 * j + 1];
-          }
-        }
-      };
-      if (!P.fft_x)
-        run(std::false_type{}, std::true_type{}, 1);
-      else if (ntr == 1)
-        run(std::true_type{}, std::false_type{}, nxt);
-      else
-        run(std::true_type{}, std::true_type{}, nxt);
-    } else {
+    {
       cpx<float> beta[2 * kPPT];
       load_state(beta);
       // the capture launch records the frame: per-trajectory means, mean
@@ -403,10 +444,24 @@ __global__ void sweep_init_kernel(const SweepPointDev* points, int n_points, con
   }
 }
 
-// dynamic LDS: the capture launch holds bufA, bufB and the FFT tables; the
-// step launch only bufA (so more workgroups fit on a CU)
-size_t sweep_lds_bytes(bool capture) {
-  return capture ? 64 + 2 * kSweepMaxSites * 8 + (kMaxNx + kMaxNy) * (8 + 4) : 64 + kSweepMaxSites * 8;
+const void* step_kernel(bool u_real) {
+  return u_real ? (const void*)sweep_step_kernel<true> : (const void*)sweep_step_kernel<false>;
+}
+
+// dynamic LDS: two copies of an item's state, the capture launch the FFT tables too
+size_t sweep_lds_bytes(bool capture) { return 64 + 2 * kSweepMaxSites * 8 + (capture ? (kMaxNx + kMaxNy) * 8 : 0); }
+
+// a step launch's LDS limit (above the default 64 KB) and its workgroups per CU
+hipError_t step_occupancy(bool u_real, int* per_cu) {
+  const int lds = (int)sweep_lds_bytes(false);
+  hipError_t e = hipFuncSetAttribute(step_kernel(u_real), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+  if (e == hipSuccess) e = hipOccupancyMaxActiveBlocksPerMultiprocessor(per_cu, step_kernel(u_real), kStepBlock, lds);
+  return e;
+}
+
+hipError_t launch_step(const SweepArgs& a, bool u_real, int grid, hipStream_t s) {
+  void* args[] = {const_cast<SweepArgs*>(&a)};
+  return hipLaunchKernel(step_kernel(u_real), dim3(grid), dim3(kStepBlock), args, sweep_lds_bytes(false), s);
 }
 
 }  // namespace
@@ -427,6 +482,7 @@ struct SweepCtx {
   std::vector<twmc_sweep_point> pts;
   std::vector<SweepPointDev> dev_pts;
   std::vector<int> tb;  // trajectories per work item, per point
+  bool u_real = true;   // Im U = 0 in every point
   std::vector<cpx<float>> tw_pool;
   std::vector<float> kc_pool;
   std::vector<unsigned char> bin_pool;
@@ -527,15 +583,15 @@ hipError_t launch_segment(SweepCtx* c, const SweepArgs& a) {
     ca.counter = (unsigned int*)c->d_counter;
     ca.items = (const SweepItemDev*)c->d_items_cap;
     ca.n_items = c->n_items_cap;
-    hipLaunchKernelGGL(sweep_step_kernel<true>, dim3(c->grid_cap), dim3(kSweepBlock), sweep_lds_bytes(true), c->stream,
+    hipLaunchKernelGGL(sweep_capture_kernel, dim3(c->grid_cap), dim3(kSweepBlock), sweep_lds_bytes(true), c->stream,
                        ca);
   }
   if (a.n_steps > 0) {
     SweepArgs sa = a;
     sa.capture = 0;
     sa.counter = (unsigned int*)c->d_counter + 1;
-    hipLaunchKernelGGL(sweep_step_kernel<false>, dim3(c->grid), dim3(kSweepBlock), sweep_lds_bytes(false), c->stream,
-                       sa);
+    hipError_t e = launch_step(sa, c->u_real, c->grid, c->stream);
+    if (e != hipSuccess) return e;
   }
   return hipGetLastError();
 }
@@ -588,7 +644,6 @@ hipError_t stack_prepare(StackPlan& sp, int nx, int ny, int n_traj, const double
   P.nx = nx;
   P.ny = ny;
   P.fft_x = nx > 1 ? 1 : 0;
-  P.tb = std::max(1, std::min({n_traj, 2048 / (nx * ny), kMaxRows}));
   P.rsl_re = float(rsl[0]);
   P.rsl_im = float(rsl[1]);
   P.u_re = float(u[0]);
@@ -598,17 +653,25 @@ hipError_t stack_prepare(StackPlan& sp, int nx, int ny, int n_traj, const double
   P.dt4 = float(dt4);
   P.kscale = float(kscale);
   P.n_traj = n_traj;
+  int dev = 0, cus = 0, per_cu = 0;
+  hipError_t e = hipGetDevice(&dev);
+  if (e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
+  sp.u_real = u[1] == 0.0;
+  if (e == hipSuccess) e = step_occupancy(sp.u_real, &per_cu);
+  if (e != hipSuccess) return e;
+  // Trajectories per item: about 2048 sites, one pair per thread, when the batch
+  // fills every workgroup slot of the chip (16x16 x 128 sweep points: 6.5e11
+  // site-steps/s with 2048 sites, 6.1e11 with 1024 and 6.2e11 with 4096), and no
+  // more than it takes to give every slot an item: a few trajectories then run
+  // side by side on as many CUs (8x16 x 32: 0.37 us per step one to an item,
+  // 0.70 stacked sixteen to an item).
+  const int slots = std::max(1, per_cu) * cus;
+  P.tb = std::max(1, std::min({(n_traj + slots - 1) / slots, 2048 / (nx * ny), kMaxRows}));
   std::vector<SweepItemDev> items;
   for (int t0 = 0; t0 < n_traj; t0 += P.tb) items.push_back(SweepItemDev{0, t0});
   sp.n_items = (int)items.size();
   sp.tb = P.tb;
-  int dev = 0, cus = 0, per_cu = 0;
-  hipError_t e = hipGetDevice(&dev);
-  if (e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-  if (e == hipSuccess)
-    e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void*)sweep_step_kernel<false>, kSweepBlock,
-                                                     sweep_lds_bytes(false));
-  sp.grid = std::max(1, std::min(sp.n_items, std::max(1, per_cu) * cus));
+  sp.grid = std::min(sp.n_items, slots);
   if (e == hipSuccess) e = hipMalloc(&sp.d_point, sizeof(SweepPointDev));
   if (e == hipSuccess) e = hipMalloc(&sp.d_items, items.size() * sizeof(SweepItemDev));
   if (e == hipSuccess) e = hipMalloc(&sp.d_counter, 2 * sizeof(unsigned int));
@@ -633,8 +696,7 @@ hipError_t stack_launch(const StackPlan& sp, const StepArgs& a, hipStream_t s) {
   g.n_steps = a.n_steps;
   g.traj_ids = a.traj_ids;
   hipLaunchKernelGGL(sweep_reset_kernel, dim3(1), dim3(64), 0, s, (unsigned int*)sp.d_counter);
-  hipLaunchKernelGGL(sweep_step_kernel<false>, dim3(sp.grid), dim3(kSweepBlock), sweep_lds_bytes(false), s, g);
-  return hipGetLastError();
+  return launch_step(g, sp.u_real, sp.grid, s);
 }
 
 void stack_release(StackPlan& sp) {
@@ -705,6 +767,7 @@ int twmc_sweep_create(const twmc_sweep_point* pts, uint64_t n_points, double dt,
     P.rsl_im = float(-q.omega[0]);
     P.u_re = float(q.U[0]);
     P.u_im = float(q.U[1]);
+    if (q.U[1] != 0.0) c->u_real = false;
     P.f_re = float(q.F[0]);
     P.f_im = float(q.F[1]);
     P.dt4 = float(std::sqrt(q.gamma * dt / 4.0));
@@ -747,11 +810,10 @@ int twmc_sweep_create(const twmc_sweep_point* pts, uint64_t n_points, double dt,
   if (e == hipSuccess) e = hipMemcpy(c->d_tw, c->tw_pool.data(), c->tw_pool.size() * sizeof(cpx<float>), hipMemcpyHostToDevice);
   if (e == hipSuccess) e = hipMemcpy(c->d_kc, c->kc_pool.data(), c->kc_pool.size() * sizeof(float), hipMemcpyHostToDevice);
   if (e == hipSuccess) e = hipMemcpy(c->d_binit, binit.data(), binit.size() * 8, hipMemcpyHostToDevice);
-  if (e == hipSuccess) e = hipFuncSetAttribute((const void*)sweep_step_kernel<false>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)sweep_lds_bytes(false));
-  if (e == hipSuccess) e = hipFuncSetAttribute((const void*)sweep_step_kernel<true>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)sweep_lds_bytes(true));
+  if (e == hipSuccess) e = hipFuncSetAttribute((const void*)sweep_capture_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)sweep_lds_bytes(true));
   int per_cu = 0, per_cu_cap = 0, cus = 0;
-  if (e == hipSuccess) e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void*)sweep_step_kernel<false>, kSweepBlock, sweep_lds_bytes(false));
-  if (e == hipSuccess) e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu_cap, (const void*)sweep_step_kernel<true>, kSweepBlock, sweep_lds_bytes(true));
+  if (e == hipSuccess) e = step_occupancy(c->u_real, &per_cu);
+  if (e == hipSuccess) e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu_cap, (const void*)sweep_capture_kernel, kSweepBlock, sweep_lds_bytes(true));
   if (e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device);
   if (e != hipSuccess) {
     std::string m = std::string("sweep setup: ") + hipGetErrorString(e);
@@ -902,7 +964,7 @@ int twmc_sweep_run(twmc_sweep_ctx* ctx, double t_start, double t_end, int32_t us
   for (size_t p = 0; p < c->pts.size(); ++p)
     c->stats.site_steps += (uint64_t)c->dev_pts[p].n_traj * c->dev_pts[p].nx * c->dev_pts[p].ny * i_step;
   c->stats.grid = c->grid;
-  c->stats.block = kSweepBlock;
+  c->stats.block = kStepBlock;
   c->stats.lds_bytes = (int)sweep_lds_bytes(false);
   if (kernel_ms) *kernel_ms = ms;
   if (n_frames_out) *n_frames_out = frames;

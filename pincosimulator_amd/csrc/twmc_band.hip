@@ -29,6 +29,18 @@ __device__ __forceinline__ float from_next_lane(float v) {
   return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), 0x134, 0xf, 0xf, true));
 }
 
+// The W sites at either end of every lane's block, in the wave's LDS.
+template <int W>
+struct alignas(W == 2 ? 16 : 8) Edge {
+  cpx<float> v[W];
+};
+
+// order of the wave's own LDS accesses (the hardware runs them in order)
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
 // the Lieb chain's bonds as offsets d of the coupled site j + d, by the site
 // index mod 3 (A_i = 3i, B_i = 3i + 1, C_i = 3i + 2; TWMCLiebSolver.cpp:52-85):
 // A-B (+1); B-A (-1), B-C (+1), B-C of the previous cell (-2); C-B (-1),
@@ -40,10 +52,34 @@ __host__ __device__ constexpr bool lieb_bond(int r, int d) {
 // LIEB (S = 6, W = 2): each lane's six sites are two whole cells, so the
 // offsets without a bond are known per register and their multiplications
 // by zero are left out (6 of the 10 complex products per cell remain)
-template <int S, int W, bool FT, bool LIEB>
-__global__ void __launch_bounds__(64) band_step_kernel(StepArgs g) {
+// UNI: Re rsl, F and a real U are the same at every site, so of the site tables
+// only Im rsl (the on-site energies) takes registers, and 64 of them hold the
+// kernel at eight waves per SIMD.
+// DENSE: more than two waves per SIMD.  Bound by VALU issue: 41 instructions per
+// site-step of the 384-site Lieb chain, 37 beside the transcendental ones, which
+// have a unit of their own.  Free-running waves bunch up before that unit and
+// leave the VALU idle; raising a wave's priority while it forms its Box-Muller
+// samples keeps the unit fed (384 sites x 8192 trajectories, us per step: 3.55
+// without, 3.20 with; two sites per lane, one pair per step, do not bunch and
+// take no priority: 126 sites x 16384 2.63 without, 2.65 with).  The lanes' edge
+// sites go through LDS, two writes and two reads instead of 4 W DPP moves (x
+// 16384: 6.20 -> 6.13, 126 sites 2.77 -> 2.63).  Otherwise, bound by the latency
+// of a step: DPP and no priority (384 sites x 1000: 0.57 against 0.68 us).
+// Before, 99 registers and the latency form for all: 384 sites x 8192 3.69, x
+// 16384 7.16 us per step (8.8e11 -> 1.03e12 site-steps/s).
+// waves per SIMD that the uniform form's registers allow without spills
+constexpr int uni_waves(int s, int w, bool lieb) {
+  return s == 2 || lieb ? 8 : s == 4 ? (w <= 2 ? 7 : 6) : s == 6 ? (w == 1 ? 7 : 5) : w == 1 ? 5 : 4;
+}
+template <int S, int W, bool FT, bool LIEB, bool UNI, bool DENSE>
+__global__ void __launch_bounds__(64, UNI ? uni_waves(S, W, LIEB) : 1) band_step_kernel(StepArgs g) {
   static_assert(!LIEB || (S == 6 && W == 2), "the Lieb pattern needs two cells per lane");
+  static_assert(!UNI || !FT, "F(t) is per site");
+  static_assert(!DENSE || !FT, "F(t) runs the latency form");
+  constexpr bool LDSX = DENSE, PRIO = DENSE && S >= 4;
   constexpr int D = 2 * W + 1;
+  constexpr int SP = UNI ? 1 : S;  // entries of a uniform table
+  __shared__ Edge<W> first[64], last[64];
   const int lane = threadIdx.x;
   const int n = g.n;
   const int base = lane * S;
@@ -53,7 +89,7 @@ __global__ void __launch_bounds__(64) band_step_kernel(StepArgs g) {
   // this lane's coefficients and site tables; the site parameters are shared
   // by all trajectories (the kernel is chosen only then):
   //   dt (rsl + i U (|b|^2 - 1)) = (A0 - Ui |b|^2) + i (B0 + Ur |b|^2), dt i F = (fr, fi)
-  float cf[S][D], A0[S], B0[S], Ur[S], Ui[S], fr[S], fi[S];
+  float cf[S][D], A0[SP], B0[S], Ur[SP], Ui[SP], fr[SP], fi[SP];
 #pragma unroll
   for (int s = 0; s < S; ++s) {
     const int j = base + s;
@@ -63,12 +99,23 @@ __global__ void __launch_bounds__(64) band_step_kernel(StepArgs g) {
     const cpx<float> r = live ? reinterpret_cast<const cpx<float>*>(g.rsl)[j] : mk(0.f, 0.f);
     const cpx<float> u = live ? reinterpret_cast<const cpx<float>*>(g.U)[j] : mk(0.f, 0.f);
     const cpx<float> f = live ? reinterpret_cast<const cpx<float>*>(g.F)[j] : mk(0.f, 0.f);
-    A0[s] = dt * (r.re + u.im);
     B0[s] = dt * (r.im - u.re);
-    Ur[s] = dt * u.re;
-    Ui[s] = dt * u.im;
-    fr[s] = -dt * f.im;
-    fi[s] = dt * f.re;
+    if constexpr (!UNI) {
+      A0[s] = dt * (r.re + u.im);
+      Ur[s] = dt * u.re;
+      Ui[s] = dt * u.im;
+      fr[s] = -dt * f.im;
+      fi[s] = dt * f.re;
+    }
+  }
+  if constexpr (UNI) {
+    const cpx<float> r = reinterpret_cast<const cpx<float>*>(g.rsl)[0], u = reinterpret_cast<const cpx<float>*>(g.U)[0],
+                     f = reinterpret_cast<const cpx<float>*>(g.F)[0];
+    A0[0] = dt * (r.re + u.im);
+    Ur[0] = dt * u.re;
+    Ui[0] = 0.f;
+    fr[0] = -dt * f.im;
+    fi[0] = dt * f.re;
   }
 
   for (int b = blockIdx.x; b < g.n_traj; b += gridDim.x) {
@@ -132,18 +179,31 @@ __global__ void __launch_bounds__(64) band_step_kernel(StepArgs g) {
       } else {
 #pragma unroll
         for (int s = 0; s < S; ++s) {
-          dr[s] = fr[s];
-          di[s] = fi[s];
+          dr[s] = fr[UNI ? 0 : s];
+          di[s] = fi[UNI ? 0 : s];
         }
       }
       // old values of the W sites before and after this lane's block
-      float lre[W], lim[W], rre[W], rim[W];
+      Edge<W> el, er;
+      if constexpr (LDSX) {
+        Edge<W> e0, e1;
 #pragma unroll
-      for (int k = 0; k < W; ++k) {
-        lre[k] = from_prev_lane(br[S - W + k]);
-        lim[k] = from_prev_lane(bi[S - W + k]);
-        rre[k] = from_next_lane(br[k]);
-        rim[k] = from_next_lane(bi[k]);
+        for (int k = 0; k < W; ++k) {
+          e0.v[k] = mk(br[k], bi[k]);
+          e1.v[k] = mk(br[S - W + k], bi[S - W + k]);
+        }
+        first[lane] = e0;
+        last[lane] = e1;
+        wave_sync();
+        el = last[(lane - 1) & 63];
+        er = first[(lane + 1) & 63];
+        wave_sync();
+      } else {
+#pragma unroll
+        for (int k = 0; k < W; ++k) {
+          el.v[k] = mk(from_prev_lane(br[S - W + k]), from_prev_lane(bi[S - W + k]));
+          er.v[k] = mk(from_next_lane(br[k]), from_next_lane(bi[k]));
+        }
       }
       // dt h_j = -i sum_d dt C_(j+d) j beta_(j+d): (sum c Im beta, -sum c Re beta)
 #pragma unroll
@@ -152,24 +212,27 @@ __global__ void __launch_bounds__(64) band_step_kernel(StepArgs g) {
         for (int d = -W; d <= W; ++d) {
           if (LIEB && !lieb_bond(s % 3, d)) continue;
           const int t = s + d;
-          const float vre = t < 0 ? lre[W + t] : t >= S ? rre[t - S] : br[t];
-          const float vim = t < 0 ? lim[W + t] : t >= S ? rim[t - S] : bi[t];
+          const float vre = t < 0 ? el.v[(t + 2 * W) % W].re : t >= S ? er.v[(t - S) % W].re : br[t < 0 || t >= S ? 0 : t];
+          const float vim = t < 0 ? el.v[(t + 2 * W) % W].im : t >= S ? er.v[(t - S) % W].im : bi[t < 0 || t >= S ? 0 : t];
           dr[s] = fmaf(cf[s][d + W], vim, dr[s]);
           di[s] = fmaf(-cf[s][d + W], vre, di[s]);
         }
       // noise and update
 #pragma unroll
       for (int p = 0; p < S / 2; ++p) {
-        const u32x4 w = philox4x32_10(make_counter(traj, TAG_WIENER, step, pbase + (uint32_t)p), g.key0, g.key1);
+        const u32x4 w = philox4x32_10_wave(make_counter(traj, TAG_WIENER, step, pbase + (uint32_t)p), g.key0, g.key1);
         float rn[2], cs[2], sn[2];
+        if constexpr (PRIO) __builtin_amdgcn_s_setprio(2);
         box_muller_f32_scaled(w.x, w.y, nl, rn[0], cs[0], sn[0]);
         box_muller_f32_scaled(w.z, w.w, nl, rn[1], cs[1], sn[1]);
+        if constexpr (PRIO) __builtin_amdgcn_s_setprio(0);
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
           const int s = 2 * p + h;
           const float x = br[s], y = bi[s];
           const float mq = fmaf(y, y, x * x);
-          const float cr = fmaf(-Ui[s], mq, A0[s]), ci = fmaf(Ur[s], mq, B0[s]);
+          const int t = UNI ? 0 : s;
+          const float cr = UNI ? A0[0] : fmaf(-Ui[t], mq, A0[t]), ci = fmaf(Ur[t], mq, B0[s]);
           // increment = noise + dt iF + dt h + drift, all small, added to beta once
           float ur = fmaf(rn[h], cs[h], dr[s]);
           ur = fmaf(cr, x, ur);
@@ -191,30 +254,33 @@ __global__ void __launch_bounds__(64) band_step_kernel(StepArgs g) {
   }
 }
 
-template <int S, int W>
-hipError_t launch_sw(const StepArgs& a, int grid, hipStream_t s) {
-  if constexpr (S == 6 && W == 2) {
-    if (a.band_lieb) {
-      if (a.ft_n > 0)
-        hipLaunchKernelGGL((band_step_kernel<6, 2, true, true>), dim3(grid), dim3(64), 0, s, a);
-      else
-        hipLaunchKernelGGL((band_step_kernel<6, 2, false, true>), dim3(grid), dim3(64), 0, s, a);
-      return hipGetLastError();
-    }
-  }
-  if (a.ft_n > 0)
-    hipLaunchKernelGGL((band_step_kernel<S, W, true, false>), dim3(grid), dim3(64), 0, s, a);
-  else
-    hipLaunchKernelGGL((band_step_kernel<S, W, false, false>), dim3(grid), dim3(64), 0, s, a);
-  return hipGetLastError();
+template <int S, int W, bool LIEB>
+const void* kernel_swl(bool ft, bool uni, bool dense) {
+  if (ft) return (const void*)band_step_kernel<S, W, true, LIEB, false, false>;
+  if (uni)
+    return dense ? (const void*)band_step_kernel<S, W, false, LIEB, true, true>
+                 : (const void*)band_step_kernel<S, W, false, LIEB, true, false>;
+  return dense ? (const void*)band_step_kernel<S, W, false, LIEB, false, true>
+               : (const void*)band_step_kernel<S, W, false, LIEB, false, false>;
 }
 
 template <int S>
-hipError_t launch_s(const StepArgs& a, int grid, hipStream_t s) {
-  switch (a.band_w) {
-    case 1: return launch_sw<S, 1>(a, grid, s);
-    case 2: return launch_sw<S, 2>(a, grid, s);
-    default: return launch_sw<S, 3>(a, grid, s);
+const void* kernel_s(int w, bool lieb, bool ft, bool uni, bool dense) {
+  if constexpr (S == 6)
+    if (lieb && w == 2) return kernel_swl<6, 2, true>(ft, uni, dense);
+  switch (w) {
+    case 1: return kernel_swl<S, 1, false>(ft, uni, dense);
+    case 2: return kernel_swl<S, 2, false>(ft, uni, dense);
+    default: return kernel_swl<S, 3, false>(ft, uni, dense);
+  }
+}
+
+const void* kernel_for(int n, int w, bool lieb, bool ft, bool uni, bool dense) {
+  switch (band_sites_per_lane(n)) {
+    case 2: return kernel_s<2>(w, lieb, ft, uni, dense);
+    case 4: return kernel_s<4>(w, lieb, ft, uni, dense);
+    case 6: return kernel_s<6>(w, lieb, ft, uni, dense);
+    default: return kernel_s<8>(w, lieb, ft, uni, dense);
   }
 }
 
@@ -267,37 +333,19 @@ bool band_lieb_pattern(const float* coef, int n, int w) {
 }
 
 hipError_t launch_band(const StepArgs& a, int grid, hipStream_t s) {
-  switch (band_sites_per_lane(a.n)) {
-    case 2: return launch_s<2>(a, grid, s);
-    case 4: return launch_s<4>(a, grid, s);
-    case 6: return launch_s<6>(a, grid, s);
-    default: return launch_s<8>(a, grid, s);
-  }
+  const void* f = kernel_for(a.n, a.band_w, a.band_lieb != 0, a.ft_n > 0, a.band_uni != 0, a.band_dense != 0);
+  void* args[] = {const_cast<StepArgs*>(&a)};
+  return hipLaunchKernel(f, dim3(grid), dim3(64), args, 0, s);
 }
 
-// occupancy of the instantiation launch_band runs for (n, w, lieb) (the
-// FT = false variant, the larger of the two)
-template <int S>
-const void* band_kernel_for(int w, int lieb) {
-  if constexpr (S == 6) {
-    if (lieb && w == 2) return (const void*)band_step_kernel<6, 2, false, true>;
-  }
-  switch (w) {
-    case 1: return (const void*)band_step_kernel<S, 1, false, false>;
-    case 2: return (const void*)band_step_kernel<S, 2, false, false>;
-    default: return (const void*)band_step_kernel<S, 3, false, false>;
-  }
-}
+// the batch gives every SIMD more than two waves
+bool band_dense(size_t n_traj, int cus) { return n_traj > 2 * 4 * (size_t)cus; }
 
-hipError_t band_occupancy(int n, int w, int lieb, int* blocks_per_cu) {
-  const void* f = nullptr;
-  switch (band_sites_per_lane(n)) {
-    case 2: f = band_kernel_for<2>(w, lieb); break;
-    case 4: f = band_kernel_for<4>(w, lieb); break;
-    case 6: f = band_kernel_for<6>(w, lieb); break;
-    default: f = band_kernel_for<8>(w, lieb); break;
-  }
-  return hipOccupancyMaxActiveBlocksPerMultiprocessor(blocks_per_cu, f, 64, 0);
+// occupancy of the instantiation launch_band runs (for F(t) that of a static
+// drive, the larger of the two)
+hipError_t band_occupancy(int n, int w, int lieb, int uni, int dense, int* blocks_per_cu) {
+  return hipOccupancyMaxActiveBlocksPerMultiprocessor(
+      blocks_per_cu, kernel_for(n, w, lieb != 0, false, uni != 0, dense != 0), 64, 0);
 }
 
 }  // namespace twmc

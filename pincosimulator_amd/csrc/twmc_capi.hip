@@ -86,6 +86,7 @@ struct Ctx {
   int np = 0;  // padded site count of the MFMA kernel
   int band_w = -1;  // half-width of the coupling matrix (matrix hopping), -1: not banded
   int band_lieb = 0;  // the banded coupling has the Lieb chain's pattern
+  int band_uni = 0;   // banded kernel: only Im rsl differs from site to site
   int ell_m = 0;      // TWMC_KERNEL_GENERIC, matrix hopping: entries per column of the sparse kernel, 0: not used
   StackPlan stack;  // TWMC_KERNEL_STACK: the batch's point and work items on the sweep kernel
   // per-batch buffers
@@ -112,6 +113,7 @@ struct Ctx {
   int grid = 0, block = 256;
   int cap_grid = 0;  // stencil64: grid of the capture launch (the 64x64 FFT kernel's)
   SparsePlan sparse;  // LDS kernel, matrix hopping: its steps on the sparse kernel
+  bool band_dense = false;  // banded kernel: the batch's form (band_dense)
   int grid_nn = 0;   // LDS kernel, FFT hopping: grid of the nearest-neighbour step launch
   size_t lds_nn = 0;
   size_t lds = 0;
@@ -250,6 +252,17 @@ bool site_uniform(const Ctx* c) {
   for (int k = 0; k < 3; ++k)
     for (int i = 1; i < c->n; ++i)
       if (c->base[k][2 * i] != c->base[k][0] || c->base[k][2 * i + 1] != c->base[k][1]) return false;
+  return true;
+}
+
+// Re rsl (the imaginary part of omega or E), a real U and a static F the same at
+// every site
+bool all_but_energy_uniform(const Ctx* c) {
+  if (c->noisy_params || c->ft_n > 0) return false;
+  for (int i = 0; i < c->n; ++i)
+    if (c->base[0][2 * i + 1] != c->base[0][1] || c->base[1][2 * i] != c->base[1][0] || c->base[1][2 * i + 1] != 0.0 ||
+        c->base[2][2 * i] != c->base[2][0] || c->base[2][2 * i + 1] != c->base[2][1])
+      return false;
   return true;
 }
 
@@ -490,6 +503,7 @@ struct Geometry {
   int grid_nn = 0;  // LDS kernel with FFT hopping: the step launch without the FFT's second buffer
   size_t lds_nn = 0;
   SparsePlan sparse;  // LDS kernel with matrix hopping: the step launch on the sparse kernel
+  bool band_dense = false;
 };
 
 int step_geometry(Ctx* c, size_t B, Geometry& geo) {
@@ -512,7 +526,8 @@ int step_geometry(Ctx* c, size_t B, Geometry& geo) {
   } else if (c->kernel == TWMC_KERNEL_BAND) {
     geo.block = 64;
     geo.lds = 0;
-    HIPCHK(c, band_occupancy(c->n, c->band_w, c->band_lieb, &per_cu));
+    geo.band_dense = band_dense(B, cus) && c->ft_n == 0;
+    HIPCHK(c, band_occupancy(c->n, c->band_w, c->band_lieb, c->band_uni, geo.band_dense, &per_cu));
   } else if (c->kernel == TWMC_KERNEL_MFMA) {
     geo.block = mfma_block(c->np);
     geo.lds = mfma_lds_bytes(c->np);
@@ -578,6 +593,7 @@ StepArgs shared_step_args(const Ctx* c) {
   a.band_coef = static_cast<const float*>(c->d_band.p);
   a.band_w = c->band_w;
   a.band_lieb = c->band_lieb;
+  a.band_uni = c->band_uni;
   a.ell_coef = c->d_ell_coef.p;
   a.ell_row = static_cast<const int*>(c->d_ell_row.p);
   a.ell_m = c->ell_m;
@@ -841,6 +857,7 @@ int twmc_create(const twmc_params* p, int device, twmc_ctx** ctx_out) {
     std::vector<float> coef((size_t)64 * S * (2 * c->band_w + 1));
     band_coefficients(p->coupling, c->n, c->band_w, p->dt, coef.data());
     c->band_lieb = band_lieb_pattern(coef.data(), c->n, c->band_w) ? 1 : 0;
+    c->band_uni = all_but_energy_uniform(c) ? 1 : 0;
     hipError_t ee = upload(c->d_band, coef.data(), coef.size() * sizeof(float), s);
     if (ee == hipSuccess) ee = hipStreamSynchronize(s);
     if (ee != hipSuccess) fail_rc = hip_fail(c, ee, "upload band coefficients");
@@ -954,6 +971,7 @@ int twmc_batch_begin(twmc_ctx* ctx, const twmc_batch_desc* d) {
     c->lds = geo.lds;
     c->cap_grid = geo.cap_grid;
     c->sparse = geo.sparse;
+    c->band_dense = geo.band_dense;
     c->grid_nn = geo.grid_nn;
     c->lds_nn = geo.lds_nn;
   }
@@ -1100,6 +1118,7 @@ int twmc_batch_advance(twmc_ctx* ctx, uint64_t n_segments) {
         int rc = advance_stencil(c, a, s);
         if (rc != TWMC_OK) return rc;
       } else if (c->kernel == TWMC_KERNEL_BAND) {
+        a.band_dense = c->band_dense ? 1 : 0;
         int rc = advance_band(c, a, s);
         if (rc != TWMC_OK) return rc;
       } else if (c->kernel == TWMC_KERNEL_STACK) {
@@ -1366,6 +1385,7 @@ int twmc_advance_noalloc(twmc_ctx* ctx, const uint64_t* d_traj_ids, uint64_t n_t
     if (c->kernel == TWMC_KERNEL_STENCIL64) {
       HIPCHK(c, launch_stencil64(a, geo.grid, s));
     } else if (c->kernel == TWMC_KERNEL_BAND) {
+      a.band_dense = geo.band_dense ? 1 : 0;
       HIPCHK(c, launch_band(a, geo.grid, s));
     } else if (c->kernel == TWMC_KERNEL_FUSED64) {
       HIPCHK(c, launch_fused64(a, geo.grid, s));

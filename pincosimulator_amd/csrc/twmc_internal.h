@@ -93,6 +93,8 @@ struct StepArgs {
   const int* ell_row;
   int ell_m;
   int band_lieb;             // banded kernel: the coupling has the Lieb chain's pattern (S = 6, W = 2)
+  int band_dense;            // banded kernel: the form for batches that fill the SIMDs (band_dense)
+  int band_uni;              // banded kernel: Re rsl, F and a real U the same at every site, F static
   // time-dependent drive: F(t) = ft_vals[id] + (t - ft_times[id]) ft_slopes[id]
   // with id the last table time below t (F = ft_vals[0] up to ft_times[0]);
   // t = t0 + s dt before step s of this launch, in FP64
@@ -238,7 +240,8 @@ void band_coefficients(const double* coupling, int n, int w, double dt, float* o
 // bonds (A: +1; B: -2, -1, +1; C: -1, +2, by site index mod 3) and S = 6, W = 2
 bool band_lieb_pattern(const float* coef, int n, int w);
 hipError_t launch_band(const StepArgs& a, int grid, hipStream_t s);
-hipError_t band_occupancy(int n, int w, int lieb, int* blocks_per_cu);
+bool band_dense(size_t n_traj, int cus);  // the batch fills the SIMDs: StepArgs::band_dense
+hipError_t band_occupancy(int n, int w, int lieb, int uni, int dense, int* blocks_per_cu);
 
 // matrix hopping with at most six nonzeros per column (`most`), up to 512 sites:
 // whole trajectories in a wave's registers, FP64 or FP32

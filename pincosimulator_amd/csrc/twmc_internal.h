@@ -248,6 +248,7 @@ hipError_t band_occupancy(int n, int w, int lieb, int uni, int dense, int* block
 constexpr int kSparseMaxSites = 512;
 struct SparsePlan {
   int s = 0;  // sites per lane, 0: not planned
+  bool prio = false;
   int grid = 0;
   size_t lds = 0;
 };

@@ -177,8 +177,13 @@ __device__ __forceinline__ void step_item(const SweepArgs& g, const SweepPointDe
         const u32x4 w = MULTI ? philox4x32_10(make_counter(trj[j], TAG_WIENER, step, pair), g.key0, g.key1)
                               : philox4x32_10_wave(make_counter(traj0, TAG_WIENER, step, pair), g.key0, g.key1);
         float rs[2], cs[2], sn[2];
+        // a wave forming its samples goes first, so that the waves do not bunch up
+        // before the transcendental unit (48x48 x 1999: 5.17 -> 4.92 us per step;
+        // stacked 2D items lose by it: 30x30 x 2500 2.6 -> 3.0)
+        if constexpr (!MULTI) __builtin_amdgcn_s_setprio(2);
         box_muller_f32_scaled(w.x, w.y, nl, rs[0], cs[0], sn[0]);
         box_muller_f32_scaled(w.z, w.w, nl, rs[1], cs[1], sn[1]);
+        if constexpr (!MULTI) __builtin_amdgcn_s_setprio(0);
         const cpx<float> z0 = beta[2 * j], z1 = beta[2 * j + 1];
         float sr[2], si[2];
         sr[0] = z1.re + L.re;

@@ -81,7 +81,7 @@ struct Ctx {
   // device-resident constants
   DevBuf d_base[5], d_amp[5], d_twx, d_twy, d_kcx, d_kcy, d_cscp, d_cscr, d_cscv, d_perm_site,
       d_perm_k, d_ahi, d_alo, d_kamp, d_ft_times, d_ft_vals, d_ft_slopes, d_band,
-      d_ell_coef, d_ell_row;
+      d_ell_coef, d_ell_row, d_queue;
   int ft_n = 0;  // F(t) table times (0: static F)
   int np = 0;  // padded site count of the MFMA kernel
   int band_w = -1;  // half-width of the coupling matrix (matrix hopping), -1: not banded
@@ -900,7 +900,7 @@ void twmc_destroy(twmc_ctx* ctx) {
   DevBuf* bufs[] = {&c->d_twx,       &c->d_twy,      &c->d_kcx,       &c->d_kcy,  &c->d_cscp, &c->d_cscr,
                     &c->d_cscv,      &c->d_perm_site, &c->d_perm_k,   &c->d_ahi,  &c->d_alo,  &c->d_kamp,
                     &c->d_ft_times,  &c->d_ft_vals,  &c->d_ft_slopes, &c->d_band, &c->d_ids,  &c->d_beta,
-                    &c->d_ell_coef,  &c->d_ell_row,
+                    &c->d_ell_coef,  &c->d_ell_row, &c->d_queue,
                     &c->d_rsl,       &c->d_U,        &c->d_F,         &c->d_partials, &c->d_obs, &c->d_m2,
                     &c->d_m4,        &c->d_traj,     &c->d_prev};
   for (DevBuf* b : bufs) b->release();
@@ -994,6 +994,7 @@ int twmc_batch_begin(twmc_ctx* ctx, const twmc_batch_desc* d) {
 
   size_t sets = c->noisy_params ? B : 1;
   HIPCHK(c, upload(c->d_ids, d->traj_ids, B * sizeof(uint64_t), s));
+  if (c->kernel == TWMC_KERNEL_STENCIL64) HIPCHK(c, c->d_queue.ensure(256));
   HIPCHK(c, c->d_beta.ensure(B * n * c->es));
   HIPCHK(c, c->d_rsl.ensure(sets * n * c->es));
   HIPCHK(c, c->d_U.ensure(sets * n * c->es));
@@ -1113,6 +1114,7 @@ int twmc_batch_advance(twmc_ctx* ctx, uint64_t n_segments) {
       a.traj_m2 = static_cast<double*>(c->d_m2.p);
       a.traj_m4 = static_cast<double*>(c->d_m4.p);
       a.traj_out = c->d_traj.p;
+      a.queue = static_cast<unsigned int*>(c->d_queue.p);
       a.t0 = c->desc.t_start + double(c->steps_done) * c->p.dt;
       if (c->kernel == TWMC_KERNEL_STENCIL64) {
         int rc = advance_stencil(c, a, s);
@@ -1326,9 +1328,10 @@ int twmc_advance_noalloc(twmc_ctx* ctx, const uint64_t* d_traj_ids, uint64_t n_t
   unsigned char* base = static_cast<unsigned char*>(scratch_address(c->device));
   if (!base) return fail(c, TWMC_ERR_STATE, "no scratch address for this device");
   const int n = c->n;
-  // scratch layout: rsl, U, F tables (n complex each), then [chunks][kQ][n] doubles
+  // scratch layout: rsl, U, F tables (n complex each), the work queue, then
+  // [chunks][kQ][n] doubles
   const size_t table = ((size_t)n * c->es + 255) / 256 * 256;
-  const size_t params = 3 * table;
+  const size_t params = 3 * table + 256;
   const size_t per_chunk = (size_t)kQ * n * sizeof(double);
   if (params + per_chunk > (size_t)TWMC_NOALLOC_SCRATCH_BYTES)
     return fail(c, TWMC_ERR_INVALID, "lattice too large for the allocation-free scratch array");
@@ -1381,6 +1384,7 @@ int twmc_advance_noalloc(twmc_ctx* ctx, const uint64_t* d_traj_ids, uint64_t n_t
     a.U = U;
     a.F = F;
     a.partials = partials;
+    a.queue = reinterpret_cast<unsigned int*>(base + 3 * table);
     a.t0 = double(step0 + done) * c->p.dt;
     if (c->kernel == TWMC_KERNEL_STENCIL64) {
       HIPCHK(c, launch_stencil64(a, geo.grid, s));

@@ -83,6 +83,7 @@ struct StepArgs {
   const void* a_hi;
   const void* a_lo;
   int np;                    // n padded to a multiple of 32
+  unsigned int* queue;       // 64x64 stencil kernel: work queue of the launch (one word)
   int u_real;                // 1: Im U = 0 at every site, in every trajectory
   int site_uniform;          // 1: rsl, U and F are the same at every site and in every trajectory, F static
   const float* band_coef;    // banded kernel: [64 S][2W + 1] dt C_(j+d) j

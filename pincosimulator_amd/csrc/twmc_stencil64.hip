@@ -38,16 +38,24 @@ constexpr int kL = 64;
 //
 // What bounds it: VALU issue, 44.5 instructions per site-step of which the four
 // transcendental ones run on their own unit beside the others when other waves
-// have work: 64 registers for eight waves per SIMD, two workgroups per CU.
-// 16384 trajectories: 69.6 us per step = 9.64e11 site-steps/s, 0.99 of the issue
-// rate of the other 40.5.  Before, one wave per trajectory with its rows in
-// registers (128 VGPRs, four waves per SIMD) took 80.2 us, the same count of
-// instructions at 0.86; this form at four waves (66 VGPRs) 75.8.  Few
-// trajectories have a whole CU each instead of one SIMD: 64 of them 5.85 -> 1.27
-// us per step, 1024 6.23 -> 4.93.  Each site's operations and their order are
-// those of that kernel: the same bits.
+// have work: 64 registers for eight waves per SIMD, two workgroups per CU.  The
+// two do not advance evenly (the older one is served first), so trajectories are
+// taken from a queue: dealt out by workgroup, one of the two finished early and
+// left the other to a half-filled CU.  16384 trajectories, 500-step launches:
+// 60.9 us per step = 1.10e12 site-steps/s; dealt out 69.6; one wave per trajectory
+// with its rows in registers (128 VGPRs, four waves per SIMD), the form before
+// both, 80.2; this form at four waves per SIMD 75.8; raised priority around the
+// samples, as in the banded kernel, 61.8.  Few trajectories have a whole CU each
+// instead of one SIMD: 64 of them 5.85 -> 1.27 us per step, 1024 6.23 -> 4.5.  Each
+// site's operations and their order are those of the one-wave form: the same
+// bits.
 constexpr int kBlock = 1024;
 constexpr int kPairs = kL * kL / 2;
+
+// clears the launch's work queue
+__global__ void queue_reset_kernel(unsigned int* queue) {
+  if (threadIdx.x == 0) *queue = 0u;
+}
 
 template <bool UI0>
 __global__ void __launch_bounds__(kBlock, 8) stencil64_step_kernel(StepArgs g) {
@@ -68,7 +76,8 @@ __global__ void __launch_bounds__(kBlock, 8) stencil64_step_kernel(StepArgs g) {
   const int lft = row + ((p0 - 1) & 31), rgt = row + ((p0 + 1) & 31);
   const int dn0 = (p0 - 32) & (kPairs - 1), up1 = (p0 + kBlock + 32) & (kPairs - 1);
 
-  for (int b = blockIdx.x; b < g.n_traj; b += gridDim.x) {
+  // the first trajectory by workgroup, the next ones from the queue
+  for (int b = blockIdx.x; b < g.n_traj;) {
     const uint64_t traj = g.traj_ids[b];
     float4* gb = reinterpret_cast<float4*>(reinterpret_cast<cpx<float>*>(g.beta) + (size_t)b * kL * kL);
     cpx<float> beta[4];
@@ -133,7 +142,12 @@ __global__ void __launch_bounds__(kBlock, 8) stencil64_step_kernel(StepArgs g) {
       const cpx<float> v0 = beta[2 * j], v1 = beta[2 * j + 1];
       gb[p0 + kBlock * j] = make_float4(v0.re, v0.im, v1.re, v1.im);
     }
-    __syncthreads();  // the next trajectory's load overwrites copy 0
+    // the next trajectory, through a word of copy 1 (its load writes copy 0)
+    int* next = reinterpret_cast<int*>(&st[1][0][0]);
+    __syncthreads();
+    if (threadIdx.x == 0) *next = (int)(gridDim.x + atomicAdd(g.queue, 1u));
+    __syncthreads();
+    b = __builtin_amdgcn_readfirstlane(*next);
   }
 }
 
@@ -144,6 +158,7 @@ bool stencil64_supported(int nx, int ny, int hopping, int precision, int param_s
 }
 
 hipError_t launch_stencil64(const StepArgs& a, int grid, hipStream_t s) {
+  hipLaunchKernelGGL(queue_reset_kernel, dim3(1), dim3(64), 0, s, a.queue);
   if (a.u_real)
     hipLaunchKernelGGL(stencil64_step_kernel<true>, dim3(grid), dim3(kBlock), 0, s, a);
   else

@@ -114,6 +114,7 @@ struct Ctx {
   int cap_grid = 0;  // stencil64: grid of the capture launch (the 64x64 FFT kernel's)
   SparsePlan sparse;  // LDS kernel, matrix hopping: its steps on the sparse kernel
   bool band_dense = false;  // banded kernel: the batch's form (band_dense)
+  bool nn64 = false;        // LDS kernel, FFT hopping: its steps on the nn64 kernel
   int grid_nn = 0;   // LDS kernel, FFT hopping: grid of the nearest-neighbour step launch
   size_t lds_nn = 0;
   size_t lds = 0;
@@ -252,6 +253,14 @@ bool site_uniform(const Ctx* c) {
   for (int k = 0; k < 3; ++k)
     for (int i = 1; i < c->n; ++i)
       if (c->base[k][2 * i] != c->base[k][0] || c->base[k][2 * i + 1] != c->base[k][1]) return false;
+  return true;
+}
+
+// Im U = 0 at every site, in every trajectory
+bool u_real(const Ctx* c) {
+  if (c->noise[1] != TWMC_NOISE_NONE) return false;
+  for (int i = 0; i < c->n; ++i)
+    if (c->base[1][2 * i + 1] != 0.0) return false;
   return true;
 }
 
@@ -504,6 +513,7 @@ struct Geometry {
   size_t lds_nn = 0;
   SparsePlan sparse;  // LDS kernel with matrix hopping: the step launch on the sparse kernel
   bool band_dense = false;
+  bool nn64 = false;  // LDS kernel with FFT hopping: the step launch on the nn64 kernel
 };
 
 int step_geometry(Ctx* c, size_t B, Geometry& geo) {
@@ -538,7 +548,14 @@ int step_geometry(Ctx* c, size_t B, Geometry& geo) {
     geo.lds = generic_lds_bytes(c->p.nx, c->p.ny, c->precision);
     HIPCHK(c, generic_occupancy(c->precision, c->n, geo.block, geo.lds, &per_cu));
     if (c->ell_m > 0) HIPCHK(c, sparse_plan(c->n, c->precision, c->ell_m, B, cus, &geo.sparse));
-    if (c->p.hopping == TWMC_HOP_FFT) {
+    if (c->p.hopping == TWMC_HOP_FFT && nn64_supported(c->p.nx, c->p.ny, c->precision, site_uniform(c)) &&
+        nn64_pays(c->n, B, cus)) {
+      int per_cu_nn = 0;
+      HIPCHK(c, nn64_occupancy(c->p.nx, c->p.ny, u_real(c), &per_cu_nn));
+      if (per_cu_nn < 1) return fail(c, TWMC_ERR_UNSUPPORTED, "step kernel does not fit on a CU");
+      geo.nn64 = true;
+      geo.grid_nn = (int)std::min<size_t>(B, (size_t)per_cu_nn * cus);
+    } else if (c->p.hopping == TWMC_HOP_FFT) {
       int per_cu_nn = 0;
       geo.lds_nn = generic_nn_lds_bytes(c->p.nx, c->p.ny, c->precision, site_uniform(c));
       HIPCHK(c, generic_nn_occupancy(c->precision, c->p.nx, c->p.ny, geo.lds_nn, site_uniform(c), &per_cu_nn));
@@ -587,9 +604,7 @@ StepArgs shared_step_args(const Ctx* c) {
   a.ft_vals = c->d_ft_vals.p;
   a.ft_slopes = c->d_ft_slopes.p;
   a.site_uniform = site_uniform(c) ? 1 : 0;
-  a.u_real = 1;
-  for (int i = 0; i < c->n && a.u_real; ++i) a.u_real = c->base[1][2 * i + 1] == 0.0;
-  if (c->noise[1] != TWMC_NOISE_NONE) a.u_real = 0;
+  a.u_real = u_real(c) ? 1 : 0;
   a.band_coef = static_cast<const float*>(c->d_band.p);
   a.band_w = c->band_w;
   a.band_lieb = c->band_lieb;
@@ -627,7 +642,10 @@ int advance_generic_fft(Ctx* c, const StepArgs& a, hipStream_t s) {
     sa.capture = 0;
     hipEvent_t e0 = nullptr;
     HIPCHK(c, timed(c, c->ev_step, s, true, e0));
-    HIPCHK(c, launch_generic_nn(sa, c->precision, c->grid_nn, c->lds_nn, s));
+    if (c->nn64)
+      HIPCHK(c, launch_nn64(sa, c->grid_nn, s));
+    else
+      HIPCHK(c, launch_generic_nn(sa, c->precision, c->grid_nn, c->lds_nn, s));
     HIPCHK(c, timed(c, c->ev_step, s, false, e0));
     c->stats.site_steps += (uint64_t)a.n_steps * (uint64_t)n * c->n_traj;
   }
@@ -972,6 +990,7 @@ int twmc_batch_begin(twmc_ctx* ctx, const twmc_batch_desc* d) {
     c->cap_grid = geo.cap_grid;
     c->sparse = geo.sparse;
     c->band_dense = geo.band_dense;
+    c->nn64 = geo.nn64;
     c->grid_nn = geo.grid_nn;
     c->lds_nn = geo.lds_nn;
   }
@@ -994,7 +1013,7 @@ int twmc_batch_begin(twmc_ctx* ctx, const twmc_batch_desc* d) {
 
   size_t sets = c->noisy_params ? B : 1;
   HIPCHK(c, upload(c->d_ids, d->traj_ids, B * sizeof(uint64_t), s));
-  if (c->kernel == TWMC_KERNEL_STENCIL64) HIPCHK(c, c->d_queue.ensure(256));
+  if (c->kernel == TWMC_KERNEL_STENCIL64 || c->nn64) HIPCHK(c, c->d_queue.ensure(256));
   HIPCHK(c, c->d_beta.ensure(B * n * c->es));
   HIPCHK(c, c->d_rsl.ensure(sets * n * c->es));
   HIPCHK(c, c->d_U.ensure(sets * n * c->es));
@@ -1395,6 +1414,8 @@ int twmc_advance_noalloc(twmc_ctx* ctx, const uint64_t* d_traj_ids, uint64_t n_t
       HIPCHK(c, launch_fused64(a, geo.grid, s));
     } else if (c->kernel == TWMC_KERNEL_MFMA) {
       HIPCHK(c, launch_mfma(a, geo.grid, s));
+    } else if (geo.nn64) {
+      HIPCHK(c, launch_nn64(a, geo.grid_nn, s));
     } else if (c->p.hopping == TWMC_HOP_FFT) {
       HIPCHK(c, launch_generic_nn(a, c->precision, geo.grid_nn, geo.lds_nn, s));
     } else if (c->ell_m > 0) {

@@ -70,6 +70,13 @@ TWMC_HD inline double fma3(double a, double b, double c) {
 #endif
 }
 
+// The same for a coefficient c in scalar registers (SG: a kernel with few vector
+// registers keeps them there), which v_fma_f64 reads as it is.
+template <bool SG>
+TWMC_HD inline double fma3k(double a, double b, double c) {
+  return SG ? fma(a, b, c) : fma3(a, b, c);
+}
+
 TWMC_HD inline uint64_t bits(double x) {
   uint64_t u;
   memcpy(&u, &x, sizeof u);
@@ -150,6 +157,17 @@ TWMC_HD inline void pin(Series& k) {
 #endif
 }
 
+// The same with the coefficients in scalar registers, for SG.
+TWMC_HD inline void pin_scalar(Series& k) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm volatile("" : "+s"(k.s_top), "+s"(k.c_top), "+s"(k.l_top));
+  for (int j = 0; j < 2; ++j) asm volatile("" : "+s"(k.ks[j]), "+s"(k.kc[j]));
+  for (int j = 0; j < 6; ++j) asm volatile("" : "+s"(k.kl[j]));
+#else
+  (void)k;
+#endif
+}
+
 // The tables (TWMC_F64_TABLES, 768 doubles): the ln rows (2 c_j, L_j) from
 // kTabLog, the sin / cos rows (cos theta_j, sin theta_j) from kTabSinCos.  On
 // the host the functions read them from kTables; device code hands them a copy
@@ -163,7 +181,7 @@ struct alignas(16) Row {
 };
 
 // sin and cos of 2 pi b[i] 2^-32, i < N.
-template <int N>
+template <int N, bool SG = false>
 TWMC_HD inline void sincos_turn32(const uint32_t* b, double* s, double* c, const Series& k = kSeries,
                                   const double* tab = kTables) {
   TWMC_NO_CONTRACT
@@ -186,8 +204,8 @@ TWMC_HD inline void sincos_turn32(const uint32_t* b, double* s, double* c, const
   for (int j = 0; j < 2; ++j)
     TWMC_UNROLL
     for (int i = 0; i < N; ++i) {
-      ps[i] = fma3(ps[i], z[i], k.ks[j]);
-      pc[i] = fma3(pc[i], z[i], k.kc[j]);
+      ps[i] = fma3k<SG>(ps[i], z[i], k.ks[j]);
+      pc[i] = fma3k<SG>(pc[i], z[i], k.kc[j]);
     }
   TWMC_UNROLL
   for (int i = 0; i < N; ++i) {
@@ -202,7 +220,7 @@ TWMC_HD inline void sincos_turn32(const uint32_t* b, double* s, double* c, const
 // ln((a[i] + 1/2) 2^-32), in (-22.9, 0), i < N.  A row (2 c, L) of the ln
 // table: r = m c - 1 and ln m = L + ln(1 + r), the exponent raised by one for
 // m > sqrt 2, which L absorbs as -ln 2.
-template <int N>
+template <int N, bool SG = false>
 TWMC_HD inline void log_u32(const uint32_t* a, double* out, const Series& k = kSeries,
                             const double* tab = kTables) {
   TWMC_NO_CONTRACT
@@ -228,7 +246,7 @@ TWMC_HD inline void log_u32(const uint32_t* a, double* out, const Series& k = kS
   TWMC_UNROLL
   for (int j = 0; j < 6; ++j)
     TWMC_UNROLL
-    for (int i = 0; i < N; ++i) p[i] = fma3(p[i], r[i], k.kl[j]);
+    for (int i = 0; i < N; ++i) p[i] = fma3k<SG>(p[i], r[i], k.kl[j]);
   TWMC_UNROLL
   for (int i = 0; i < N; ++i) {
     const double t = lt[i] + fma(r[i] * r[i], p[i], r[i]);
@@ -239,13 +257,13 @@ TWMC_HD inline void log_u32(const uint32_t* a, double* out, const Series& k = kS
 
 // N complex N(0, 1) samples from the Philox word pairs (a[i], b[i]):
 // Re = sqrt(-2 ln u1) cos(2 pi theta), Im = sqrt(-2 ln u1) sin(2 pi theta).
-template <int N>
+template <int N, bool SG = false>
 TWMC_HD inline void box_muller(const uint32_t* a, const uint32_t* b, double* re, double* im,
                                const Series& k = kSeries, const double* tab = kTables) {
   TWMC_NO_CONTRACT
   double l[N], s[N], c[N];
-  log_u32<N>(a, l, k, tab);
-  sincos_turn32<N>(b, s, c, k, tab);
+  log_u32<N, SG>(a, l, k, tab);
+  sincos_turn32<N, SG>(b, s, c, k, tab);
   TWMC_UNROLL
   for (int i = 0; i < N; ++i) {
     const double r = sqrt_normal(-2.0 * l[i]);

@@ -83,7 +83,7 @@ struct StepArgs {
   const void* a_hi;
   const void* a_lo;
   int np;                    // n padded to a multiple of 32
-  unsigned int* queue;       // 64x64 stencil kernel: work queue of the launch (one word)
+  unsigned int* queue;       // 64x64 stencil and nn64 kernels: work queue of the launch (one word)
   int u_real;                // 1: Im U = 0 at every site, in every trajectory
   int site_uniform;          // 1: rsl, U and F are the same at every site and in every trajectory, F static
   const float* band_coef;    // banded kernel: [64 S][2W + 1] dt C_(j+d) j
@@ -243,6 +243,14 @@ bool band_lieb_pattern(const float* coef, int n, int w);
 hipError_t launch_band(const StepArgs& a, int grid, hipStream_t s);
 bool band_dense(size_t n_traj, int cus);  // the batch fills the SIMDs: StepArgs::band_dense
 hipError_t band_occupancy(int n, int w, int lieb, int uni, int dense, int* blocks_per_cu);
+
+// FP64, FFT hopping, site-uniform, even rows, 257 to 4096 sites: the step launch of
+// the LDS kernel (TWMC_KERNEL_GENERIC) where it pays; needs StepArgs::queue
+bool nn64_supported(int nx, int ny, int precision, bool site_uniform);
+bool nn64_pays(int n, size_t n_traj, int cus);
+int nn64_block(int n);
+hipError_t nn64_occupancy(int nx, int ny, bool u_real, int* blocks_per_cu);
+hipError_t launch_nn64(const StepArgs& a, int grid, hipStream_t s);
 
 // matrix hopping with at most six nonzeros per column (`most`), up to 512 sites:
 // whole trajectories in a wave's registers, FP64 or FP32

@@ -114,7 +114,7 @@ struct Ctx {
   int cap_grid = 0;  // stencil64: grid of the capture launch (the 64x64 FFT kernel's)
   SparsePlan sparse;  // LDS kernel, matrix hopping: its steps on the sparse kernel
   bool band_dense = false;  // banded kernel: the batch's form (band_dense)
-  bool nn64 = false;        // LDS kernel, FFT hopping: its steps on the nn64 kernel
+  bool nn = false;          // LDS kernel, FFT hopping: its steps on the nn kernel
   int grid_nn = 0;   // LDS kernel, FFT hopping: grid of the nearest-neighbour step launch
   size_t lds_nn = 0;
   size_t lds = 0;
@@ -246,15 +246,21 @@ void plan_segments(Ctx* c) {
   }
 }
 
+// a bit for each of rsl, U and F: drawn per trajectory, or not the same at every site
+int param_vary(const Ctx* c) {
+  int v = 0;
+  for (int k = 0; k < 3; ++k) {
+    bool same = c->noise[k] == TWMC_NOISE_NONE;
+    for (int i = 1; i < c->n && same; ++i)
+      same = c->base[k][2 * i] == c->base[k][0] && c->base[k][2 * i + 1] == c->base[k][1];
+    if (!same) v |= 1 << k;
+  }
+  return v;
+}
+
 // rsl, U and F the same at every site and in every trajectory, F static: the
 // tables the init kernel forms are then uniform
-bool site_uniform(const Ctx* c) {
-  if (c->noisy_params || c->ft_n > 0) return false;
-  for (int k = 0; k < 3; ++k)
-    for (int i = 1; i < c->n; ++i)
-      if (c->base[k][2 * i] != c->base[k][0] || c->base[k][2 * i + 1] != c->base[k][1]) return false;
-  return true;
-}
+bool site_uniform(const Ctx* c) { return c->ft_n == 0 && param_vary(c) == 0; }
 
 // Im U = 0 at every site, in every trajectory
 bool u_real(const Ctx* c) {
@@ -513,7 +519,7 @@ struct Geometry {
   size_t lds_nn = 0;
   SparsePlan sparse;  // LDS kernel with matrix hopping: the step launch on the sparse kernel
   bool band_dense = false;
-  bool nn64 = false;  // LDS kernel with FFT hopping: the step launch on the nn64 kernel
+  bool nn = false;  // LDS kernel with FFT hopping: the step launch on the nn kernel
 };
 
 int step_geometry(Ctx* c, size_t B, Geometry& geo) {
@@ -548,12 +554,13 @@ int step_geometry(Ctx* c, size_t B, Geometry& geo) {
     geo.lds = generic_lds_bytes(c->p.nx, c->p.ny, c->precision);
     HIPCHK(c, generic_occupancy(c->precision, c->n, geo.block, geo.lds, &per_cu));
     if (c->ell_m > 0) HIPCHK(c, sparse_plan(c->n, c->precision, c->ell_m, B, cus, &geo.sparse));
-    if (c->p.hopping == TWMC_HOP_FFT && nn64_supported(c->p.nx, c->p.ny, c->precision, site_uniform(c)) &&
-        nn64_pays(c->n, B, cus)) {
+    if (c->p.hopping == TWMC_HOP_FFT && c->ft_n == 0 &&
+        nn_supported(c->p.nx, c->p.ny, c->precision, param_vary(c)) &&
+        nn_pays(c->p.nx, c->p.ny, c->precision, param_vary(c), B, cus)) {
       int per_cu_nn = 0;
-      HIPCHK(c, nn64_occupancy(c->p.nx, c->p.ny, u_real(c), &per_cu_nn));
+      HIPCHK(c, nn_occupancy(c->p.nx, c->p.ny, c->precision, param_vary(c), u_real(c), &per_cu_nn));
       if (per_cu_nn < 1) return fail(c, TWMC_ERR_UNSUPPORTED, "step kernel does not fit on a CU");
-      geo.nn64 = true;
+      geo.nn = true;
       geo.grid_nn = (int)std::min<size_t>(B, (size_t)per_cu_nn * cus);
     } else if (c->p.hopping == TWMC_HOP_FFT) {
       int per_cu_nn = 0;
@@ -605,6 +612,7 @@ StepArgs shared_step_args(const Ctx* c) {
   a.ft_slopes = c->d_ft_slopes.p;
   a.site_uniform = site_uniform(c) ? 1 : 0;
   a.u_real = u_real(c) ? 1 : 0;
+  a.vary = param_vary(c);
   a.band_coef = static_cast<const float*>(c->d_band.p);
   a.band_w = c->band_w;
   a.band_lieb = c->band_lieb;
@@ -642,8 +650,8 @@ int advance_generic_fft(Ctx* c, const StepArgs& a, hipStream_t s) {
     sa.capture = 0;
     hipEvent_t e0 = nullptr;
     HIPCHK(c, timed(c, c->ev_step, s, true, e0));
-    if (c->nn64)
-      HIPCHK(c, launch_nn64(sa, c->grid_nn, s));
+    if (c->nn)
+      HIPCHK(c, launch_nn(sa, c->precision, c->grid_nn, s));
     else
       HIPCHK(c, launch_generic_nn(sa, c->precision, c->grid_nn, c->lds_nn, s));
     HIPCHK(c, timed(c, c->ev_step, s, false, e0));
@@ -990,7 +998,7 @@ int twmc_batch_begin(twmc_ctx* ctx, const twmc_batch_desc* d) {
     c->cap_grid = geo.cap_grid;
     c->sparse = geo.sparse;
     c->band_dense = geo.band_dense;
-    c->nn64 = geo.nn64;
+    c->nn = geo.nn;
     c->grid_nn = geo.grid_nn;
     c->lds_nn = geo.lds_nn;
   }
@@ -1013,7 +1021,7 @@ int twmc_batch_begin(twmc_ctx* ctx, const twmc_batch_desc* d) {
 
   size_t sets = c->noisy_params ? B : 1;
   HIPCHK(c, upload(c->d_ids, d->traj_ids, B * sizeof(uint64_t), s));
-  if (c->kernel == TWMC_KERNEL_STENCIL64 || c->nn64) HIPCHK(c, c->d_queue.ensure(256));
+  if (c->kernel == TWMC_KERNEL_STENCIL64 || c->nn) HIPCHK(c, c->d_queue.ensure(256));
   HIPCHK(c, c->d_beta.ensure(B * n * c->es));
   HIPCHK(c, c->d_rsl.ensure(sets * n * c->es));
   HIPCHK(c, c->d_U.ensure(sets * n * c->es));
@@ -1414,8 +1422,8 @@ int twmc_advance_noalloc(twmc_ctx* ctx, const uint64_t* d_traj_ids, uint64_t n_t
       HIPCHK(c, launch_fused64(a, geo.grid, s));
     } else if (c->kernel == TWMC_KERNEL_MFMA) {
       HIPCHK(c, launch_mfma(a, geo.grid, s));
-    } else if (geo.nn64) {
-      HIPCHK(c, launch_nn64(a, geo.grid_nn, s));
+    } else if (geo.nn) {
+      HIPCHK(c, launch_nn(a, c->precision, geo.grid_nn, s));
     } else if (c->p.hopping == TWMC_HOP_FFT) {
       HIPCHK(c, launch_generic_nn(a, c->precision, geo.grid_nn, geo.lds_nn, s));
     } else if (c->ell_m > 0) {

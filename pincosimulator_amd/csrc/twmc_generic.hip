@@ -890,7 +890,7 @@ const void* generic_nn_ptr_l(int ppt, int block, int tpb) {
            : tpb == 2 ? (const void*)generic_step_kernel<T, 1, true, UNIF, LAY, 64, 2>
                       : (const void*)generic_step_kernel<T, 1, true, UNIF, LAY, 64>;
   if (block == 128) return (const void*)generic_step_kernel<T, 1, true, UNIF, LAY, 128>;
-  // FP64 site-uniform even rows of 257 to 2048 sites step on the nn64 kernel
+  // FP64 site-uniform even rows of 257 to 2048 sites step on the nn kernel (twmc_nn.hip)
   if constexpr (sizeof(T) == 8 && UNIF && LAY != 0)
     return (const void*)generic_step_kernel<T, 32, true, UNIF, LAY>;
   return ppt == 1   ? (const void*)generic_step_kernel<T, 1, true, UNIF, LAY>
@@ -929,7 +929,7 @@ const void* generic_nn_ptr(int precision, int ppt, bool unif, int lay, int block
 // threads per workgroup of a nearest-neighbour step launch: one or two waves
 // for lattices of up to 128 or 256 sites (a pair per thread, every wave busy),
 // 1024 for FP64 site-uniform lattices of 2049 to 4096 sites (with even rows and
-// more than two trajectories per CU the nn64 kernel takes them), else kBlock
+// more than two trajectories per CU the nn kernel takes them), else kBlock
 int generic_nn_block(int precision, int n, bool unif) {
   const int np = (n + 1) / 2;
   if (np <= 64) return 64;

@@ -83,8 +83,9 @@ struct StepArgs {
   const void* a_hi;
   const void* a_lo;
   int np;                    // n padded to a multiple of 32
-  unsigned int* queue;       // 64x64 stencil and nn64 kernels: work queue of the launch (one word)
+  unsigned int* queue;       // 64x64 stencil and nn kernels: work queue of the launch (one word)
   int u_real;                // 1: Im U = 0 at every site, in every trajectory
+  int vary;                  // a bit for each of rsl, U, F: not one value for all sites and trajectories
   int site_uniform;          // 1: rsl, U and F are the same at every site and in every trajectory, F static
   const float* band_coef;    // banded kernel: [64 S][2W + 1] dt C_(j+d) j
   int band_w;                // banded kernel: half-width W
@@ -244,13 +245,15 @@ hipError_t launch_band(const StepArgs& a, int grid, hipStream_t s);
 bool band_dense(size_t n_traj, int cus);  // the batch fills the SIMDs: StepArgs::band_dense
 hipError_t band_occupancy(int n, int w, int lieb, int uni, int dense, int* blocks_per_cu);
 
-// FP64, FFT hopping, site-uniform, even rows, 257 to 4096 sites: the step launch of
-// the LDS kernel (TWMC_KERNEL_GENERIC) where it pays; needs StepArgs::queue
-bool nn64_supported(int nx, int ny, int precision, bool site_uniform);
-bool nn64_pays(int n, size_t n_traj, int cus);
-int nn64_block(int n);
-hipError_t nn64_occupancy(int nx, int ny, bool u_real, int* blocks_per_cu);
-hipError_t launch_nn64(const StepArgs& a, int grid, hipStream_t s);
+// FFT hopping, 129 to 4096 sites, static parameters of which at most one varies from
+// site to site or is drawn (StepArgs::vary); FP32 uniform lattices only with odd rows
+// (the stacked kernel takes the even ones): the step launch of the LDS kernel
+// (TWMC_KERNEL_GENERIC) where it pays; needs StepArgs::queue
+constexpr int kVaryNone = 0, kVaryRsl = 1, kVaryF = 4;  // a bit for each of rsl, U, F
+bool nn_supported(int nx, int ny, int precision, int vary);
+bool nn_pays(int nx, int ny, int precision, int vary, size_t n_traj, int cus);
+hipError_t nn_occupancy(int nx, int ny, int precision, int vary, bool u_real, int* blocks_per_cu);
+hipError_t launch_nn(const StepArgs& a, int precision, int grid, hipStream_t s);
 
 // matrix hopping with at most six nonzeros per column (`most`), up to 512 sites:
 // whole trajectories in a wave's registers, FP64 or FP32

@@ -1,0 +1,227 @@
+// twmc_ahead.hip -- step kernel for small periodic lattices (up to 256 sites) in small
+// batches, the hopping in its nearest-neighbour form (the exact real-space form of the
+// reference's FFT product, TWMCBaseSolver.cpp:80-88, :235-242).
+//
+// What bounds it: the latency of one step after the other; the chip is mostly idle.
+// In the LDS kernel (twmc_generic.hip) a wave's step is the whole chain of ten Philox
+// rounds, Box-Muller and update.  But the noise does not depend on the state, so here
+// a workgroup of four waves (eight above 128 sites) owns a trajectory: one wave steps
+// it, one, two or four sites per lane, and the others write the next steps' noise into
+// LDS, a chunk ahead, every lane a pair of some step.  The chain is then one LDS
+// exchange and the update.  Every operation is the LDS kernel's, so the bits are the
+// same for either.  us per step, before -> now: 256 trajectories of 64 sites, FP64,
+// 0.54 -> 0.17 (0.15 us is 360 clocks); 100 of 4x4 with a drawn drive, FP64, 0.74 ->
+// 0.16; 256 of 5x13, FP32, 0.65 -> 0.21.
+#include <algorithm>
+
+#include "twmc_cplx.h"
+#include "twmc_f64math.h"
+#include "twmc_internal.h"
+#include "twmc_rng.h"
+
+namespace twmc {
+
+namespace {
+
+// the FP64 Box-Muller's ln and sin / cos tables (twmc_f64math.h)
+alignas(16) __device__ const double kF64TabDev[f64::kTabSize] = TWMC_F64_TABLES;
+
+constexpr int waves_of(int spl) { return spl == 4 ? 8 : 4; }
+constexpr int chunk_sites(int spl) { return spl == 4 ? 2048 : 1024; }  // noise of a chunk: steps x sites (rounded up to even)
+constexpr int kChunkSteps = 64;    // at most
+
+template <typename T>
+constexpr int kTab = sizeof(T) == 8 ? f64::kTabSize : 0;
+
+template <typename T, int SPL>
+struct Lds {
+  double tab[kTab<T> + 2];
+  cpx<T> st[64 * SPL];
+  // lanes past the lattice read, and drop, up to 64 SPL entries past a step's row
+  cpx<T> noise[2][chunk_sites(SPL) + 64 * SPL];
+};
+
+// what a lane wrote is seen by the wave's other lanes (LDS operations of a wave are
+// in order; this keeps the compiler's)
+__device__ __forceinline__ void lds_order() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+// SPL: sites per lane of the stepping wave.  UNIF: StepArgs::site_uniform.
+// XN: the lattice has x neighbours (nx > 1).
+template <typename T, int SPL, bool UNIF, bool XN>
+__global__ void __launch_bounds__(64 * waves_of(SPL)) ahead_step_kernel(StepArgs g) {
+  constexpr int kWaves = waves_of(SPL);
+  constexpr bool kF64 = sizeof(T) == 8;
+  constexpr bool kOnePlus = kF64 && UNIF;  // (1 + c) z with 1 + dt Re rsl formed once
+  extern __shared__ __align__(16) unsigned char smem[];
+  Lds<T, SPL>& lds = *reinterpret_cast<Lds<T, SPL>*>(smem);
+  if constexpr (kF64)
+    for (int i = threadIdx.x; i < f64::kTabSize; i += 64 * kWaves) lds.tab[i] = kF64TabDev[i];
+  __syncthreads();
+
+  const int n = g.n, np = (n + 1) / 2, stride = 2 * np, b = blockIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const uint64_t traj = g.traj_ids[b];
+  const int ksteps = min(kChunkSteps, chunk_sites(SPL) / stride);
+  // item / np as umulhi (items below 2^16)
+  const uint32_t magic = np > 1 ? (uint32_t)((0x100000000ull + (uint32_t)np - 1) / (uint32_t)np) : 0u;
+  auto produce = [&](int buf, int s0, int first, int waves) {
+    const int items = min(ksteps, g.n_steps - s0) * np;
+    for (int q = 64 * first + lane; q < items; q += 64 * waves) {
+      const int k = np > 1 ? (int)__umulhi((uint32_t)q, magic) : q, p = q - k * np;
+      const u32x4 x = philox4x32_10(make_counter(traj, TAG_WIENER, uint32_t(g.step0 + (uint64_t)(s0 + k)), (uint32_t)p),
+                                    g.key0, g.key1);
+      T re[2], im[2];
+      if constexpr (kF64) {
+        const uint32_t wa[2] = {x.x, x.z}, wb[2] = {x.y, x.w};
+        f64::box_muller<2>(wa, wb, re, im, f64::kSeries, lds.tab);
+      } else {
+        box_muller_f32(x.x, x.y, re[0], im[0]);
+        box_muller_f32(x.z, x.w, re[1], im[1]);
+      }
+      cpx<T>* out = lds.noise[buf] + 2 * q;  // row k, sites 2p and 2p + 1
+      out[0] = mk(re[0], im[0]);
+      out[1] = mk(re[1], im[1]);
+    }
+  };
+
+  // the stepping wave's sites lane + 64 j: state, constants scaled by dt, neighbours
+  cpx<T> z[SPL], rd[SPL], ud[SPL], fd[SPL];
+  int nb[SPL][4];
+  const T dt = T(g.dt), dt4 = T(g.dt4), djv = T(-0.5 * g.kscale * g.dt);
+  cpx<T>* const gb = reinterpret_cast<cpx<T>*>(g.beta) + (size_t)b * n;
+  const size_t poff = g.param_stride ? (size_t)b * n : 0;
+#pragma unroll
+  for (int j = 0; j < SPL; ++j) {
+    const int i = lane + 64 * j, x = i / g.ny, y = i - x * g.ny;
+    const bool in = wave == 0 && i < n;
+    const size_t ip = UNIF ? 0 : poff + (in ? i : 0);
+    const cpx<T> r = reinterpret_cast<const cpx<T>*>(g.rsl)[ip], u = reinterpret_cast<const cpx<T>*>(g.U)[ip],
+                 f = reinterpret_cast<const cpx<T>*>(g.F)[ip];
+    rd[j] = mk(kOnePlus ? T(1) + dt * r.re : dt * r.re, dt * r.im);
+    ud[j] = mk(dt * u.re, dt * u.im);
+    fd[j] = mk(-dt * f.im, dt * f.re);
+    z[j] = in ? gb[i] : mk(T(0), T(0));
+    nb[j][0] = y + 1 == g.ny ? i + 1 - g.ny : i + 1;
+    nb[j][1] = y == 0 ? i + g.ny - 1 : i - 1;
+    nb[j][2] = i + g.ny >= n ? i + g.ny - n : i + g.ny;
+    nb[j][3] = i < g.ny ? i - g.ny + n : i - g.ny;
+    if (!in) nb[j][0] = nb[j][1] = nb[j][2] = nb[j][3] = 0;
+  }
+
+  produce(0, 0, wave, kWaves);
+  __syncthreads();
+  for (int s0 = 0, c = 0; s0 < g.n_steps; s0 += ksteps, c ^= 1) {
+    if (wave == 0) {
+      const int steps = min(ksteps, g.n_steps - s0);
+      const cpx<T>* row = lds.noise[c] + lane;
+      cpx<T> xi[SPL];
+#pragma unroll
+      for (int j = 0; j < SPL; ++j) xi[j] = row[64 * j];
+      for (int k = 0; k < steps; ++k) {
+#pragma unroll
+        for (int j = 0; j < SPL; ++j) lds.st[lane + 64 * j] = z[j];
+        lds_order();
+        cpx<T> a[SPL][4];
+#pragma unroll
+        for (int j = 0; j < SPL; ++j)
+#pragma unroll
+          for (int h = 0; h < (XN ? 4 : 2); ++h) a[j][h] = lds.st[nb[j][h]];
+        lds_order();
+        row += k + 1 < steps ? stride : 0;
+        cpx<T> next[SPL];
+#pragma unroll
+        for (int j = 0; j < SPL; ++j) next[j] = row[64 * j];
+#pragma unroll
+        for (int j = 0; j < SPL; ++j) {
+          // y + 1 and y - 1 neighbours, then x + 1 and x - 1
+          T sr = a[j][0].re + a[j][1].re, si = a[j][0].im + a[j][1].im;
+          if constexpr (XN) {
+            sr += a[j][2].re + a[j][3].re;
+            si += a[j][2].im + a[j][3].im;
+          }
+          // increment dt (c z + h + i F) + dt4 xi as one FMA chain per component;
+          // dt h = dt J (S_im, -S_re)
+          const cpx<T> w = z[j];
+          const T q = fma(w.re, w.re, fma(w.im, w.im, T(-1)));
+          const T ci = fma(ud[j].re, q, rd[j].im), cr = fma(-ud[j].im, q, rd[j].re);
+          T dr = fma(dt4, xi[j].re, fd[j].re);
+          dr = fma(djv, si, dr);
+          T di = fma(dt4, xi[j].im, fd[j].im);
+          di = fma(-djv, sr, di);
+          if constexpr (kOnePlus) {
+            dr = fma(-ci, w.im, dr);
+            di = fma(ci, w.re, di);
+            z[j] = mk(fma(cr, w.re, dr), fma(cr, w.im, di));
+          } else {
+            dr = fma(cr, w.re, dr);
+            dr = fma(-ci, w.im, dr);
+            di = fma(cr, w.im, di);
+            di = fma(ci, w.re, di);
+            z[j] = mk(w.re + dr, w.im + di);
+          }
+          xi[j] = next[j];
+        }
+      }
+    } else if (s0 + ksteps < g.n_steps) {
+      produce(c ^ 1, s0 + ksteps, wave - 1, kWaves - 1);
+    }
+    __syncthreads();
+  }
+#pragma unroll
+  for (int j = 0; j < SPL; ++j) {
+    const int i = lane + 64 * j;
+    if (wave == 0 && i < n) gb[i] = z[j];
+  }
+}
+
+struct Launch {
+  const void* f;
+  int block;
+  size_t lds;
+};
+
+template <typename T, int SPL>
+Launch launch_s(bool unif, bool xn) {
+  return {unif ? (xn ? (const void*)ahead_step_kernel<T, SPL, true, true> : (const void*)ahead_step_kernel<T, SPL, true, false>)
+               : (xn ? (const void*)ahead_step_kernel<T, SPL, false, true> : (const void*)ahead_step_kernel<T, SPL, false, false>),
+          64 * waves_of(SPL), sizeof(Lds<T, SPL>)};
+}
+
+template <typename T>
+Launch launch_t(int n, bool unif, bool xn) {
+  return n <= 64 ? launch_s<T, 1>(unif, xn) : n <= 128 ? launch_s<T, 2>(unif, xn) : launch_s<T, 4>(unif, xn);
+}
+
+}  // namespace
+
+// A step costs the same for any batch until the CUs hold several workgroups; from
+// then on the LDS and nn kernels, whose waves are full, overtake it.  Measured, us per
+// step, those kernels against this one:
+//   FP64, 1x64   256 trajectories 0.54 / 0.17, 1000 0.58 / 0.36, 2000 0.63 / 0.62, 4000 0.96 / 1.14
+//   FP64, 4x4, drawn F   100 trajectories 0.74 / 0.16, 2000 0.73 / 0.50, 4000 0.75 / 0.91
+//   FP64, 1x128  256 trajectories 0.55 / 0.23, 1000 0.63 / 0.60, 2000 0.96 / 1.10
+//   FP32, 1x64   256 trajectories 0.34 / 0.13, 2000 0.39 / 0.30, 4000 0.51 / 0.50, 8000 0.85 / 0.90
+//   FP32, 1x128, drawn F   256 trajectories 0.47 / 0.19, 4000 1.00 / 0.84
+//   FP64, 16x16  256 trajectories 0.67 / 0.42, 512 1.00 / 0.81, 1000 1.13 / 1.58
+//   FP32, 9x21   256 trajectories 0.50 / 0.36, 512 0.57 / 0.43, 2000 0.96 / 1.04
+bool ahead_pays(int nx, int ny, int precision, size_t n_traj, int cus) {
+  const int n = nx * ny;
+  const int per_cu = n > 128 ? 2 : precision == 32 ? 16 : n > 64 ? 4 : 8;
+  return ny > 1 && n <= 256 && n_traj <= (size_t)per_cu * cus;
+}
+
+hipError_t launch_ahead(const StepArgs& a, int precision, hipStream_t s) {
+  const Launch l = precision == 64 ? launch_t<double>(a.n, a.site_uniform != 0, a.nx > 1)
+                                   : launch_t<float>(a.n, a.site_uniform != 0, a.nx > 1);
+  if (l.lds > 65536) {
+    hipError_t e = hipFuncSetAttribute(l.f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)l.lds);
+    if (e != hipSuccess) return e;
+  }
+  void* args[] = {const_cast<StepArgs*>(&a)};
+  return hipLaunchKernel(l.f, dim3(a.n_traj), dim3(l.block), args, l.lds, s);
+}
+
+}  // namespace twmc

@@ -114,6 +114,7 @@ struct Ctx {
   int cap_grid = 0;  // stencil64: grid of the capture launch (the 64x64 FFT kernel's)
   SparsePlan sparse;  // LDS kernel, matrix hopping: its steps on the sparse kernel
   bool band_dense = false;  // banded kernel: the batch's form (band_dense)
+  bool ahead = false;       // LDS kernel, FFT hopping: its steps on the ahead kernel
   bool nn = false;          // LDS kernel, FFT hopping: its steps on the nn kernel
   int grid_nn = 0;   // LDS kernel, FFT hopping: grid of the nearest-neighbour step launch
   size_t lds_nn = 0;
@@ -519,7 +520,8 @@ struct Geometry {
   size_t lds_nn = 0;
   SparsePlan sparse;  // LDS kernel with matrix hopping: the step launch on the sparse kernel
   bool band_dense = false;
-  bool nn = false;  // LDS kernel with FFT hopping: the step launch on the nn kernel
+  bool ahead = false;  // LDS kernel with FFT hopping: the step launch on the ahead kernel
+  bool nn = false;     // LDS kernel with FFT hopping: the step launch on the nn kernel
 };
 
 int step_geometry(Ctx* c, size_t B, Geometry& geo) {
@@ -554,7 +556,9 @@ int step_geometry(Ctx* c, size_t B, Geometry& geo) {
     geo.lds = generic_lds_bytes(c->p.nx, c->p.ny, c->precision);
     HIPCHK(c, generic_occupancy(c->precision, c->n, geo.block, geo.lds, &per_cu));
     if (c->ell_m > 0) HIPCHK(c, sparse_plan(c->n, c->precision, c->ell_m, B, cus, &geo.sparse));
-    if (c->p.hopping == TWMC_HOP_FFT && c->ft_n == 0 &&
+    if (c->p.hopping == TWMC_HOP_FFT && c->ft_n == 0 && ahead_pays(c->p.nx, c->p.ny, c->precision, B, cus)) {
+      geo.ahead = true;
+    } else if (c->p.hopping == TWMC_HOP_FFT && c->ft_n == 0 &&
         nn_supported(c->p.nx, c->p.ny, c->precision, param_vary(c)) &&
         nn_pays(c->p.nx, c->p.ny, c->precision, param_vary(c), B, cus)) {
       int per_cu_nn = 0;
@@ -650,7 +654,9 @@ int advance_generic_fft(Ctx* c, const StepArgs& a, hipStream_t s) {
     sa.capture = 0;
     hipEvent_t e0 = nullptr;
     HIPCHK(c, timed(c, c->ev_step, s, true, e0));
-    if (c->nn)
+    if (c->ahead)
+      HIPCHK(c, launch_ahead(sa, c->precision, s));
+    else if (c->nn)
       HIPCHK(c, launch_nn(sa, c->precision, c->grid_nn, s));
     else
       HIPCHK(c, launch_generic_nn(sa, c->precision, c->grid_nn, c->lds_nn, s));
@@ -998,6 +1004,7 @@ int twmc_batch_begin(twmc_ctx* ctx, const twmc_batch_desc* d) {
     c->cap_grid = geo.cap_grid;
     c->sparse = geo.sparse;
     c->band_dense = geo.band_dense;
+    c->ahead = geo.ahead;
     c->nn = geo.nn;
     c->grid_nn = geo.grid_nn;
     c->lds_nn = geo.lds_nn;
@@ -1422,6 +1429,8 @@ int twmc_advance_noalloc(twmc_ctx* ctx, const uint64_t* d_traj_ids, uint64_t n_t
       HIPCHK(c, launch_fused64(a, geo.grid, s));
     } else if (c->kernel == TWMC_KERNEL_MFMA) {
       HIPCHK(c, launch_mfma(a, geo.grid, s));
+    } else if (geo.ahead) {
+      HIPCHK(c, launch_ahead(a, c->precision, s));
     } else if (geo.nn) {
       HIPCHK(c, launch_nn(a, c->precision, geo.grid_nn, s));
     } else if (c->p.hopping == TWMC_HOP_FFT) {

@@ -491,12 +491,27 @@ __global__ void __launch_bounds__(BLOCK) generic_step_kernel(StepArgs g) {
               } else {
                 cpx<T> r = rsl[i], u = Up[i], f = fv[i];
                 if (fs) f = mk(f.re + fdt * fs[i].re, f.im + fdt * fs[i].im);
-                T q = z.re * z.re + z.im * z.im - T(1);
-                cpx<T> c = mk(r.re + (-u.im) * q, r.im + u.re * q);
-                cpx<T> cb = cmul(c, z);
-                cpx<T> sdr = mk(cb.re + hh.re + (-f.im), cb.im + hh.im + f.re);
-                cpx<T> a = mk(sdr.re * dt, sdr.im * dt);
-                z = mk(z.re + a.re + dt4 * xr[h], z.im + a.im + dt4 * xi[h]);
+                if constexpr (NN) {
+                  // the site-uniform form, its constants scaled by dt here
+                  const T q = fma(z.re, z.re, fma(z.im, z.im, T(-1)));
+                  const T ci = fma(dt * u.re, q, dt * r.im), cr = fma(-(dt * u.im), q, dt * r.re);
+                  T dr = fma(dt4, xr[h], -dt * f.im);
+                  dr = fma(djv, si, dr);
+                  dr = fma(cr, z.re, dr);
+                  dr = fma(-ci, z.im, dr);
+                  T di = fma(dt4, xi[h], dt * f.re);
+                  di = fma(-djv, sr, di);
+                  di = fma(cr, z.im, di);
+                  di = fma(ci, z.re, di);
+                  z = mk(z.re + dr, z.im + di);
+                } else {
+                  T q = z.re * z.re + z.im * z.im - T(1);
+                  cpx<T> c = mk(r.re + (-u.im) * q, r.im + u.re * q);
+                  cpx<T> cb = cmul(c, z);
+                  cpx<T> sdr = mk(cb.re + hh.re + (-f.im), cb.im + hh.im + f.re);
+                  cpx<T> a = mk(sdr.re * dt, sdr.im * dt);
+                  z = mk(z.re + a.re + dt4 * xr[h], z.im + a.im + dt4 * xi[h]);
+                }
               }
               if constexpr (kSplit)
                 znew[h] = z;

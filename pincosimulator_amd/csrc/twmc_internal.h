@@ -255,6 +255,11 @@ bool nn_pays(int nx, int ny, int precision, int vary, size_t n_traj, int cus);
 hipError_t nn_occupancy(int nx, int ny, int precision, int vary, bool u_real, int* blocks_per_cu);
 hipError_t launch_nn(const StepArgs& a, int precision, int grid, hipStream_t s);
 
+// FFT hopping, up to 256 sites, static parameters: the step launch of the LDS kernel
+// (TWMC_KERNEL_GENERIC) for small batches, one workgroup per trajectory
+bool ahead_pays(int nx, int ny, int precision, size_t n_traj, int cus);
+hipError_t launch_ahead(const StepArgs& a, int precision, hipStream_t s);
+
 // matrix hopping with at most six nonzeros per column (`most`), up to 512 sites:
 // whole trajectories in a wave's registers, FP64 or FP32
 constexpr int kSparseMaxSites = 512;

@@ -114,6 +114,7 @@ struct Ctx {
   int cap_grid = 0;  // stencil64: grid of the capture launch (the 64x64 FFT kernel's)
   SparsePlan sparse;  // LDS kernel, matrix hopping: its steps on the sparse kernel
   bool band_dense = false;  // banded kernel: the batch's form (band_dense)
+  int tb = 0;               // MFMA kernel: trajectories per workgroup
   bool ahead = false;       // LDS kernel, FFT hopping: its steps on the ahead kernel
   bool nn = false;          // LDS kernel, FFT hopping: its steps on the nn kernel
   int grid_nn = 0;   // LDS kernel, FFT hopping: grid of the nearest-neighbour step launch
@@ -520,6 +521,7 @@ struct Geometry {
   size_t lds_nn = 0;
   SparsePlan sparse;  // LDS kernel with matrix hopping: the step launch on the sparse kernel
   bool band_dense = false;
+  int tb = 0;          // MFMA kernel: trajectories per workgroup
   bool ahead = false;  // LDS kernel with FFT hopping: the step launch on the ahead kernel
   bool nn = false;     // LDS kernel with FFT hopping: the step launch on the nn kernel
 };
@@ -547,10 +549,11 @@ int step_geometry(Ctx* c, size_t B, Geometry& geo) {
     geo.band_dense = band_dense(B, cus) && c->ft_n == 0;
     HIPCHK(c, band_occupancy(c->n, c->band_w, c->band_lieb, c->band_uni, geo.band_dense, &per_cu));
   } else if (c->kernel == TWMC_KERNEL_MFMA) {
-    geo.block = mfma_block(c->np);
-    geo.lds = mfma_lds_bytes(c->np);
-    units = (B + 31) / 32;
-    HIPCHK(c, mfma_occupancy(c->np, &per_cu));
+    geo.block = 512;
+    geo.tb = mfma_tb(c->np, B, cus);
+    geo.lds = mfma_lds_bytes(c->np, geo.tb);
+    units = (B + geo.tb - 1) / geo.tb;
+    HIPCHK(c, mfma_occupancy(c->n, geo.tb, &per_cu));
   } else {
     geo.block = 256;
     geo.lds = generic_lds_bytes(c->p.nx, c->p.ny, c->precision);
@@ -610,6 +613,7 @@ StepArgs shared_step_args(const Ctx* c) {
   a.a_hi = c->d_ahi.p;
   a.a_lo = c->d_alo.p;
   a.np = c->np;
+  a.tb = c->tb;
   a.ft_n = c->ft_n;
   a.ft_times = static_cast<const double*>(c->d_ft_times.p);
   a.ft_vals = c->d_ft_vals.p;
@@ -869,13 +873,12 @@ int twmc_create(const twmc_params* p, int device, twmc_ctx** ctx_out) {
     // A = C^T, zero-padded to np x np, split into BF16 high and low parts
     c->np = mfma_padded(c->n);
     const int np = c->np;
-    const int rows = mfma_rows(np);
-    std::vector<double> a((size_t)rows * np, 0.0);
+    std::vector<double> a((size_t)np * np, 0.0);
     for (int i = 0; i < c->n; ++i)
       for (int j = 0; j < c->n; ++j) a[(size_t)j * np + i] = p->coupling[(size_t)i * c->n + j];
     std::vector<double> as(a.size());
-    mfma_swizzle(a.data(), rows, np, as.data());
-    std::vector<uint16_t> hi((size_t)rows * np), lo((size_t)rows * np);
+    mfma_swizzle(a.data(), np, as.data());
+    std::vector<uint16_t> hi(a.size()), lo(a.size());
     mfma_split(as.data(), as.size(), hi.data(), lo.data());
     hipError_t ee = upload(c->d_ahi, hi.data(), hi.size() * 2, s);
     if (ee == hipSuccess) ee = upload(c->d_alo, lo.data(), lo.size() * 2, s);
@@ -1004,6 +1007,7 @@ int twmc_batch_begin(twmc_ctx* ctx, const twmc_batch_desc* d) {
     c->cap_grid = geo.cap_grid;
     c->sparse = geo.sparse;
     c->band_dense = geo.band_dense;
+    c->tb = geo.tb;
     c->ahead = geo.ahead;
     c->nn = geo.nn;
     c->grid_nn = geo.grid_nn;
@@ -1428,6 +1432,7 @@ int twmc_advance_noalloc(twmc_ctx* ctx, const uint64_t* d_traj_ids, uint64_t n_t
     } else if (c->kernel == TWMC_KERNEL_FUSED64) {
       HIPCHK(c, launch_fused64(a, geo.grid, s));
     } else if (c->kernel == TWMC_KERNEL_MFMA) {
+      a.tb = geo.tb;
       HIPCHK(c, launch_mfma(a, geo.grid, s));
     } else if (geo.ahead) {
       HIPCHK(c, launch_ahead(a, c->precision, s));

@@ -82,7 +82,8 @@ struct StepArgs {
   // MFMA matrix hopping: A = C^T split into BF16 high and low parts, [np][np]
   const void* a_hi;
   const void* a_lo;
-  int np;                    // n padded to a multiple of 32
+  int np;                    // n padded to a multiple of 128
+  int tb;                    // MFMA kernel: trajectories per workgroup
   unsigned int* queue;       // 64x64 stencil and nn kernels: work queue of the launch (one word)
   int u_real;                // 1: Im U = 0 at every site, in every trajectory
   int vary;                  // a bit for each of rsl, U, F: not one value for all sites and trajectories
@@ -212,7 +213,8 @@ hipError_t stencil64_occupancy(int* blocks_per_cu);
 // matrix hopping on MFMA (FP32 state, BF16 x 3 products, FP32 accumulation)
 bool mfma_supported(int n, int hopping, int precision, int param_stride);
 int mfma_padded(int n);
-size_t mfma_lds_bytes(int np);
+size_t mfma_lds_bytes(int np, int tb);
+int mfma_tb(int np, size_t n_traj, int cus);  // trajectories per workgroup
 hipError_t launch_mfma(const StepArgs& a, int grid, hipStream_t s);
 
 // one-point batches of the main API on the sweep kernel: FP32, FFT hopping,
@@ -274,12 +276,10 @@ bool sparse_supported(int n, int hopping, int most);
 hipError_t sparse_plan(int n, int precision, int most, size_t n_traj, int cus, SparsePlan* plan);
 hipError_t launch_sparse(const StepArgs& a, int precision, const SparsePlan& plan, hipStream_t s);
 
-hipError_t mfma_occupancy(int np, int* blocks_per_cu);
+hipError_t mfma_occupancy(int n, int tb, int* blocks_per_cu);
 // splits A (row-major np x np, FP64) into BF16 hi and lo parts (raw 16-bit)
 void mfma_split(const double* a, size_t count, uint16_t* hi, uint16_t* lo);
-int mfma_rows(int np);  // rows of the zero-padded A operand
-int mfma_block(int np);  // threads per workgroup of the MFMA step kernel
-void mfma_swizzle(const double* a, int rows, int np, double* out);  // row-major -> fragment order
+void mfma_swizzle(const double* a, int np, double* out);  // row-major -> fragment order
 
 }  // namespace twmc
 

@@ -1,7 +1,8 @@
 // twmc_sparse.hip -- step kernel for matrix hopping with few nonzeros per column
 // (the Lieb chain open or periodic, disordered chains, ladders and square
 // lattices) of up to 512 sites, in FP64, or in FP32 with parameters drawn per
-// trajectory: the cases the FP32 banded kernel does not take.
+// trajectory: the cases the FP32 banded kernel does not take (twmc_ahead.hip steps
+// small batches of them).
 //
 // The reference's Lieb solver applies h_j = -i sum_i beta_i C_ij with a sparse
 // product per step (TWMCLiebSolver.cpp:259-267).  Here a wave holds one or more
@@ -43,6 +44,9 @@ alignas(16) __device__ const double kF64TabDev[f64::kTabSize] = TWMC_F64_TABLES;
 template <typename T, bool PRIO>
 __device__ __forceinline__ void pair_noise(const u32x4& x, T sig, T (&re)[2], T (&im)[2], const f64::Series& k,
                                            const double* ltab) {
+  // rounded products: fused into the update in some forms of the step and not in
+  // others, they would make a trajectory's bits depend on the batch
+  TWMC_NO_CONTRACT
   if constexpr (sizeof(T) == 8) {
     const uint32_t a[2] = {x.x, x.z}, b[2] = {x.y, x.w};
     f64::box_muller<2>(a, b, re, im, k, ltab);

@@ -115,7 +115,7 @@ struct Ctx {
   SparsePlan sparse;  // LDS kernel, matrix hopping: its steps on the sparse kernel
   bool band_dense = false;  // banded kernel: the batch's form (band_dense)
   int tb = 0;               // MFMA kernel: trajectories per workgroup
-  bool ahead = false;       // LDS kernel, FFT hopping: its steps on the ahead kernel
+  bool ahead = false;       // LDS kernel: its steps on the ahead kernel
   bool nn = false;          // LDS kernel, FFT hopping: its steps on the nn kernel
   int grid_nn = 0;   // LDS kernel, FFT hopping: grid of the nearest-neighbour step launch
   size_t lds_nn = 0;
@@ -487,7 +487,10 @@ int advance_sparse(Ctx* c, const StepArgs& a, hipStream_t s) {
     sa.capture = 0;
     hipEvent_t e0 = nullptr;
     HIPCHK(c, timed(c, c->ev_step, s, true, e0));
-    HIPCHK(c, launch_sparse(sa, c->precision, c->sparse, s));
+    if (c->ahead)
+      HIPCHK(c, launch_ahead(sa, c->precision, s));
+    else
+      HIPCHK(c, launch_sparse(sa, c->precision, c->sparse, s));
     HIPCHK(c, timed(c, c->ev_step, s, false, e0));
     c->stats.site_steps += (uint64_t)a.n_steps * (uint64_t)n * c->n_traj;
   }
@@ -522,7 +525,7 @@ struct Geometry {
   SparsePlan sparse;  // LDS kernel with matrix hopping: the step launch on the sparse kernel
   bool band_dense = false;
   int tb = 0;          // MFMA kernel: trajectories per workgroup
-  bool ahead = false;  // LDS kernel with FFT hopping: the step launch on the ahead kernel
+  bool ahead = false;  // LDS kernel: the step launch on the ahead kernel
   bool nn = false;     // LDS kernel with FFT hopping: the step launch on the nn kernel
 };
 
@@ -558,7 +561,10 @@ int step_geometry(Ctx* c, size_t B, Geometry& geo) {
     geo.block = 256;
     geo.lds = generic_lds_bytes(c->p.nx, c->p.ny, c->precision);
     HIPCHK(c, generic_occupancy(c->precision, c->n, geo.block, geo.lds, &per_cu));
-    if (c->ell_m > 0) HIPCHK(c, sparse_plan(c->n, c->precision, c->ell_m, B, cus, &geo.sparse));
+    if (c->ell_m > 0) {
+      HIPCHK(c, sparse_plan(c->n, c->precision, c->ell_m, B, cus, &geo.sparse));
+      geo.ahead = c->ft_n == 0 && ahead_pays_sparse(c->n, c->ell_m, c->precision, B, cus);
+    }
     if (c->p.hopping == TWMC_HOP_FFT && c->ft_n == 0 && ahead_pays(c->p.nx, c->p.ny, c->precision, B, cus)) {
       geo.ahead = true;
     } else if (c->p.hopping == TWMC_HOP_FFT && c->ft_n == 0 &&

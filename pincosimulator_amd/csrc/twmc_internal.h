@@ -260,6 +260,8 @@ hipError_t launch_nn(const StepArgs& a, int precision, int grid, hipStream_t s);
 // FFT hopping, up to 256 sites, static parameters: the step launch of the LDS kernel
 // (TWMC_KERNEL_GENERIC) for small batches, one workgroup per trajectory
 bool ahead_pays(int nx, int ny, int precision, size_t n_traj, int cus);
+// matrix hopping with few nonzeros per column, up to 512 sites, static parameters: the same
+bool ahead_pays_sparse(int n, int most, int precision, size_t n_traj, int cus);
 hipError_t launch_ahead(const StepArgs& a, int precision, hipStream_t s);
 
 // matrix hopping with at most six nonzeros per column (`most`), up to 512 sites:

@@ -15,6 +15,7 @@
 #include <cstring>
 #include <mutex>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "../../include/twmc_hip.h"
@@ -63,7 +64,34 @@ struct DevBuf {
   }
 };
 
+// Pinned staging of large read-backs (read_states): two chunks per reader
+constexpr int kReaders = 4;
+constexpr size_t kStageBytes = 512 * 1024;
+constexpr size_t kStagedRead = 1024 * 1024;  // smaller ones are read in one piece
+struct Stage {
+  unsigned char* p = nullptr;
+  hipEvent_t done[2 * kReaders] = {};
+  hipError_t ensure() {
+    if (p) return hipSuccess;
+    for (hipEvent_t& e : done)
+      if (!e) {
+        hipError_t rc = hipEventCreateWithFlags(&e, hipEventDisableTiming);
+        if (rc != hipSuccess) return rc;
+      }
+    return hipHostMalloc(reinterpret_cast<void**>(&p), 2 * kReaders * kStageBytes, hipHostMallocDefault);
+  }
+  void release() {
+    for (hipEvent_t& e : done) {
+      if (e) (void)hipEventDestroy(e);
+      e = nullptr;
+    }
+    if (p) (void)hipHostFree(p);
+    p = nullptr;
+  }
+};
+
 struct Ctx {
+  Stage stage;
   std::string err;
   int device = 0;
   hipStream_t stream = nullptr;
@@ -115,6 +143,8 @@ struct Ctx {
   SparsePlan sparse;  // LDS kernel, matrix hopping: its steps on the sparse kernel
   bool band_dense = false;  // banded kernel: the batch's form (band_dense)
   int tb = 0;               // MFMA kernel: trajectories per workgroup
+  int vary = 0;              // scan_vary and scan_u_real: the parameters are fixed
+  bool u_is_real = false;
   bool ahead = false;       // LDS kernel: its steps on the ahead kernel
   bool nn = false;          // LDS kernel, FFT hopping: its steps on the nn kernel
   int grid_nn = 0;   // LDS kernel, FFT hopping: grid of the nearest-neighbour step launch
@@ -249,7 +279,7 @@ void plan_segments(Ctx* c) {
 }
 
 // a bit for each of rsl, U and F: drawn per trajectory, or not the same at every site
-int param_vary(const Ctx* c) {
+int scan_vary(const Ctx* c) {
   int v = 0;
   for (int k = 0; k < 3; ++k) {
     bool same = c->noise[k] == TWMC_NOISE_NONE;
@@ -262,10 +292,10 @@ int param_vary(const Ctx* c) {
 
 // rsl, U and F the same at every site and in every trajectory, F static: the
 // tables the init kernel forms are then uniform
-bool site_uniform(const Ctx* c) { return c->ft_n == 0 && param_vary(c) == 0; }
+bool site_uniform(const Ctx* c) { return c->ft_n == 0 && c->vary == 0; }
 
 // Im U = 0 at every site, in every trajectory
-bool u_real(const Ctx* c) {
+bool scan_u_real(const Ctx* c) {
   if (c->noise[1] != TWMC_NOISE_NONE) return false;
   for (int i = 0; i < c->n; ++i)
     if (c->base[1][2 * i + 1] != 0.0) return false;
@@ -568,10 +598,10 @@ int step_geometry(Ctx* c, size_t B, Geometry& geo) {
     if (c->p.hopping == TWMC_HOP_FFT && c->ft_n == 0 && ahead_pays(c->p.nx, c->p.ny, c->precision, B, cus)) {
       geo.ahead = true;
     } else if (c->p.hopping == TWMC_HOP_FFT && c->ft_n == 0 &&
-        nn_supported(c->p.nx, c->p.ny, c->precision, param_vary(c)) &&
-        nn_pays(c->p.nx, c->p.ny, c->precision, param_vary(c), B, cus)) {
+        nn_supported(c->p.nx, c->p.ny, c->precision, c->vary) &&
+        nn_pays(c->p.nx, c->p.ny, c->precision, c->vary, B, cus)) {
       int per_cu_nn = 0;
-      HIPCHK(c, nn_occupancy(c->p.nx, c->p.ny, c->precision, param_vary(c), u_real(c), &per_cu_nn));
+      HIPCHK(c, nn_occupancy(c->p.nx, c->p.ny, c->precision, c->vary, c->u_is_real, &per_cu_nn));
       if (per_cu_nn < 1) return fail(c, TWMC_ERR_UNSUPPORTED, "step kernel does not fit on a CU");
       geo.nn = true;
       geo.grid_nn = (int)std::min<size_t>(B, (size_t)per_cu_nn * cus);
@@ -625,8 +655,8 @@ StepArgs shared_step_args(const Ctx* c) {
   a.ft_vals = c->d_ft_vals.p;
   a.ft_slopes = c->d_ft_slopes.p;
   a.site_uniform = site_uniform(c) ? 1 : 0;
-  a.u_real = u_real(c) ? 1 : 0;
-  a.vary = param_vary(c);
+  a.u_real = c->u_is_real ? 1 : 0;
+  a.vary = c->vary;
   a.band_coef = static_cast<const float*>(c->d_band.p);
   a.band_w = c->band_w;
   a.band_lieb = c->band_lieb;
@@ -673,6 +703,70 @@ int advance_generic_fft(Ctx* c, const StepArgs& a, hipStream_t s) {
     HIPCHK(c, timed(c, c->ev_step, s, false, e0));
     c->stats.site_steps += (uint64_t)a.n_steps * (uint64_t)n * c->n_traj;
   }
+  return TWMC_OK;
+}
+
+// `count` complex states from device memory into FP64 at dst.  FP32 states from 1 MiB
+// on go in chunks through pinned memory, each converted by one of four threads while
+// the next ones are on their way: the copy through a pageable buffer and one thread's
+// conversion took longer than the run (64 trajectories of 64x64, three frames, 12.6 MB
+// here: the whole call 1.20 -> 0.86 ms).  FP64 states are copied as they are: the same
+// way through pinned memory was no faster there (5.5 MB: the call 1.15 and 1.17 ms).
+int read_states(Ctx* c, const void* src, size_t count, double* dst) {
+  if (c->precision == 64) {
+    HIPCHK(c, hipMemcpy(dst, src, count * 16, hipMemcpyDeviceToHost));
+    return TWMC_OK;
+  }
+  const size_t bytes = count * 8;
+  if (bytes < kStagedRead) {
+    std::vector<float> tmp(count * 2);
+    HIPCHK(c, hipMemcpy(tmp.data(), src, bytes, hipMemcpyDeviceToHost));
+    for (size_t i = 0; i < count * 2; ++i) dst[i] = tmp[i];
+    return TWMC_OK;
+  }
+  HIPCHK(c, c->stage.ensure());
+  const size_t chunks = (bytes + kStageBytes - 1) / kStageBytes;
+  auto reader = [&](int w) -> hipError_t {  // chunks w, w + kReaders, ...
+    hipError_t e = hipSetDevice(c->device);
+    auto slot = [&](size_t k) { return 2 * w + (int)((k / kReaders) & 1); };
+    auto size = [&](size_t k) { return std::min(kStageBytes, bytes - k * kStageBytes); };
+    auto fetch = [&](size_t k) {
+      if (e != hipSuccess || k >= chunks) return;
+      e = hipMemcpyAsync(c->stage.p + slot(k) * kStageBytes, static_cast<const unsigned char*>(src) + k * kStageBytes,
+                         size(k), hipMemcpyDeviceToHost, c->stream);
+      if (e == hipSuccess) e = hipEventRecord(c->stage.done[slot(k)], c->stream);
+    };
+    fetch(w);
+    for (size_t k = w; k < chunks && e == hipSuccess; k += kReaders) {
+      fetch(k + kReaders);
+      if (e == hipSuccess) e = hipEventSynchronize(c->stage.done[slot(k)]);
+      if (e != hipSuccess) break;
+      const float* x = reinterpret_cast<const float*>(c->stage.p + slot(k) * kStageBytes);
+      double* d = dst + k * (kStageBytes / 4);
+      for (size_t i = 0; i < size(k) / 4; ++i) d[i] = x[i];
+    }
+    return e;
+  };
+  hipError_t rc[kReaders] = {};
+  std::thread threads[kReaders];
+  for (int w = 1; w < kReaders; ++w) {
+    try {
+      threads[w] = std::thread([&, w] { rc[w] = reader(w); });
+    } catch (...) {  // no thread to be had: its chunks are read below
+    }
+  }
+  rc[0] = reader(0);
+  for (int w = 1; w < kReaders; ++w) {
+    if (threads[w].joinable())
+      threads[w].join();
+    else
+      rc[w] = reader(w);
+  }
+  // nothing is left in flight towards the staging memory, whatever failed
+  hipError_t e = hipStreamSynchronize(c->stream);
+  for (int w = 0; w < kReaders; ++w)
+    if (rc[w] != hipSuccess) e = rc[w];
+  HIPCHK(c, e);
   return TWMC_OK;
 }
 
@@ -747,6 +841,8 @@ int twmc_create(const twmc_params* p, int device, twmc_ctx** ctx_out) {
   c->p.omega.base = c->p.U.base = c->p.F.base = c->p.beta_init.base = c->p.beta_sigma.base = nullptr;
   c->p.omega.amp = c->p.U.amp = c->p.F.amp = c->p.beta_init.amp = c->p.beta_sigma.amp = nullptr;
   c->noisy_params = (c->noise[0] || c->noise[1] || c->noise[2]) ? 1 : 0;
+  c->vary = scan_vary(c);
+  c->u_is_real = scan_u_real(c);
 
   if (p->hopping == TWMC_HOP_FFT) {
     if (!make_radix_plan(p->nx, c->px) || !make_radix_plan(p->ny, c->py)) {
@@ -949,6 +1045,7 @@ void twmc_destroy(twmc_ctx* ctx) {
     c->d_base[k].release();
     c->d_amp[k].release();
   }
+  c->stage.release();
   if (c->stream) (void)hipStreamDestroy(c->stream);
   delete c;
 }
@@ -1264,26 +1361,16 @@ int twmc_batch_read(twmc_ctx* ctx, twmc_output* out) {
   }
   if (nf > 0 && out->traj_m2) HIPCHK(c, hipMemcpy(out->traj_m2, c->d_m2.p, B * nf * 8, hipMemcpyDeviceToHost));
   if (nf > 0 && out->traj_m4) HIPCHK(c, hipMemcpy(out->traj_m4, c->d_m4.p, B * nf * 8, hipMemcpyDeviceToHost));
-  auto to_f64 = [&](const DevBuf& b, size_t count, double* dst) -> int {
-    if (c->precision == 64) {
-      HIPCHK(c, hipMemcpy(dst, b.p, count * 16, hipMemcpyDeviceToHost));
-    } else {
-      std::vector<float> tmp(count * 2);
-      HIPCHK(c, hipMemcpy(tmp.data(), b.p, count * 8, hipMemcpyDeviceToHost));
-      for (size_t i = 0; i < count * 2; ++i) dst[i] = tmp[i];
-    }
-    return TWMC_OK;
-  };
   if (out->traj) {
     if (!(c->desc.outputs & TWMC_OUT_TRAJ))
       return fail(c, TWMC_ERR_STATE, "trajectory frames were not requested (TWMC_OUT_TRAJ)");
     if (nf > 0) {
-      int rc = to_f64(c->d_traj, B * nf * n, out->traj);
+      int rc = read_states(c, c->d_traj.p, B * nf * n, out->traj);
       if (rc) return rc;
     }
   }
   if (out->beta_final) {
-    int rc = to_f64(c->d_beta, B * n, out->beta_final);
+    int rc = read_states(c, c->d_beta.p, B * n, out->beta_final);
     if (rc) return rc;
   }
   return TWMC_OK;

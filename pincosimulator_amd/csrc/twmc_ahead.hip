@@ -150,6 +150,16 @@ __global__ void __launch_bounds__(64 * waves_of(SPL)) ahead_step_kernel(StepArgs
   }
   if (M > 0 && threadIdx.x == 0) lds.st[64 * SPL] = mk(T(0), T(0));
 
+  int due = 0, frame = 0;  // steps to the next stored frame, frames stored
+  auto store_frame = [&] {
+    cpx<T>* out = reinterpret_cast<cpx<T>*>(g.frames) + ((size_t)b * g.frames_stride + g.frame0 + frame) * n;
+#pragma unroll
+    for (int j = 0; j < SPL; ++j)
+      if (lane + 64 * j < n) out[lane + 64 * j] = z[j];
+    ++frame;
+    due = g.group_steps;
+  };
+
   produce(0, 0, wave, kWaves);
   __syncthreads();
   for (int s0 = 0, c = 0; s0 < g.n_steps; s0 += ksteps, c ^= 1) {
@@ -160,6 +170,10 @@ __global__ void __launch_bounds__(64 * waves_of(SPL)) ahead_step_kernel(StepArgs
 #pragma unroll
       for (int j = 0; j < SPL; ++j) xi[j] = row[64 * j];
       for (int k = 0; k < steps; ++k) {
+        if (due-- == 0 && frame < g.group) {
+          store_frame();
+          --due;
+        }
 #pragma unroll
         for (int j = 0; j < SPL; ++j) lds.st[lane + 64 * j] = z[j];
         lds_order();
@@ -224,6 +238,7 @@ __global__ void __launch_bounds__(64 * waves_of(SPL)) ahead_step_kernel(StepArgs
     }
     __syncthreads();
   }
+  if (wave == 0 && frame < g.group) store_frame();  // the state after the last step
 #pragma unroll
   for (int j = 0; j < SPL; ++j) {
     const int i = lane + 64 * j;

@@ -118,7 +118,7 @@ struct Ctx {
   int ell_m = 0;      // TWMC_KERNEL_GENERIC, matrix hopping: entries per column of the sparse kernel, 0: not used
   StackPlan stack;  // TWMC_KERNEL_STACK: the batch's point and work items on the sweep kernel
   // per-batch buffers
-  DevBuf d_ids, d_beta, d_rsl, d_U, d_F, d_partials, d_obs, d_m2, d_m4, d_traj, d_prev;
+  DevBuf d_ids, d_beta, d_rsl, d_U, d_F, d_partials, d_obs, d_m2, d_m4, d_traj, d_prev, d_frames;
   int csc_nnz = 0;
   // batch state
   bool batch_active = false;
@@ -143,6 +143,7 @@ struct Ctx {
   SparsePlan sparse;  // LDS kernel, matrix hopping: its steps on the sparse kernel
   bool band_dense = false;  // banded kernel: the batch's form (band_dense)
   int tb = 0;               // MFMA kernel: trajectories per workgroup
+  int group = 1, group_slots = 0;  // ahead kernel: most frames in one launch, their partial slots
   int vary = 0;              // scan_vary and scan_u_real: the parameters are fixed
   bool u_is_real = false;
   bool ahead = false;       // LDS kernel: its steps on the ahead kernel
@@ -595,7 +596,8 @@ int step_geometry(Ctx* c, size_t B, Geometry& geo) {
       HIPCHK(c, sparse_plan(c->n, c->precision, c->ell_m, B, cus, &geo.sparse));
       geo.ahead = c->ft_n == 0 && ahead_pays_sparse(c->n, c->ell_m, c->precision, B, cus);
     }
-    if (c->p.hopping == TWMC_HOP_FFT && c->ft_n == 0 && ahead_pays(c->p.nx, c->p.ny, c->precision, B, cus)) {
+    if (c->kernel == TWMC_KERNEL_GENERIC && c->p.hopping == TWMC_HOP_FFT && c->ft_n == 0 &&
+        ahead_pays(c->p.nx, c->p.ny, c->precision, B, cus)) {
       geo.ahead = true;
     } else if (c->p.hopping == TWMC_HOP_FFT && c->ft_n == 0 &&
         nn_supported(c->p.nx, c->p.ny, c->precision, c->vary) &&
@@ -767,6 +769,76 @@ int read_states(Ctx* c, const void* src, size_t count, double* dst) {
   for (int w = 0; w < kReaders; ++w)
     if (rc[w] != hipSuccess) e = rc[w];
   HIPCHK(c, e);
+  return TWMC_OK;
+}
+
+// Most frames that a launch of the ahead kernel takes: it stores the states of
+// several (into the trajectory output if it was asked for), whose sums one capture
+// and one reduction launch then form.  A frame of a small lattice is otherwise three
+// launches of which the steps are a small part (256 trajectories of 64 sites, FP64, 21
+// frames of 200 steps: the call 1.17 -> 1.00 ms; 100 of 4x4, 21 of 100: 0.67 -> 0.46).  The states and the
+// partial sums of a group stay within 16 MiB each, its steps within 16384 (a few ms).
+void plan_group(Ctx* c, size_t B) {
+  c->group = 1;
+  c->group_slots = 0;
+  if (!c->ahead || !generic_capture_overwrites(c->n)) return;
+  size_t most = std::min<size_t>({(size_t)c->n_frames, 64, 16384 / (size_t)c->p.frame_steps});
+  for (; most > 1; most /= 2) {
+    const size_t slots = std::min<size_t>(c->grid, std::max<size_t>(16, 2048 / most));
+    if (B * most * c->n * c->es <= (16u << 20) && most * slots * kQ * c->n * sizeof(double) <= (16u << 20)) {
+      c->group = (int)most;
+      c->group_slots = (int)slots;
+      return;
+    }
+  }
+}
+
+// segments from k on that one launch of the ahead kernel can take: each stores a
+// frame first, all but the last have the same number of steps
+int group_size(const Ctx* c, size_t k, uint64_t most) {
+  if (c->group < 2) return 1;
+  most = std::min<uint64_t>({most, (uint64_t)c->group, c->segs.size() - k});
+  uint64_t m = 0;
+  while (m < most && c->segs[k + m].capture && c->segs[k + m].frame == c->segs[k].frame + (int)m &&
+         (m == 0 || c->segs[k + m - 1].steps == c->segs[k].steps) && c->segs[k + m].steps <= 16384)
+    ++m;
+  return m > 1 && c->segs[k].steps > 0 ? (int)m : 1;
+}
+
+uint64_t sum_steps(const Ctx* c, size_t k, int m) {
+  uint64_t steps = 0;
+  for (int j = 0; j < m; ++j) steps += c->segs[k + j].steps;
+  return steps;
+}
+
+// `m` segments, a.n_steps steps in all, with the frames a.frame ..
+int advance_group(Ctx* c, StepArgs a, int m, hipStream_t s) {
+  a.group = m;
+  a.group_steps = (int)c->segs[c->next_seg].steps;
+  a.frames = a.dump ? c->d_traj.p : c->d_frames.p;
+  a.frames_stride = a.dump ? a.n_frames : c->group;
+  a.frame0 = a.dump ? a.frame : 0;
+  a.dump = 0;
+  a.capture = 0;
+  hipEvent_t e0 = nullptr, r0 = nullptr;
+  HIPCHK(c, timed(c, c->ev_step, s, true, e0));
+  HIPCHK(c, launch_ahead(a, c->precision, s));
+  HIPCHK(c, timed(c, c->ev_step, s, false, e0));
+  c->stats.site_steps += (uint64_t)a.n_steps * (uint64_t)c->n * c->n_traj;
+  HIPCHK(c, timed(c, c->ev_red, s, true, r0));
+  a.capture = 1;
+  a.n_steps = 0;
+  HIPCHK(c, launch_generic(a, c->precision, c->group_slots, c->block, c->lds, s));
+  ReduceArgs r{};
+  r.n = c->n;
+  r.slots = c->group_slots;
+  r.keep = 1;
+  r.frames = m;
+  r.partials_in = static_cast<const double*>(c->d_partials.p);
+  r.partials = static_cast<double*>(c->d_partials.p);
+  r.obs = static_cast<double*>(c->d_obs.p) + (size_t)a.frame * kQ * c->n;
+  HIPCHK(c, launch_reduce(r, s));
+  HIPCHK(c, timed(c, c->ev_red, s, false, r0));
   return TWMC_OK;
 }
 
@@ -1039,7 +1111,7 @@ void twmc_destroy(twmc_ctx* ctx) {
                     &c->d_ft_times,  &c->d_ft_vals,  &c->d_ft_slopes, &c->d_band, &c->d_ids,  &c->d_beta,
                     &c->d_ell_coef,  &c->d_ell_row, &c->d_queue,
                     &c->d_rsl,       &c->d_U,        &c->d_F,         &c->d_partials, &c->d_obs, &c->d_m2,
-                    &c->d_m4,        &c->d_traj,     &c->d_prev};
+                    &c->d_m4,        &c->d_traj,     &c->d_prev,      &c->d_frames};
   for (DevBuf* b : bufs) b->release();
   for (int k = 0; k < 5; ++k) {
     c->d_base[k].release();
@@ -1145,7 +1217,9 @@ int twmc_batch_begin(twmc_ctx* ctx, const twmc_batch_desc* d) {
   int ss_chunk = 0;
   const int slots = std::max({c->grid, c->cap_grid, site_sum_chunks(B, kSiteSumChunks, &ss_chunk)});
   size_t part_bytes = (size_t)slots * kQ * n * sizeof(double);
-  HIPCHK(c, c->d_partials.ensure(part_bytes));
+  plan_group(c, B);
+  HIPCHK(c, c->d_partials.ensure(std::max(part_bytes, (size_t)c->group * c->group_slots * kQ * n * sizeof(double))));
+  if (c->group > 1 && !(d->outputs & TWMC_OUT_TRAJ)) HIPCHK(c, c->d_frames.ensure(B * c->group * n * c->es));
   // only the launches that add to their rows need them cleared (168 MB for the
   // 64x64 ensemble's 1024 slots): the capture inside a step launch, and the
   // LDS kernel's capture of a lattice above generic_capture_overwrites
@@ -1231,10 +1305,11 @@ int twmc_batch_advance(twmc_ctx* ctx, uint64_t n_segments) {
   HIPCHK(c, hipSetDevice(c->device));
   hipStream_t s = c->stream;
   const int n = c->n;
-  for (uint64_t k = 0; k < n_segments && c->next_seg < c->segs.size(); ++k) {
+  for (uint64_t k = 0; k < n_segments && c->next_seg < c->segs.size();) {
     const Segment& sg = c->segs[c->next_seg];
+    const int m = group_size(c, c->next_seg, n_segments - k);
     // a segment longer than 2^31 steps is split; captures stay on the first piece
-    uint64_t left = sg.steps;
+    uint64_t left = sum_steps(c, c->next_seg, m);
     bool first = true;
     do {
       int steps = (int)std::min<uint64_t>(left, 1u << 30);
@@ -1257,7 +1332,10 @@ int twmc_batch_advance(twmc_ctx* ctx, uint64_t n_segments) {
       a.traj_out = c->d_traj.p;
       a.queue = static_cast<unsigned int*>(c->d_queue.p);
       a.t0 = c->desc.t_start + double(c->steps_done) * c->p.dt;
-      if (c->kernel == TWMC_KERNEL_STENCIL64) {
+      if (m > 1) {
+        int rc = advance_group(c, a, m, s);
+        if (rc != TWMC_OK) return rc;
+      } else if (c->kernel == TWMC_KERNEL_STENCIL64) {
         int rc = advance_stencil(c, a, s);
         if (rc != TWMC_OK) return rc;
       } else if (c->kernel == TWMC_KERNEL_BAND) {
@@ -1318,13 +1396,15 @@ int twmc_batch_advance(twmc_ctx* ctx, uint64_t n_segments) {
       left -= (uint64_t)steps;
       first = false;
     } while (left > 0);
-    {
+    uint64_t done = c->steps_done - sum_steps(c, c->next_seg, m);
+    for (int j = 0; j < m; ++j, ++k) {
       std::lock_guard<std::mutex> lk(c->prog_mu);
       HIPCHK(c, hipEventRecord(c->seg_ev[c->next_seg], s));
-      c->seg_steps[c->next_seg] = c->steps_done;
+      done += c->segs[c->next_seg].steps;
+      c->seg_steps[c->next_seg] = done;
       c->seg_recorded = c->next_seg + 1;
+      c->next_seg++;
     }
-    c->next_seg++;
   }
   return TWMC_OK;
 }

@@ -590,9 +590,12 @@ __global__ void __launch_bounds__(BLOCK) generic_capture_kernel(StepArgs g) {
   }
   const int wave = tid >> 6, lane = tid & 63;
 
+  const int frame = g.frame + (int)blockIdx.y;
   for (int b = blockIdx.x; b < g.n_traj; b += gridDim.x) {
-    const cpx<T>* gbeta = reinterpret_cast<const cpx<T>*>(g.beta) + (size_t)b * n;
-    cpx<T>* out = g.dump ? reinterpret_cast<cpx<T>*>(g.traj_out) + ((size_t)b * g.n_frames + g.frame) * n : nullptr;
+    const cpx<T>* gbeta = g.group > 0 ? reinterpret_cast<const cpx<T>*>(g.frames) +
+                                            ((size_t)b * g.frames_stride + g.frame0 + blockIdx.y) * n
+                                      : reinterpret_cast<const cpx<T>*>(g.beta) + (size_t)b * n;
+    cpx<T>* out = g.dump ? reinterpret_cast<cpx<T>*>(g.traj_out) + ((size_t)b * g.n_frames + frame) * n : nullptr;
     double m2 = 0.0, m4 = 0.0;
 #pragma unroll
     for (int j = 0; j < PPT; ++j) {
@@ -627,8 +630,8 @@ __global__ void __launch_bounds__(BLOCK) generic_capture_kernel(StepArgs g) {
         a2 += red[2 * w];
         a4 += red[2 * w + 1];
       }
-      g.traj_m2[(size_t)b * g.n_frames + g.frame] = a2 / double(n);
-      g.traj_m4[(size_t)b * g.n_frames + g.frame] = a4 / double(n);
+      g.traj_m2[(size_t)b * g.n_frames + frame] = a2 / double(n);
+      g.traj_m4[(size_t)b * g.n_frames + frame] = a4 / double(n);
     }
     if (g.hopping == 0) {
       const cpx<T>* cur = fft2d<-1>(bufA, bufB, g, twx, twy);
@@ -644,7 +647,7 @@ __global__ void __launch_bounds__(BLOCK) generic_capture_kernel(StepArgs g) {
     __syncthreads();  // the next trajectory overwrites the LDS state and the wave sums
   }
 
-  double* part = g.partials + (size_t)blockIdx.x * kQ * n;
+  double* part = g.partials + ((size_t)blockIdx.y * gridDim.x + blockIdx.x) * kQ * n;
 #pragma unroll
   for (int j = 0; j < PPT; ++j) {
     const int p = tid + BLOCK * j;
@@ -823,7 +826,7 @@ __global__ void __launch_bounds__(kRedOut* kRedGroups) reduce_kernel(ReduceArgs 
   double s = 0.0;
   if (idx < total) {
     const int ns = (idx / a.n == 2 && a.slots_k > 0) ? a.slots_k : a.slots;
-    const double* in = a.partials_in + idx;
+    const double* in = a.partials_in + (size_t)blockIdx.y * a.slots * total + idx;
     int sl = g;
     for (; sl + 15 * kRedGroups < ns; sl += 16 * kRedGroups) {
       double v[16];
@@ -844,7 +847,7 @@ __global__ void __launch_bounds__(kRedOut* kRedGroups) reduce_kernel(ReduceArgs 
     for (int u = 0; u < kRedGroups; ++u) s += sums[u][o];
     const int q = idx / a.n, j = idx - q * a.n;
     const int* perm = (q == 2) ? a.perm_k : a.perm_site;
-    a.obs[q * a.n + (perm ? perm[j] : j)] = s;
+    a.obs[(size_t)blockIdx.y * total + q * a.n + (perm ? perm[j] : j)] = s;
   }
 }
 
@@ -864,7 +867,7 @@ hipError_t launch_generic_capture_t(const StepArgs& a, int grid, size_t lds, hip
     hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) return e;
   }
-  hipLaunchKernelGGL((generic_capture_kernel<T, PPT, BLOCK>), dim3(grid), dim3(BLOCK), lds, s, a);
+  hipLaunchKernelGGL((generic_capture_kernel<T, PPT, BLOCK>), dim3(grid, std::max(1, a.group)), dim3(BLOCK), lds, s, a);
   return hipGetLastError();
 }
 
@@ -1076,7 +1079,7 @@ hipError_t launch_gauss_init(const GaussArgs& a, int precision, int grid, hipStr
 
 hipError_t launch_reduce(const ReduceArgs& a, hipStream_t s) {
   const int grid = (kQ * a.n + kRedOut - 1) / kRedOut;
-  hipLaunchKernelGGL(reduce_kernel, dim3(grid), dim3(kRedOut * kRedGroups), 0, s, a);
+  hipLaunchKernelGGL(reduce_kernel, dim3(grid, std::max(1, a.frames)), dim3(kRedOut * kRedGroups), 0, s, a);
   return hipGetLastError();
 }
 

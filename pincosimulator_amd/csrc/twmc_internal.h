@@ -85,6 +85,12 @@ struct StepArgs {
   int np;                    // n padded to a multiple of 128
   int tb;                    // MFMA kernel: trajectories per workgroup
   unsigned int* queue;       // 64x64 stencil and nn kernels: work queue of the launch (one word)
+  // several frames in one launch (ahead kernel, capture-only launch of the LDS kernel):
+  // frame0 + k, k < group, lies at frames[trajectory][frames_stride][n]; the steps
+  // store it after k group_steps steps
+  void* frames;
+  int frames_stride, frame0, group;
+  int group_steps;
   int u_real;                // 1: Im U = 0 at every site, in every trajectory
   int vary;                  // a bit for each of rsl, U, F: not one value for all sites and trajectories
   int site_uniform;          // 1: rsl, U and F are the same at every site and in every trajectory, F static
@@ -161,6 +167,7 @@ struct ReduceArgs {
   const int* perm_k;
   int slots_k;  // slots of the k-space row (q = 2) when > 0, else slots
   int keep;     // 1: the producers overwrite their rows, no clearing
+  int frames;   // consecutive frames, each with its own slots (0: one)
 };
 
 // per-site real-space sums in site-major order (rows 0, 1, 3, 4 of the slots);

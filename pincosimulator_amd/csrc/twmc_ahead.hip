@@ -30,7 +30,10 @@ namespace {
 alignas(16) __device__ const double kF64TabDev[f64::kTabSize] = TWMC_F64_TABLES;
 
 constexpr int waves_of(int spl) { return spl >= 4 ? 8 : 4; }
-constexpr int chunk_sites(int spl) { return spl == 8 ? 3072 : spl == 4 ? 2048 : 1024; }  // noise of a chunk: steps x sites (rounded up to even)
+// noise of a chunk: steps x sites (rounded up to even).  512: the LDS then holds six
+// workgroups per CU, with 1024 three (1000 trajectories of 72 sites, FP64: 0.46 ->
+// 0.40 us per step; up to 768 the same)
+constexpr int chunk_sites(int spl) { return spl == 8 ? 3072 : spl == 4 ? 2048 : 512; }
 constexpr int kChunkSteps = 64;    // at most
 
 template <typename T>

@@ -254,7 +254,7 @@ hipError_t launch_band(const StepArgs& a, int grid, hipStream_t s);
 bool band_dense(size_t n_traj, int cus);  // the batch fills the SIMDs: StepArgs::band_dense
 hipError_t band_occupancy(int n, int w, int lieb, int uni, int dense, int* blocks_per_cu);
 
-// FFT hopping, 129 to 4096 sites, static parameters of which at most one varies from
+// FFT hopping, 65 (129: FP64, even rows) to 4096 sites, static parameters of which at most one varies from
 // site to site or is drawn (StepArgs::vary); FP32 uniform lattices only with odd rows
 // (the stacked kernel takes the even ones): the step launch of the LDS kernel
 // (TWMC_KERNEL_GENERIC) where it pays; needs StepArgs::queue

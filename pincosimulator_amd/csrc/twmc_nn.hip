@@ -1,4 +1,4 @@
-// twmc_nn.hip -- step kernel for periodic lattices of 129 to 4096 sites, the hopping
+// twmc_nn.hip -- step kernel for periodic lattices of 65 to 4096 sites, the hopping
 // in its nearest-neighbour form (the exact real-space form of the reference's FFT
 // product, TWMCBaseSolver.cpp:80-88, :235-242): FP64, and the FP32 lattices that the
 // stacked kernel does not take (rows of odd length, an energy or a drive that varies
@@ -245,7 +245,8 @@ Launch launch_x(bool xn) {
 template <typename T, int V, bool ODD, bool UI0>
 Launch launch_s(int n, bool xn) {
   const int np = (n + 1) / 2;
-  return np <= 128    ? launch_x<T, 128, 1, V, ODD, UI0>(xn)
+  return np <= 64     ? launch_x<T, 64, 1, V, ODD, UI0>(xn)
+         : np <= 128  ? launch_x<T, 128, 1, V, ODD, UI0>(xn)
          : np <= 256  ? launch_x<T, 256, 1, V, ODD, UI0>(xn)
          : np <= 512  ? launch_x<T, 512, 1, V, ODD, UI0>(xn)
          : np <= 1024 ? launch_x<T, 1024, 1, V, ODD, UI0>(xn)
@@ -282,10 +283,16 @@ hipError_t allow_lds(const Launch& l) {
 
 }  // namespace
 
+// From 65 sites on (below, the LDS kernel packs two or four trajectories into a wave),
+// FP64 with even rows from 129 on: there the LDS kernel's two waves of one trajectory
+// are as fast.  us per step, LDS kernel against this one, 4500 / 10000 trajectories:
+// FP32 5x13 1.43, 2.55 to 1.01, 1.80, 8x16 with a drawn F 1.30, 2.44 to 1.04, 1.88; FP64 5x13
+// 2.60, 5.11 to 2.26, 4.69, 8x16 with a drawn F 2.56, 5.9 to 2.72, 4.81 (4x8 and 7x9,
+// FP64, 4500: 1.60, 1.72 to 2.52, 2.17).
 bool nn_supported(int nx, int ny, int precision, int vary) {
   const int n = nx * ny;
-  return (vary == kVaryNone || vary == kVaryRsl || vary == kVaryF) && ny > 1 && n > 128 && n <= 4096 &&
-         (precision == 64 || vary != kVaryNone || ny % 2);
+  return (vary == kVaryNone || vary == kVaryRsl || vary == kVaryF) && ny > 1 && n <= 4096 &&
+         n > (precision == 64 && ny % 2 == 0 ? 128 : 64) && (precision == 64 || vary != kVaryNone || ny % 2);
 }
 
 // Two pairs per thread (above 2048 sites) and at most two trajectories per CU: the LDS

@@ -691,51 +691,58 @@ __device__ void gen_param(const InitArgs& a, int which, uint32_t tag, uint64_t t
   im += zi * a.amp[which][2 * i + 1];
 }
 
+// One site pair per thread and pass: the state's Philox draw and trajectory once for both.
+// Bound by VALU work, of which a 64-bit division per site and a second Philox draw per
+// pair were a third: 16384 trajectories of 64x64, FP32, 1.06 -> 0.66 ms.
 template <typename T>
 __global__ void init_kernel(InitArgs a) {
-  const size_t total = (size_t)a.n_traj * a.n;
-  for (size_t idx = blockIdx.x * (size_t)blockDim.x + threadIdx.x; idx < total;
-       idx += (size_t)gridDim.x * blockDim.x) {
-    int b = (int)(idx / a.n);
-    int i = (int)(idx - (size_t)b * a.n);
-    uint64_t traj = a.traj_ids[b];
-    cpx<T>* beta = reinterpret_cast<cpx<T>*>(a.beta) + (size_t)b * a.n;
-    if (a.mode == 0) {
-      double br, bi, sr, si;
-      gen_param(a, 3, TAG_BINIT, traj, i, br, bi);
-      gen_param(a, 4, TAG_BSIGMA, traj, i, sr, si);
-      u32x4 x = philox4x32_10(make_counter(traj, TAG_INIT, 0u, (uint32_t)(i >> 1)), a.key0, a.key1);
-      double zr, zi;
-      if (i & 1) box_muller_f64(x.z, x.w, zr, zi); else box_muller_f64(x.x, x.y, zr, zi);
-      // beta_init + sigma (.) xi, complex product (TWMCBaseSolver.cpp:126-134)
-      double pr = sr * zr - si * zi, pi = sr * zi + si * zr;
-      beta[i] = mk(T(br + pr), T(bi + pi));
-    } else if (a.mode == 1) {
-      beta[i] = mk(T(a.base[3][2 * i]), T(a.base[3][2 * i + 1]));
-    } else if (a.mode == 2) {
-      const double* bp = a.beta_prev + 2 * ((size_t)b * a.n + i);
-      beta[i] = mk(T(bp[0]), T(bp[1]));
-    }  // mode 3: gauss_init_kernel writes the state
-    if (a.per_traj_params || b == 0) {
-      size_t off = (size_t)(a.per_traj_params ? b : 0) * a.n + i;
-      double orr, oi, ur, ui, fr, fi;
-      gen_param(a, 0, TAG_OMEGA, traj, i, orr, oi);
-      gen_param(a, 1, TAG_U, traj, i, ur, ui);
-      gen_param(a, 2, TAG_F, traj, i, fr, fi);
-      double rr, ri;
-      if (a.onsite == 0) {
-        // rsl = -i omega - gamma/2 (TWMCBaseSolver.cpp:74)
-        rr = oi - a.gamma / 2.0;
-        ri = -orr;
-      } else {
-        // delta = -E + detuning; rsl = -i delta - gamma/2 (TWMCLiebSolver.cpp:44-45)
-        double dr = -orr + a.detuning, di = -oi;
-        rr = di - a.gamma / 2.0;
-        ri = -dr;
+  const int np = (a.n + 1) / 2;
+  const uint64_t total = (uint64_t)a.n_traj * np;
+  for (uint64_t idx = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; idx < total;
+       idx += (uint64_t)gridDim.x * blockDim.x) {
+    const int b = total >> 32 ? (int)(idx / (uint32_t)np) : (int)((uint32_t)idx / (uint32_t)np);
+    const int p = (int)(idx - (uint64_t)b * (uint32_t)np);
+    const uint64_t traj = a.traj_ids[b];
+    u32x4 xp{};
+    if (a.mode == 0) xp = philox4x32_10(make_counter(traj, TAG_INIT, 0u, (uint32_t)p), a.key0, a.key1);
+    for (int i = 2 * p; i < min(2 * p + 2, a.n); ++i) {
+      cpx<T>* beta = reinterpret_cast<cpx<T>*>(a.beta) + (size_t)b * a.n;
+      if (a.mode == 0) {
+        double br, bi, sr, si;
+        gen_param(a, 3, TAG_BINIT, traj, i, br, bi);
+        gen_param(a, 4, TAG_BSIGMA, traj, i, sr, si);
+        double zr, zi;
+        box_muller_f64(i & 1 ? xp.z : xp.x, i & 1 ? xp.w : xp.y, zr, zi);
+        // beta_init + sigma (.) xi, complex product (TWMCBaseSolver.cpp:126-134)
+        double pr = sr * zr - si * zi, pi = sr * zi + si * zr;
+        beta[i] = mk(T(br + pr), T(bi + pi));
+      } else if (a.mode == 1) {
+        beta[i] = mk(T(a.base[3][2 * i]), T(a.base[3][2 * i + 1]));
+      } else if (a.mode == 2) {
+        const double* bp = a.beta_prev + 2 * ((size_t)b * a.n + i);
+        beta[i] = mk(T(bp[0]), T(bp[1]));
+      }  // mode 3: gauss_init_kernel writes the state
+      if (a.per_traj_params || b == 0) {
+        size_t off = (size_t)(a.per_traj_params ? b : 0) * a.n + i;
+        double orr, oi, ur, ui, fr, fi;
+        gen_param(a, 0, TAG_OMEGA, traj, i, orr, oi);
+        gen_param(a, 1, TAG_U, traj, i, ur, ui);
+        gen_param(a, 2, TAG_F, traj, i, fr, fi);
+        double rr, ri;
+        if (a.onsite == 0) {
+          // rsl = -i omega - gamma/2 (TWMCBaseSolver.cpp:74)
+          rr = oi - a.gamma / 2.0;
+          ri = -orr;
+        } else {
+          // delta = -E + detuning; rsl = -i delta - gamma/2 (TWMCLiebSolver.cpp:44-45)
+          double dr = -orr + a.detuning, di = -oi;
+          rr = di - a.gamma / 2.0;
+          ri = -dr;
+        }
+        reinterpret_cast<cpx<T>*>(a.rsl)[off] = mk(T(rr), T(ri));
+        reinterpret_cast<cpx<T>*>(a.U)[off] = mk(T(ur), T(ui));
+        reinterpret_cast<cpx<T>*>(a.F)[off] = mk(T(fr), T(fi));
       }
-      reinterpret_cast<cpx<T>*>(a.rsl)[off] = mk(T(rr), T(ri));
-      reinterpret_cast<cpx<T>*>(a.U)[off] = mk(T(ur), T(ui));
-      reinterpret_cast<cpx<T>*>(a.F)[off] = mk(T(fr), T(fi));
     }
   }
 }

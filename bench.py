@@ -178,7 +178,7 @@ def bench_sweep(args):
                    "autotuned": not args.no_autotune,
                    "kernel_ms": out["kernel_ms"]},
         "roofline": {"bound": "valu", "achieved": achieved / 1e12, "peak": PEAK_FP32 / 1e12, "unit": "TFLOP/s",
-                     "frac": achieved / PEAK_FP32, "traffic": sweep_traffic(), "kernel": "sweep_step_kernel<false>",
+                     "frac": achieved / PEAK_FP32, "traffic": sweep_traffic(), "kernel": "sweep_step_kernel<true>",
                      "avg_launch_ms": out["kernel_ms"] / args.steps,
                      "flops_basis": "algorithmic: 10 log2 N + 30 flops per site-step of each point's lattice "
                                     "(the reference's FFT hopping), over the graph's kernel time per frame "
@@ -302,7 +302,7 @@ def secondary_lines():
     a = float(N_TRAJ) * 4096 * FRAME_STEPS * FLOPS_PER_SITE_STEP / (ms * 1e-3)
     log(f"bench: FP64 64x64: {v:.4e} site-steps/s, step kernel avg {ms:.2f} ms")
     out["fp64"] = {
-        "value": v, "unit": "trajectory·site-steps/s", "dtype": "f64", "kernel": info["kernel"] + "_step_kernel",
+        "value": v, "unit": "trajectory·site-steps/s", "dtype": "f64", "kernel": "nn_step_kernel",
         "workload": "the 64x64 workload above (16384 trajectories, 500-step frames, 2 timed) with an FP64 state "
                     "and FP64 Box-Muller; the steps apply the exact nearest-neighbour form of the reference's "
                     "FFT hopping, the frame captures the FFT",
@@ -318,7 +318,7 @@ def secondary_lines():
     log(f"bench: lieb384: MFMA {v:.4e} site-steps/s ({ms:.3f} ms per launch), band {vb:.4e} ({msb:.3f} ms)")
     out["lieb384"] = {
         "workload": WORKLOAD_TEXT["lieb384"] + "; 10 timed frames",
-        "mfma": {"value": v, "unit": "trajectory·site-steps/s", "kernel": "mfma16_step_kernel", "avg_launch_ms": ms,
+        "mfma": {"value": v, "unit": "trajectory·site-steps/s", "kernel": "mfma_step_kernel", "avg_launch_ms": ms,
                  "roofline": {"bound": "mfma", "achieved": a / 1e12, "peak": PEAK_BF16 / 1e12, "unit": "TFLOP/s",
                               "frac": a / PEAK_BF16,
                               "flops_basis": "executed BF16 MFMA flops: 3 products x 4 N per site-step",
@@ -418,7 +418,7 @@ def main():
     if args.workload == "lieb384" and info["kernel"] == "mfma":
         # executed MFMA work: 3 BF16 products of the real N x N hopping on Re and Im
         flops_site = 3 * 4.0 * n_sites
-        peak, bound, kname = PEAK_BF16, "mfma", "mfma16_step_kernel"
+        peak, bound, kname = PEAK_BF16, "mfma", "mfma_step_kernel"
         basis = "executed BF16 MFMA flops: 3 products (hi.hi, hi.lo, lo.hi) x 4 N per site-step"
     elif args.workload == "lieb384":
         # the banded kernel: executed FP32 arithmetic per site-step, the

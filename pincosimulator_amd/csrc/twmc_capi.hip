@@ -178,12 +178,12 @@ int hip_fail(Ctx* c, hipError_t e, const char* what) {
 // grid-stride loop and is bound by instruction issue.  With w waves per SIMD
 // (up to what fits) the batch runs in rounds; a round with a waves active on
 // a SIMD costs about a issue periods, but no less than a latency floor of
-// 2.4 (measured: two register-resident 64x64 waves keep the main VALU 84.5%
+// 2.4 (two waves of a 64x64 lattice held in registers kept the main VALU 84.5%
 // busy), so a partly filled last round costs the floor, not nothing.  Take
-// the w with the smallest total, the larger w on ties.  16384 trajectories on
-// 1024 SIMDs: three waves per SIMD (5 full rounds and a one-wave tail, 17.4)
-// rather than two (8 rounds at the floor, 19.2) -- 2% faster measured;
-// 8192 trajectories with up to four waves: four (2 rounds, 8).
+// the w with the smallest total, the larger w on ties: 8192 trajectories on
+// 1024 SIMDs with up to eight waves, eight (one round); with up to four, four.
+// (The register kernel of that lattice, 16384 trajectories: three waves per SIMD,
+// 5 full rounds and a one-wave tail, 2% faster than two, 8 rounds at the floor.)
 int balanced_wave_grid(size_t B, int per_cu, int cus) {
   const size_t simds = 4 * (size_t)cus;
   const int wmax = std::max(1, per_cu / 4);
@@ -316,7 +316,7 @@ bool all_but_energy_uniform(const Ctx* c) {
 
 int choose_kernel(Ctx* c) {
   const twmc_params& p = c->p;
-  // the register-resident kernel takes site-uniform, trajectory-shared parameters
+  // the 64x64 kernels take site-uniform, trajectory-shared parameters
   bool uniform = true;
   for (int k = 0; k < 3; ++k)
     for (int i = 1; i < c->n && uniform; ++i)
@@ -337,10 +337,11 @@ int choose_kernel(Ctx* c) {
     return fail(c, TWMC_ERR_UNSUPPORTED,
                 "stencil 64x64 kernel needs nx = ny = 64, FFT hopping, FP32 and site-uniform, disorder-free parameters");
   // AUTO: the 64x64 nearest-neighbour form first (the same linear map as the
-  // reference's FFT hopping, about twice as fast as the register FFT), then
+  // reference's FFT hopping, four times as fast as the register FFT), then
   // the register FFT; other uniform FP32 lattices of more than 64 sites on the
   // stacked LDS stencil (up to 64 sites the LDS kernel, which packs 2 or 4
-  // trajectories per wave, is faster); for matrix hopping the banded stencil
+  // trajectories per wave or, in small batches, forms the noise ahead of the
+  // steps, is faster); for matrix hopping the banded stencil
   // when the coupling is banded (a dense product would mostly move zeros),
   // else the MFMA matrix product; the LDS kernel for everything else
   if (k == TWMC_KERNEL_AUTO)

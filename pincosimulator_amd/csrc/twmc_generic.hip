@@ -2,8 +2,8 @@
 // size (mixed-radix FFT: radices 2, 3, 4, 5, 8 and a direct-sum pass for each
 // larger prime factor) and for matrix hopping, FP32 or FP64.  One workgroup
 // advances one trajectory at a time (up to four, for lattices of up to 64
-// sites); a persistent grid walks the batch.  This kernel is the FP64 path
-// and the fallback for shapes the register-resident kernels do not cover.
+// sites); a persistent grid walks the batch.  The fallback for what the other
+// kernels do not cover; its captures serve the nn, ahead, sparse and stacked steps.
 //
 // Per step (src/TWMC/Solvers/TWMCBaseSolver.cpp:232-256):
 //   beta -> LDS, forward DFT (rows, then columns; Stockham, ping-pong),

@@ -295,16 +295,25 @@ bool nn_supported(int nx, int ny, int precision, int vary) {
          n > (precision == 64 && ny % 2 == 0 ? 128 : 64) && (precision == 64 || vary != kVaryNone || ny % 2);
 }
 
-// Two pairs per thread (above 2048 sites) and at most two trajectories per CU: the LDS
-// kernel's own launch there (1024 threads too, 128 registers, one barrier per step)
-// gives each wave more to overlap, and the eight waves per SIMD have no third
-// trajectory to take up: 64x64, us per step there against here, 32 trajectories 2.97
-// to 3.29, 512 6.38 to 6.62 (48x48: 1.96 to 2.10, 4.21 to 4.08).  From the third on
-// this kernel wins (64x64: 513 trajectories 9.28 to 8.92, 768 10.24 to 9.52); up to
-// 2048 sites it wins at every batch (32 trajectories of 32x32 1.19 to 1.03).
+// FP64 with even rows: where the LDS kernel's own launch is as fast or faster it stays.
+// Its 128 registers give each wave more to overlap, which tells until the CUs hold more
+// than four waves per SIMD.  us per step there against here:
+//   up to 256 sites, uniform: the same at every batch (16x16, 8192: 7.7, 7.4);
+//     one parameter varying (held in registers there): 16x16, 1500 trajectories
+//     1.59 / 1.81, 3000 3.14 / 3.29, 6000 6.08 / 5.65, 20000 20.1 / 16.7;
+//   257 to 512, uniform: 1x512, 130 trajectories 0.64 / 0.72, 700 1.36 / 1.42, 3000
+//     5.11 / 4.67;
+//   2049 to 4096, uniform: 64x64, 32 trajectories 2.97 / 3.29, 512 6.38 / 6.62, 768
+//     10.24 / 9.52.
+// Between, and with odd rows, this kernel wins at every batch (32x32, 32 trajectories,
+// 1.19 / 1.03).
 bool nn_pays(int nx, int ny, int precision, int vary, size_t n_traj, int cus) {
-  if (precision != 64 || vary != kVaryNone || ny % 2) return true;
-  return nx * ny > 256 && (nx * ny <= 2048 || n_traj > 2 * (size_t)cus);
+  const int n = nx * ny;
+  const size_t per_cu = n_traj / (size_t)cus;
+  if (precision != 64 || ny % 2) return true;
+  if (n <= 256) return vary != kVaryNone && per_cu >= 12;
+  if (vary != kVaryNone) return true;
+  return n <= 512 ? per_cu >= 4 : n <= 2048 || n_traj > 2 * (size_t)cus;
 }
 
 hipError_t nn_occupancy(int nx, int ny, int precision, int vary, bool u_real, int* blocks_per_cu) {

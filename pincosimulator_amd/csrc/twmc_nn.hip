@@ -235,22 +235,26 @@ struct Launch {
   size_t lds;
 };
 
+// FP32, 513 to 1024 pairs: only the waves that have pairs, so that three workgroups of 9
+// or 10 waves share a CU (27x41, us per step: 1500 trajectories 2.96 -> 2.62, 8192 15.8 ->
+// 13.7; 30x36 with a drawn F, 1500: 3.44 -> 2.60).  Fewer pairs and FP64 gain and lose
+// by batch, -10 to +8%: full workgroups.
 template <typename T, int BLOCK, int PPT, int V, bool ODD, bool UI0>
-Launch launch_x(bool xn) {
+Launch launch_x(int np, bool xn) {
   return {xn ? (const void*)nn_step_kernel<T, BLOCK, PPT, V, ODD, true, UI0>
              : (const void*)nn_step_kernel<T, BLOCK, PPT, V, ODD, false, UI0>,
-          BLOCK, kTabBytes<T> + 16 + (size_t)BLOCK * PPT * 2 * sizeof(cpx<T>) * (V == kVaryNone ? 1 : 2)};
+          sizeof(T) == 4 && BLOCK == 1024 && PPT == 1 ? (np + 63) / 64 * 64 : BLOCK, kTabBytes<T> + 16 + (size_t)BLOCK * PPT * 2 * sizeof(cpx<T>) * (V == kVaryNone ? 1 : 2)};
 }
 
 template <typename T, int V, bool ODD, bool UI0>
 Launch launch_s(int n, bool xn) {
   const int np = (n + 1) / 2;
-  return np <= 64     ? launch_x<T, 64, 1, V, ODD, UI0>(xn)
-         : np <= 128  ? launch_x<T, 128, 1, V, ODD, UI0>(xn)
-         : np <= 256  ? launch_x<T, 256, 1, V, ODD, UI0>(xn)
-         : np <= 512  ? launch_x<T, 512, 1, V, ODD, UI0>(xn)
-         : np <= 1024 ? launch_x<T, 1024, 1, V, ODD, UI0>(xn)
-                      : launch_x<T, 1024, 2, V, ODD, UI0>(xn);
+  return np <= 64     ? launch_x<T, 64, 1, V, ODD, UI0>(np, xn)
+         : np <= 128  ? launch_x<T, 128, 1, V, ODD, UI0>(np, xn)
+         : np <= 256  ? launch_x<T, 256, 1, V, ODD, UI0>(np, xn)
+         : np <= 512  ? launch_x<T, 512, 1, V, ODD, UI0>(np, xn)
+         : np <= 1024 ? launch_x<T, 1024, 1, V, ODD, UI0>(np, xn)
+                      : launch_x<T, 1024, 2, V, ODD, UI0>(np, xn);
 }
 
 template <typename T, int V>

@@ -7,7 +7,7 @@
 // stencil along the site index, and a dense or LDS-staged product only moves
 // zeros.  One wavefront owns one trajectory: lane l holds sites l S .. l S + S - 1
 // in registers (S even; N padded to 64 S, the padding sites have zero
-// coefficients and are never stored), together with the coefficients
+// coefficients, stay finite and are never stored), together with the coefficients
 // dt C_(j+d) j of its sites and its dt-scaled site parameters.  The W sites on
 // either side of a lane's block come from lanes l - 1 and l + 1 by whole-wave
 // DPP rotations.  Per step: the hopping sums of all owned sites from the old
@@ -55,6 +55,12 @@ __host__ __device__ constexpr bool lieb_bond(int r, int d) {
 // UNI: Re rsl, F and a real U are the same at every site, so of the site tables
 // only Im rsl (the on-site energies) takes registers, and 64 of them hold the
 // kernel at eight waves per SIMD.
+// PAD (UNI and DENSE): n < 64 S.  Tables per site are zero on the padding, but a uniform
+// one drives it, without the energies that may keep the real sites off resonance: it can
+// overflow, and 0 times infinity reach the first and last sites.  Each step sets it back
+// to zero (8192 trajectories, us per step, not reset / reset / parameters per site in the
+// form before: 72 sites 1.38 / 1.42 / 1.53, 210 2.36 / 2.45 / 3.18, 330 3.12 / 3.30 / 3.74,
+// 495 4.86 / 5.05 / 5.54).
 // DENSE: more than two waves per SIMD.  Bound by VALU issue: 41 instructions per
 // site-step of the 384-site Lieb chain, 37 beside the transcendental ones, which
 // have a unit of their own.  Free-running waves bunch up before that unit and
@@ -71,11 +77,12 @@ __host__ __device__ constexpr bool lieb_bond(int r, int d) {
 constexpr int uni_waves(int s, int w, bool lieb) {
   return s == 2 || lieb ? 8 : s == 4 ? (w <= 2 ? 7 : 6) : s == 6 ? (w == 1 ? 7 : 5) : w == 1 ? 5 : 4;
 }
-template <int S, int W, bool FT, bool LIEB, bool UNI, bool DENSE>
+template <int S, int W, bool FT, bool LIEB, bool UNI, bool DENSE, bool PAD>
 __global__ void __launch_bounds__(64, UNI ? uni_waves(S, W, LIEB) : 1) band_step_kernel(StepArgs g) {
   static_assert(!LIEB || (S == 6 && W == 2), "the Lieb pattern needs two cells per lane");
   static_assert(!UNI || !FT, "F(t) is per site");
   static_assert(!DENSE || !FT, "F(t) runs the latency form");
+  static_assert(!PAD || (UNI && DENSE), "parameters per site are zero on the padding");
   constexpr bool LDSX = DENSE, PRIO = DENSE && S >= 4;
   constexpr int D = 2 * W + 1;
   constexpr int SP = UNI ? 1 : S;  // entries of a uniform table
@@ -220,7 +227,8 @@ __global__ void __launch_bounds__(64, UNI ? uni_waves(S, W, LIEB) : 1) band_step
       // noise and update
 #pragma unroll
       for (int p = 0; p < S / 2; ++p) {
-        const u32x4 w = philox4x32_10_wave(make_counter(traj, TAG_WIENER, step, pbase + (uint32_t)p), g.key0, g.key1);
+        const u32x4 ctr = make_counter(traj, TAG_WIENER, step, pbase + (uint32_t)p);
+        const u32x4 w = LIEB && !DENSE ? philox4x32_10(ctr, g.key0, g.key1) : philox4x32_10_wave(ctr, g.key0, g.key1);
         float rn[2], cs[2], sn[2];
         if constexpr (PRIO) __builtin_amdgcn_s_setprio(2);
         box_muller_f32_scaled(w.x, w.y, nl, rn[0], cs[0], sn[0]);
@@ -240,8 +248,9 @@ __global__ void __launch_bounds__(64, UNI ? uni_waves(S, W, LIEB) : 1) band_step
           float ui = fmaf(rn[h], sn[h], di[s]);
           ui = fmaf(cr, y, ui);
           ui = fmaf(ci, x, ui);
-          br[s] = x + ur;
-          bi[s] = y + ui;
+          const bool live = !PAD || base + s < n;
+          br[s] = live ? x + ur : 0.f;
+          bi[s] = live ? y + ui : 0.f;
         }
       }
     }
@@ -254,33 +263,40 @@ __global__ void __launch_bounds__(64, UNI ? uni_waves(S, W, LIEB) : 1) band_step
   }
 }
 
+// Bound by latency the uniform form gains where it saves most registers, four and more
+// sites per lane without padding (512 sites, W = 2, x 1000: 0.91 -> 0.88 us per step); for
+// the Lieb chain and with padding to reset it loses (384 x 1500 0.98 / 1.05, 210 x 64
+// 0.42 / 0.45, 495 x 1000 0.90 / 0.94): those take the parameters per site.
 template <int S, int W, bool LIEB>
-const void* kernel_swl(bool ft, bool uni, bool dense) {
-  if (ft) return (const void*)band_step_kernel<S, W, true, LIEB, false, false>;
-  if (uni)
-    return dense ? (const void*)band_step_kernel<S, W, false, LIEB, true, true>
-                 : (const void*)band_step_kernel<S, W, false, LIEB, true, false>;
-  return dense ? (const void*)band_step_kernel<S, W, false, LIEB, false, true>
-               : (const void*)band_step_kernel<S, W, false, LIEB, false, false>;
+const void* kernel_swl(bool ft, bool uni, bool dense, bool pad) {
+  if (ft) return (const void*)band_step_kernel<S, W, true, LIEB, false, false, false>;
+  if (uni && dense)
+    return pad ? (const void*)band_step_kernel<S, W, false, LIEB, true, true, true>
+               : (const void*)band_step_kernel<S, W, false, LIEB, true, true, false>;
+  if constexpr (S >= 4 && !LIEB)
+    if (uni && !pad) return (const void*)band_step_kernel<S, W, false, LIEB, true, false, false>;
+  return dense ? (const void*)band_step_kernel<S, W, false, LIEB, false, true, false>
+               : (const void*)band_step_kernel<S, W, false, LIEB, false, false, false>;
 }
 
 template <int S>
-const void* kernel_s(int w, bool lieb, bool ft, bool uni, bool dense) {
+const void* kernel_s(int w, bool lieb, bool ft, bool uni, bool dense, bool pad) {
   if constexpr (S == 6)
-    if (lieb && w == 2) return kernel_swl<6, 2, true>(ft, uni, dense);
+    if (lieb && w == 2) return kernel_swl<6, 2, true>(ft, uni, dense, pad);
   switch (w) {
-    case 1: return kernel_swl<S, 1, false>(ft, uni, dense);
-    case 2: return kernel_swl<S, 2, false>(ft, uni, dense);
-    default: return kernel_swl<S, 3, false>(ft, uni, dense);
+    case 1: return kernel_swl<S, 1, false>(ft, uni, dense, pad);
+    case 2: return kernel_swl<S, 2, false>(ft, uni, dense, pad);
+    default: return kernel_swl<S, 3, false>(ft, uni, dense, pad);
   }
 }
 
 const void* kernel_for(int n, int w, bool lieb, bool ft, bool uni, bool dense) {
+  const bool pad = 64 * band_sites_per_lane(n) != n;
   switch (band_sites_per_lane(n)) {
-    case 2: return kernel_s<2>(w, lieb, ft, uni, dense);
-    case 4: return kernel_s<4>(w, lieb, ft, uni, dense);
-    case 6: return kernel_s<6>(w, lieb, ft, uni, dense);
-    default: return kernel_s<8>(w, lieb, ft, uni, dense);
+    case 2: return kernel_s<2>(w, lieb, ft, uni, dense, pad);
+    case 4: return kernel_s<4>(w, lieb, ft, uni, dense, pad);
+    case 6: return kernel_s<6>(w, lieb, ft, uni, dense, pad);
+    default: return kernel_s<8>(w, lieb, ft, uni, dense, pad);
   }
 }
 

@@ -10,7 +10,7 @@
 // vector, so Z_l = A_{l-1} W_l + b_l is a plain NN product.
 //
 // Networks of widths up to 256 (the warm start's has 256) take two launches per
-// minibatch, or one for inference:
+// minibatch, or one for inference on few rows:
 //   mlp_rows_kernel        four samples per workgroup through the whole network:
 //                          forward, loss, and back to every layer's dZ
 //   mlp_wgrad_kernel       weight and bias gradients as one product per layer,
@@ -18,7 +18,7 @@
 //   mlp_pack_kernel        their copies of the weights, W and W^T of every layer
 //                          with rows padded to 16 bytes, whenever parameters
 //                          are set (the Adam update keeps both from then on)
-// Kernels of wider networks, layer by layer:
+// Kernels of wider networks and of inference on many rows (fused_forward), layer by layer:
 //   mlp_gemm_kernel<MODE>  C[M x N] = op(A)[M x K] op(B)[K x N] with strided
 //                          operands (covers NN forward, NT for dA = dZ W^T, TN
 //                          for dW = A^T dZ), 64x64 tile per 256-thread
@@ -663,6 +663,17 @@ bool is_narrow(const MlpCtx* c) {
   return rows_lds_bytes(c->n_layers - 1, true) + 1024 <= 160 * 1024;
 }
 
+// Inference on the fused kernel: every four samples read all weights, so from some
+// number of rows on the products of 64 samples at a time take less.  The whole call,
+// fused / layer by layer, ms: 5-3x256-34 4096 rows 0.11 / 0.22, 8192 0.22 / 0.28, 16384
+// 0.39 / 0.39, 65536 1.47 / 1.12; 64-4x128-64 8192 0.35 / 0.36, 16384 0.66 / 0.56; 3-8x32-2
+// 8192 0.15 / 0.26, 16384 0.28 / 0.26; a few narrow layers: 5-2x64-8 4096 0.061 / 0.074,
+// 8192 0.091 / 0.083, 5-1x16-4 4096 0.051 / 0.049, 8192 0.075 / 0.056.  (Training gains at
+// any batch: the gradients of 65536 samples of 5-3x256-34 114 -> 3.4 ms.)
+bool fused_forward(const MlpCtx* c, uint64_t rows) {
+  return c->narrow && rows <= (max_width(c) <= 64 && c->n_layers <= 3 ? 4096u : 8192u);
+}
+
 // forward over act[0] (rows x inputs); outputs in act[n_layers]
 int forward(MlpCtx* c, int rows) {
   for (int l = 1; l <= c->n_layers; ++l) {
@@ -912,9 +923,10 @@ int twmc_mlp_forward(twmc_mlp_ctx* ctx, const float* x, uint64_t rows, float* y)
   MlpCtx* c = reinterpret_cast<MlpCtx*>(ctx);
   if (rows == 0 || rows > (1u << 24)) return mlp_fail(c, TWMC_ERR_INVALID, "rows out of range");
   MLPCHK(c, hipSetDevice(c->device));
-  int rc = c->narrow ? ensure_narrow(c, (int)rows, false) : ensure_rows(c, (int)rows);
+  const bool fused = fused_forward(c, rows);
+  int rc = fused ? ensure_narrow(c, (int)rows, false) : ensure_rows(c, (int)rows);
   if (rc != TWMC_OK) return rc;
-  if (c->narrow) {
+  if (fused) {
     MLPCHK(c, c->data_x.ensure(rows * c->width[0] * 4));
     MLPCHK(c, hipMemcpyAsync(c->data_x.p, x, rows * c->width[0] * 4, hipMemcpyHostToDevice, c->stream));
     MLPCHK(c, launch_rows(c, net_args(c, (int)rows, c->data_x.f(), nullptr, nullptr, nullptr), false));

@@ -67,7 +67,7 @@ struct DevBuf {
 // Pinned staging of large read-backs (read_states): two chunks per reader
 constexpr int kReaders = 4;
 constexpr size_t kStageBytes = 512 * 1024;
-constexpr size_t kStagedRead = 1024 * 1024;  // smaller ones are read in one piece
+constexpr size_t kStagedRead = 1024 * 1024;  // smaller ones are read in one piece, as any without pinned memory
 struct Stage {
   unsigned char* p = nullptr;
   hipEvent_t done[2 * kReaders] = {};
@@ -721,13 +721,17 @@ int read_states(Ctx* c, const void* src, size_t count, double* dst) {
     return TWMC_OK;
   }
   const size_t bytes = count * 8;
-  if (bytes < kStagedRead) {
+  bool staged = bytes >= kStagedRead;
+  if (staged && c->stage.ensure() != hipSuccess) {  // no pinned memory to be had
+    (void)hipGetLastError();
+    staged = false;
+  }
+  if (!staged) {
     std::vector<float> tmp(count * 2);
     HIPCHK(c, hipMemcpy(tmp.data(), src, bytes, hipMemcpyDeviceToHost));
     for (size_t i = 0; i < count * 2; ++i) dst[i] = tmp[i];
     return TWMC_OK;
   }
-  HIPCHK(c, c->stage.ensure());
   const size_t chunks = (bytes + kStageBytes - 1) / kStageBytes;
   auto reader = [&](int w) -> hipError_t {  // chunks w, w + kReaders, ...
     hipError_t e = hipSetDevice(c->device);

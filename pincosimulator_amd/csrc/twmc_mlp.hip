@@ -36,6 +36,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <cstdlib>
 #include <cstring>
 #include <string>
 #include <utility>
@@ -533,7 +534,8 @@ struct MlpCtx {
   Buf packed, dz[kMaxLayers + 1], loss_part;
   size_t f_off[kMaxLayers], t_off[kMaxLayers], n_packed = 0;
   int cap_narrow = 0;
-  int* perm[2] = {nullptr, nullptr};  // pinned epoch orders, one computed while the other is used
+  int* perm[2] = {nullptr, nullptr};  // epoch orders, one computed while the other is used
+  bool perm_pinned = false;
   hipEvent_t perm_ev[2] = {nullptr, nullptr};
   size_t perm_cap = 0;
   std::string err;
@@ -767,17 +769,35 @@ int upload_data(MlpCtx* c, const float* x, const float* t, const float* w, uint6
   return TWMC_OK;
 }
 
-// two pinned buffers for epoch orders of `rows` samples
+void release_perm(MlpCtx* c) {
+  for (int*& p : c->perm) {
+    if (c->perm_pinned) (void)hipHostFree(p);
+    else std::free(p);
+    p = nullptr;
+  }
+  c->perm_cap = 0;
+}
+
+// two buffers for epoch orders of `rows` samples: pinned, or if there is no pinned
+// memory to be had, pageable
 int ensure_perm(MlpCtx* c, size_t rows) {
   for (int k = 0; k < 2; ++k)
     if (!c->perm_ev[k]) MLPCHK(c, hipEventCreateWithFlags(&c->perm_ev[k], hipEventDisableTiming));
   if (rows <= c->perm_cap) return TWMC_OK;
-  c->perm_cap = 0;
-  for (int k = 0; k < 2; ++k) {
-    if (c->perm[k]) (void)hipHostFree(c->perm[k]);
-    c->perm[k] = nullptr;
-    MLPCHK(c, hipHostMalloc(reinterpret_cast<void**>(&c->perm[k]), rows * sizeof(int), hipHostMallocDefault));
-  }
+  release_perm(c);
+  c->perm_pinned = true;
+  for (int*& p : c->perm)
+    if (hipHostMalloc(reinterpret_cast<void**>(&p), rows * sizeof(int), hipHostMallocDefault) != hipSuccess) {
+      (void)hipGetLastError();
+      p = nullptr;
+      release_perm(c);
+      c->perm_pinned = false;
+      break;
+    }
+  if (!c->perm_pinned)
+    for (int*& p : c->perm)
+      if (!(p = static_cast<int*>(std::malloc(rows * sizeof(int)))))
+        return mlp_fail(c, TWMC_ERR_NOMEM, "no memory for the epochs' orders");
   c->perm_cap = rows;
   return TWMC_OK;
 }
@@ -880,10 +900,9 @@ void twmc_mlp_destroy(twmc_mlp_ctx* ctx) {
     c->act[l].release();
     c->dz[l].release();
   }
-  for (int k = 0; k < 2; ++k) {
-    if (c->perm[k]) (void)hipHostFree(c->perm[k]);
-    if (c->perm_ev[k]) (void)hipEventDestroy(c->perm_ev[k]);
-  }
+  release_perm(c);
+  for (hipEvent_t e : c->perm_ev)
+    if (e) (void)hipEventDestroy(e);
   for (int l = 0; l < kMaxLayers; ++l) c->pre[l].release();
   if (c->stream) (void)hipStreamDestroy(c->stream);
   delete c;

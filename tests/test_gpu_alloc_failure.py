@@ -56,3 +56,22 @@ def test_read_back_without_pinned_memory(run):
     assert np.all(np.any(out[0].traj != 0, axis=2))
     print("done")
     """)
+
+
+def test_training_without_pinned_memory(run):
+    run("""
+    rng = np.random.default_rng(2)
+    x, t = (rng.normal(size=(300, k)).astype(np.float32) for k in (5, 7))
+    out = []
+    for on in (1, 0):
+        fail.fail_pinned(on)
+        m = MLP(5, 7, n_hidden=20, n_hidden_layers=2, seed=4)
+        m.train(x[:50], t[:50], epochs=3, batch=16)
+        m.train(x, t, epochs=3, batch=16)  # longer orders
+        out.append(m.params)
+        fail.fail_pinned(0)
+        m.close()
+        assert fail.failures() > 0
+    np.testing.assert_array_equal(*out)
+    print("done")
+    """)

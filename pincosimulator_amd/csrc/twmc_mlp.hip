@@ -1002,7 +1002,8 @@ int twmc_mlp_train(twmc_mlp_ctx* ctx, const float* x, const float* t, const floa
       !(o->beta2 >= 0.0f && o->beta2 < 1.0f) || !(o->eps > 0.0f))
     return mlp_fail(c, TWMC_ERR_INVALID, "bad training options");
   MLPCHK(c, hipSetDevice(c->device));
-  // after an error return, nothing of the call may still read its buffers
+  // after an error return, nothing of the call may still use its buffers
+  std::vector<double> bl;
   struct Drain {
     hipStream_t s;
     ~Drain() { (void)hipStreamSynchronize(s); }
@@ -1020,7 +1021,7 @@ int twmc_mlp_train(twmc_mlp_ctx* ctx, const float* x, const float* t, const floa
   rc = upload_data(c, x, t, w, rows);
   if (rc != TWMC_OK) return rc;
   const float* wd = w ? c->data_w.f() : nullptr;
-  std::vector<double> bl((size_t)keep * n_batches);
+  bl.resize((size_t)keep * n_batches);
   uint64_t s = o->shuffle_seed;
   if (o->epochs > 0) shuffle_epoch(c->perm[0], rows, s);
   for (int ep = 0; ep < o->epochs; ++ep) {

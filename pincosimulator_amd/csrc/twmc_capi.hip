@@ -157,7 +157,9 @@ struct Ctx {
   twmc_stats stats{};
 };
 
+// (a HIP error is cleared: the next call's hipGetLastError would report it again)
 int fail(Ctx* c, int code, const std::string& msg) {
+  if (code == TWMC_ERR_HIP) (void)hipGetLastError();
   if (c) c->err = msg;
   g_last_error = msg;
   return code;

@@ -543,7 +543,9 @@ struct MlpCtx {
 
 thread_local std::string g_mlp_err;
 
+// (a HIP error is cleared: the next call's hipGetLastError would report it again)
 int mlp_fail(MlpCtx* c, int code, const std::string& m) {
+  if (code == TWMC_ERR_HIP) (void)hipGetLastError();
   if (c) c->err = m;
   g_mlp_err = m;
   return code;

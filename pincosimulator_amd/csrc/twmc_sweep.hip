@@ -508,7 +508,9 @@ struct SweepCtx {
   twmc_stats stats{};
 };
 
+// (a HIP error is cleared: the next call's hipGetLastError would report it again)
 int sfail(SweepCtx* c, int code, const std::string& m) {
+  if (code == TWMC_ERR_HIP) (void)hipGetLastError();
   if (c) c->err = m;
   g_sweep_error = m;
   return code;

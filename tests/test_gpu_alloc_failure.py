@@ -1,5 +1,5 @@
-"""Allocations that fail (tests/native/alloc_fail.c returns the error in the library's
-process; the GPU does not see them): calls that have another way take it with the same
+"""Allocations that fail (tests/native/alloc_fail.c asks the runtime for too much in the library's
+process, which the host refuses): calls that have another way take it with the same
 results, the others return an error and leave a context that later calls can use."""
 import os
 import subprocess
@@ -18,7 +18,7 @@ sys.path[:0] = [{root!r}, {tests!r}]
 fail = ctypes.CDLL({so!r}, mode=ctypes.RTLD_GLOBAL)
 fail.fail_device_above.argtypes = [ctypes.c_size_t]
 import numpy as np
-from pincosimulator_amd import Engine, System
+from pincosimulator_amd import Engine, Sweep
 from pincosimulator_amd._lib import TWMCError
 from pincosimulator_amd.mlp import MLP
 from helpers import c2_spec, system
@@ -73,5 +73,35 @@ def test_training_without_pinned_memory(run):
         m.close()
         assert fail.failures() > 0
     np.testing.assert_array_equal(*out)
+    print("done")
+    """)
+
+
+def test_error_is_reported_once(run):
+    run("""
+    def fails(call):
+        fail.fail_device_above(100000)
+        try:
+            call()
+            raise SystemExit("no error")
+        except TWMCError as e:
+            assert "memory" in str(e)
+        fail.fail_device_above(1 << 40)
+
+    m = MLP(5, 7, n_hidden=20, n_hidden_layers=2, seed=4)
+    x = np.ones((4000, 5), dtype=np.float32)
+    fails(lambda: m.forward(x))
+    assert np.all(np.isfinite(m.forward(x[:9])))
+    m.close()
+    spec = c2_spec(nx=4, ny=8, frame_steps=5, t_end=0.002 * 15.25)
+    eng = Engine(system(spec), precision=32)
+    fails(lambda: eng.begin(np.arange(5000)))
+    assert np.all(np.isfinite(eng.run(np.arange(3)).sum_n))
+    eng.close()
+    point = dict(nx=1, ny=64, gamma=1.0, J=1.0, U=0.1, F=1.0, traj_id0=0)
+    fails(lambda: Sweep([dict(point, n_traj=1000)], 0.005, 10, 3))
+    sw = Sweep([dict(point, n_traj=10)], 0.005, 10, 3)
+    assert np.all(np.isfinite(sw.run(0.2, graph=False)["m2"][0]))
+    sw.close()
     print("done")
     """)

@@ -528,12 +528,10 @@ struct MlpCtx {
   Buf pre[kMaxLayers];         // Z_l of hidden layers
   Buf dA, dB;                  // backward ping-pong, rows x max width
   Buf data_x, data_t, data_w, bt, bw, idx, loss;
-  int cap_rows = 0;
   // widths up to 256: the fused kernels' packed weights, dZ and partial losses
   bool narrow = false;
   Buf packed, dz[kMaxLayers + 1], loss_part;
   size_t f_off[kMaxLayers], t_off[kMaxLayers], n_packed = 0;
-  int cap_narrow = 0;
   int* perm[2] = {nullptr, nullptr};  // epoch orders, one computed while the other is used
   bool perm_pinned = false;
   hipEvent_t perm_ev[2] = {nullptr, nullptr};
@@ -574,8 +572,9 @@ int max_width(const MlpCtx* c) {
   return w;
 }
 
+// each buffer by its own size: after an allocation that failed, no other one's size says
+// that it is there
 int ensure_rows(MlpCtx* c, int rows) {
-  if (rows <= c->cap_rows) return TWMC_OK;
   for (int l = 0; l <= c->n_layers; ++l) MLPCHK(c, c->act[l].ensure((size_t)rows * c->width[l] * 4));
   for (int l = 1; l < c->n_layers; ++l) MLPCHK(c, c->pre[l].ensure((size_t)rows * c->width[l] * 4));
   const size_t mw = (size_t)max_width(c);
@@ -583,18 +582,16 @@ int ensure_rows(MlpCtx* c, int rows) {
   MLPCHK(c, c->dB.ensure((size_t)rows * mw * 4));
   MLPCHK(c, c->bt.ensure((size_t)rows * c->width[c->n_layers] * 4));
   MLPCHK(c, c->bw.ensure((size_t)rows * c->width[c->n_layers] * 4));
-  c->cap_rows = rows;
   return TWMC_OK;
 }
 
 // the fused kernels' buffers for `rows` rows (only act[n_layers] without training)
 int ensure_narrow(MlpCtx* c, int rows, bool train) {
   MLPCHK(c, c->act[c->n_layers].ensure((size_t)rows * c->width[c->n_layers] * 4));
-  if (!train || rows <= c->cap_narrow) return TWMC_OK;
+  if (!train) return TWMC_OK;
   for (int l = 0; l < c->n_layers; ++l) MLPCHK(c, c->act[l].ensure((size_t)rows * c->width[l] * 4));
   for (int l = 1; l <= c->n_layers; ++l) MLPCHK(c, c->dz[l].ensure((size_t)rows * c->width[l] * 4));
   MLPCHK(c, c->loss_part.ensure((size_t)(rows + kRowsBlock - 1) / kRowsBlock * 8));
-  c->cap_narrow = rows;
   return TWMC_OK;
 }
 

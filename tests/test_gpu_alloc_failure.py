@@ -105,3 +105,30 @@ def test_error_is_reported_once(run):
     sw.close()
     print("done")
     """)
+
+
+@pytest.mark.parametrize("hidden", [20, 300])
+def test_network_after_a_failed_call(run, hidden):
+    """A gradient over 20000 rows fails at its larger buffers; the smaller batches after it."""
+    run(f"""
+    rng = np.random.default_rng(2)
+    x, t = (rng.normal(size=(20000, k)).astype(np.float32) for k in (5, 7))
+    m = MLP(5, 7, n_hidden={hidden}, n_hidden_layers=2, seed=4)
+    first = m.loss_grad(x[:64], t[:64])
+    fail.fail_device_above(1000000)
+    for call in (lambda: m.loss_grad(x, t), lambda: m.forward(x), lambda: m.loss_grad(x, t)):
+        try:
+            call()
+            raise SystemExit("no error")
+        except TWMCError:
+            pass
+    assert fail.failures() == 3
+    again = m.loss_grad(x[:64], t[:64])
+    np.testing.assert_array_equal(first[1], again[1])
+    assert first[0] == again[0]
+    np.testing.assert_allclose(m.forward(x[:64]), m.forward(x[:70])[:64], rtol=0, atol=0)
+    fail.fail_device_above(1 << 40)
+    assert np.all(np.isfinite(m.loss_grad(x, t)[1]))
+    m.close()
+    print("done")
+    """)

@@ -553,17 +553,24 @@ int add_bins(SweepCtx* c, int nx, int ny) {
   return off;
 }
 
-// lays out points and the two work-item lists (largest first) for the
-// current tb: the step launch stacks tb trajectories of every point per item,
-// the capture launch takes 2D points one trajectory per item (chains as in the
-// step launch)
-int build_items(SweepCtx* c) {
+// lays out points and the two work-item lists (largest first) for tb: the step
+// launch stacks tb trajectories of every point per item, the capture launch takes
+// 2D points one trajectory per item (chains as in the step launch).  The lists in
+// use are replaced only when everything is there.
+int build_items(SweepCtx* c, const std::vector<int>& tb) {
+  struct List {
+    void* d = nullptr;
+    int n = 0;
+    ~List() {
+      if (d) (void)hipFree(d);
+    }
+  } list[2];
   for (int pass = 0; pass < 2; ++pass) {
     const bool cap = pass == 1;
     std::vector<std::pair<double, SweepItemDev>> items;
     for (size_t p = 0; p < c->pts.size(); ++p) {
       const SweepPointDev& P = c->dev_pts[p];
-      const int step = (cap && P.fft_x) ? 1 : c->tb[p];
+      const int step = (cap && P.fft_x) ? 1 : tb[p];
       for (int t0 = 0; t0 < P.n_traj; t0 += step) {
         const int rows = std::min(step, P.n_traj - t0);
         const double cost = double(rows) * P.nx * P.ny * std::log2(double(P.nx * P.ny) + 1.0);
@@ -573,16 +580,19 @@ int build_items(SweepCtx* c) {
     std::stable_sort(items.begin(), items.end(), [](auto& a, auto& b) { return a.first > b.first; });
     std::vector<SweepItemDev> flat;
     for (auto& it : items) flat.push_back(it.second);
-    void*& d = cap ? c->d_items_cap : c->d_items;
-    (cap ? c->n_items_cap : c->n_items) = (int)flat.size();
-    if (d) (void)hipFree(d);
-    d = nullptr;
-    SCHK(c, hipMalloc(&d, flat.size() * sizeof(SweepItemDev)));
-    SCHK(c, hipMemcpy(d, flat.data(), flat.size() * sizeof(SweepItemDev), hipMemcpyHostToDevice));
+    list[pass].n = (int)flat.size();
+    SCHK(c, hipMalloc(&list[pass].d, flat.size() * sizeof(SweepItemDev)));
+    SCHK(c, hipMemcpy(list[pass].d, flat.data(), flat.size() * sizeof(SweepItemDev), hipMemcpyHostToDevice));
   }
-  for (size_t p = 0; p < c->pts.size(); ++p) c->dev_pts[p].tb = c->tb[p];
-  SCHK(c, hipMemcpy(c->d_points, c->dev_pts.data(), c->dev_pts.size() * sizeof(SweepPointDev),
-                    hipMemcpyHostToDevice));
+  std::vector<SweepPointDev> pts = c->dev_pts;
+  for (size_t p = 0; p < pts.size(); ++p) pts[p].tb = tb[p];
+  SCHK(c, hipMemcpy(c->d_points, pts.data(), pts.size() * sizeof(SweepPointDev), hipMemcpyHostToDevice));
+  std::swap(c->d_items, list[0].d);
+  std::swap(c->d_items_cap, list[1].d);
+  c->n_items = list[0].n;
+  c->n_items_cap = list[1].n;
+  c->dev_pts = pts;
+  c->tb = tb;
   return TWMC_OK;
 }
 
@@ -835,7 +845,7 @@ int twmc_sweep_create(const twmc_sweep_point* pts, uint64_t n_points, double dt,
   }
   c->grid = std::max(1, per_cu) * cus;
   c->grid_cap = std::max(1, per_cu_cap) * cus;
-  int rc = build_items(c);
+  int rc = build_items(c, c->tb);
   if (rc) {
     std::string m = c->err;
     twmc_sweep_destroy(reinterpret_cast<twmc_sweep_ctx*>(c));
@@ -861,14 +871,15 @@ void twmc_sweep_destroy(twmc_sweep_ctx* ctx) {
 int twmc_sweep_set_batching(twmc_sweep_ctx* ctx, const int32_t* tb) {
   if (!ctx || !tb) return sfail(nullptr, TWMC_ERR_INVALID, "null argument");
   SweepCtx* c = reinterpret_cast<SweepCtx*>(ctx);
+  std::vector<int> next(c->pts.size());
   for (size_t p = 0; p < c->pts.size(); ++p) {
     const SweepPointDev& P = c->dev_pts[p];
     const int v = tb[p];
     if (v < 1 || v > kMaxRows || (int64_t)v * P.nx * P.ny > kSweepMaxSites)
       return sfail(c, TWMC_ERR_INVALID, "stacking exceeds 4096 sites or 256 trajectories");
-    c->tb[p] = std::min(v, P.n_traj);
+    next[p] = std::min(v, P.n_traj);
   }
-  return build_items(c);
+  return build_items(c, next);
 }
 
 int twmc_sweep_get_batching(twmc_sweep_ctx* ctx, int32_t* tb) {
@@ -906,6 +917,7 @@ int twmc_sweep_run(twmc_sweep_ctx* ctx, double t_start, double t_end, int32_t us
     if (c->d_m2) (void)hipFree(c->d_m2);
     if (c->d_m4) (void)hipFree(c->d_m4);
     c->d_m2 = c->d_m4 = nullptr;
+    c->m_cap = 0;
     SCHK(c, hipMalloc(&c->d_m2, need * 8));
     SCHK(c, hipMalloc(&c->d_m4, need * 8));
     c->m_cap = need;
@@ -914,6 +926,7 @@ int twmc_sweep_run(twmc_sweep_ctx* ctx, double t_start, double t_end, int32_t us
   if (kneed > c->ksum_cap) {
     if (c->d_ksum) (void)hipFree(c->d_ksum);
     c->d_ksum = nullptr;
+    c->ksum_cap = 0;
     SCHK(c, hipMalloc(&c->d_ksum, kneed * 8));
     c->ksum_cap = kneed;
   }

@@ -132,3 +132,30 @@ def test_network_after_a_failed_call(run, hidden):
     m.close()
     print("done")
     """)
+
+
+def test_sweep_after_a_failed_call(run):
+    """A stacking that is refused or fails, and a run whose outputs do not fit, leave the sweep as it was."""
+    run("""
+    point = dict(nx=1, ny=64, gamma=1.0, J=1.0, U=0.1, F=1.0, traj_id0=0, n_traj=1000)
+    sw = Sweep([point, dict(point, nx=4, ny=8)], 0.005, 10, 3)
+    tb = sw.batching()
+    first = sw.run(0.2, graph=False)
+    for limit, call in ((4000, lambda: sw.set_batching([1, 1])), (1 << 40, lambda: sw.set_batching([2, 1000])),
+                        (100000, lambda: sw.run(2.0, graph=False))):
+        fail.fail_device_above(limit)
+        try:
+            call()
+            raise SystemExit("no error")
+        except TWMCError:
+            pass
+        fail.fail_device_above(1 << 40)
+        assert sw.batching() == tb
+        again = sw.run(0.2, graph=False)
+        for a, b in zip(first["m2"] + first["m4"], again["m2"] + again["m4"]):
+            np.testing.assert_array_equal(a, b)
+        # added atomically, 64000 terms in any order
+        np.testing.assert_allclose(first["ksum"], again["ksum"], rtol=1e-11)
+    sw.close()
+    print("done")
+    """)

@@ -1153,6 +1153,9 @@ int twmc_batch_begin(twmc_ctx* ctx, const twmc_batch_desc* d) {
     return fail(c, TWMC_ERR_INVALID, "TWMC_INIT_PREVIOUS needs beta_prev");
   HIPCHK(c, hipSetDevice(c->device));
   HIPCHK(c, hipStreamSynchronize(c->stream));
+  // from here on the earlier batch is gone, whatever fails below: buffers are replaced
+  // one by one
+  c->batch_active = false;
   c->desc = *d;
   c->desc.traj_ids = nullptr;
   c->desc.beta_prev = nullptr;

@@ -159,3 +159,24 @@ def test_sweep_after_a_failed_call(run):
     sw.close()
     print("done")
     """)
+
+
+def test_no_batch_after_a_failed_begin(run):
+    run("""
+    spec = c2_spec(nx=4, ny=8, frame_steps=5, t_end=0.002 * 15.25)
+    eng = Engine(system(spec), precision=32)
+    want = eng.run(np.arange(3), final=True).beta_final
+    for good in (3, 40):
+        eng.begin(np.arange(good))
+        fail.fail_device_above(100000)
+        for call in (lambda: eng.begin(np.arange(5000)), lambda: eng.advance(1), eng.read):
+            try:
+                call()
+                raise SystemExit("no error")
+            except TWMCError as e:
+                assert "memory" in str(e) or "no active batch" in str(e)
+        np.testing.assert_array_equal(eng.run(np.arange(3), final=True).beta_final, want)
+        fail.fail_device_above(1 << 40)
+    eng.close()
+    print("done")
+    """)

@@ -143,7 +143,7 @@ struct Ctx {
   SparsePlan sparse;  // LDS kernel, matrix hopping: its steps on the sparse kernel
   bool band_dense = false;  // banded kernel: the batch's form (band_dense)
   int tb = 0;               // MFMA kernel: trajectories per workgroup
-  int group = 1, group_slots = 0;  // ahead kernel: most frames in one launch, their partial slots
+  int group = 1;            // ahead kernel: most frames in one launch
   int vary = 0;              // scan_vary and scan_u_real: the parameters are fixed
   bool u_is_real = false;
   bool ahead = false;       // LDS kernel: its steps on the ahead kernel
@@ -783,21 +783,17 @@ int read_states(Ctx* c, const void* src, size_t count, double* dst) {
 // several (into the trajectory output if it was asked for), whose sums one capture
 // and one reduction launch then form.  A frame of a small lattice is otherwise three
 // launches of which the steps are a small part (256 trajectories of 64 sites, FP64, 21
-// frames of 200 steps: the call 1.17 -> 1.00 ms; 100 of 4x4, 21 of 100: 0.67 -> 0.46).  The states and the
-// partial sums of a group stay within 16 MiB each, its steps within 16384 (a few ms).
+// frames of 200 steps: the call 1.17 -> 1.00 ms; 100 of 4x4, 21 of 100: 0.67 -> 0.46).
+// Every frame has the slots of a single one, so its sums do not depend on the pieces
+// a run is advanced in.  The states of a group stay within 16 MiB, the partial sums
+// within 64 MiB, its steps within 16384 (a few ms).
 void plan_group(Ctx* c, size_t B) {
   c->group = 1;
-  c->group_slots = 0;
   if (!c->ahead || !generic_capture_overwrites(c->n)) return;
-  size_t most = std::min<size_t>({(size_t)c->n_frames, 64, 16384 / (size_t)c->p.frame_steps});
-  for (; most > 1; most /= 2) {
-    const size_t slots = std::min<size_t>(c->grid, std::max<size_t>(16, 2048 / most));
-    if (B * most * c->n * c->es <= (16u << 20) && most * slots * kQ * c->n * sizeof(double) <= (16u << 20)) {
-      c->group = (int)most;
-      c->group_slots = (int)slots;
-      return;
-    }
-  }
+  const size_t state = B * c->n * c->es, sums = (size_t)c->grid * kQ * c->n * sizeof(double);
+  const size_t most = std::min<size_t>({(size_t)c->n_frames, 64, 16384 / (size_t)c->p.frame_steps,
+                                        (16u << 20) / state, (64u << 20) / sums});
+  c->group = std::max<int>(1, (int)most);
 }
 
 // segments from k on that one launch of the ahead kernel can take: each stores a
@@ -835,10 +831,10 @@ int advance_group(Ctx* c, StepArgs a, int m, hipStream_t s) {
   HIPCHK(c, timed(c, c->ev_red, s, true, r0));
   a.capture = 1;
   a.n_steps = 0;
-  HIPCHK(c, launch_generic(a, c->precision, c->group_slots, c->block, c->lds, s));
+  HIPCHK(c, launch_generic(a, c->precision, c->grid, c->block, c->lds, s));
   ReduceArgs r{};
   r.n = c->n;
-  r.slots = c->group_slots;
+  r.slots = c->grid;
   r.keep = 1;
   r.frames = m;
   r.partials_in = static_cast<const double*>(c->d_partials.p);
@@ -1228,7 +1224,7 @@ int twmc_batch_begin(twmc_ctx* ctx, const twmc_batch_desc* d) {
   const int slots = std::max({c->grid, c->cap_grid, site_sum_chunks(B, kSiteSumChunks, &ss_chunk)});
   size_t part_bytes = (size_t)slots * kQ * n * sizeof(double);
   plan_group(c, B);
-  HIPCHK(c, c->d_partials.ensure(std::max(part_bytes, (size_t)c->group * c->group_slots * kQ * n * sizeof(double))));
+  HIPCHK(c, c->d_partials.ensure(std::max(part_bytes, (size_t)c->group * c->grid * kQ * n * sizeof(double))));
   if (c->group > 1 && !(d->outputs & TWMC_OUT_TRAJ)) HIPCHK(c, c->d_frames.ensure(B * c->group * n * c->es));
   // only the launches that add to their rows need them cleared (168 MB for the
   // 64x64 ensemble's 1024 slots): the capture inside a step launch, and the

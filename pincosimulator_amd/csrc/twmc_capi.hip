@@ -1224,8 +1224,13 @@ int twmc_batch_begin(twmc_ctx* ctx, const twmc_batch_desc* d) {
   const int slots = std::max({c->grid, c->cap_grid, site_sum_chunks(B, kSiteSumChunks, &ss_chunk)});
   size_t part_bytes = (size_t)slots * kQ * n * sizeof(double);
   plan_group(c, B);
-  HIPCHK(c, c->d_partials.ensure(std::max(part_bytes, (size_t)c->group * c->grid * kQ * n * sizeof(double))));
-  if (c->group > 1 && !(d->outputs & TWMC_OUT_TRAJ)) HIPCHK(c, c->d_frames.ensure(B * c->group * n * c->es));
+  if (c->group > 1 &&
+      (c->d_partials.ensure(std::max(part_bytes, (size_t)c->group * c->grid * kQ * n * sizeof(double))) != hipSuccess ||
+       (!(d->outputs & TWMC_OUT_TRAJ) && c->d_frames.ensure(B * c->group * n * c->es) != hipSuccess))) {
+    (void)hipGetLastError();  // no memory for several frames: one per launch
+    c->group = 1;
+  }
+  HIPCHK(c, c->d_partials.ensure(part_bytes));
   // only the launches that add to their rows need them cleared (168 MB for the
   // 64x64 ensemble's 1024 slots): the capture inside a step launch, and the
   // LDS kernel's capture of a lattice above generic_capture_overwrites

@@ -180,3 +180,20 @@ def test_no_batch_after_a_failed_begin(run):
     eng.close()
     print("done")
     """)
+
+
+def test_frames_one_by_one_without_memory_for_groups(run):
+    """256 trajectories of 64 sites, 20 frames: 0.7 MB of partial sums and 0.3 MB of states a frame."""
+    run("""
+    spec = c2_spec(nx=1, ny=64, frame_steps=4, t_end=0.002 * 76.25)
+    out = []
+    for bytes in (1000000, 1 << 40):
+        fail.fail_device_above(bytes)
+        eng = Engine(system(spec), precision=64, kernel="generic")
+        out.append(eng.run(np.arange(256), final=True))
+        eng.close()
+    assert out[0].n_frames == 20 and fail.failures() == 1
+    for k in ("beta_final", "traj_m2", "sum_n", "sum_nk"):
+        np.testing.assert_array_equal(getattr(out[0], k), getattr(out[1], k))
+    print("done")
+    """)

@@ -268,13 +268,15 @@ Launch launch_s(int m, bool unif, bool xn) {
 }
 
 template <typename T>
-Launch launch_t(const StepArgs& a) {
-  const int m = a.hopping == 1 ? a.ell_m : 0;
-  const bool unif = a.site_uniform != 0, xn = a.nx > 1;
-  return a.n <= 64    ? launch_s<T, 1>(m, unif, xn)
-         : a.n <= 128 ? launch_s<T, 2>(m, unif, xn)
-         : a.n <= 256 ? launch_s<T, 4>(m, unif, xn)
-                      : launch_s<T, 8>(m, unif, xn);
+Launch launch_t(int n, int m, bool unif, bool xn) {
+  return n <= 64    ? launch_s<T, 1>(m, unif, xn)
+         : n <= 128 ? launch_s<T, 2>(m, unif, xn)
+         : n <= 256 ? launch_s<T, 4>(m, unif, xn)
+                    : launch_s<T, 8>(m, unif, xn);
+}
+
+Launch launch_of(int precision, int n, int m, bool unif, bool xn) {
+  return precision == 64 ? launch_t<double>(n, m, unif, xn) : launch_t<float>(n, m, unif, xn);
 }
 
 }  // namespace
@@ -307,8 +309,13 @@ bool ahead_pays_sparse(int n, int most, int precision, size_t n_traj, int cus) {
   return (n <= 256 || (n <= 512 && most <= 3)) && n_traj <= (size_t)per_cu * cus;
 }
 
+LaunchShape ahead_shape(int n, int ell_m, int precision, size_t n_traj) {
+  const Launch l = launch_of(precision, n, ell_m, false, false);  // the same for all forms
+  return {(int)n_traj, l.block, l.lds};
+}
+
 hipError_t launch_ahead(const StepArgs& a, int precision, hipStream_t s) {
-  const Launch l = precision == 64 ? launch_t<double>(a) : launch_t<float>(a);
+  const Launch l = launch_of(precision, a.n, a.hopping == 1 ? a.ell_m : 0, a.site_uniform != 0, a.nx > 1);
   if (l.lds > 65536) {
     hipError_t e = hipFuncSetAttribute(l.f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)l.lds);
     if (e != hipSuccess) return e;

@@ -139,6 +139,7 @@ struct Ctx {
   size_t seg_recorded = 0;
   mutable size_t seg_completed = 0;
   int grid = 0, block = 256;
+  LaunchShape step;  // the step launch, whichever kernel takes it (twmc_query)
   int cap_grid = 0;  // stencil64: grid of the capture launch (the 64x64 FFT kernel's)
   SparsePlan sparse;  // LDS kernel, matrix hopping: its steps on the sparse kernel
   bool band_dense = false;  // banded kernel: the batch's form (band_dense)
@@ -556,6 +557,7 @@ struct Geometry {
   size_t lds = 0;
   int grid_nn = 0;  // LDS kernel with FFT hopping: the step launch without the FFT's second buffer
   size_t lds_nn = 0;
+  LaunchShape step;   // the step launch, whichever kernel takes it
   SparsePlan sparse;  // LDS kernel with matrix hopping: the step launch on the sparse kernel
   bool band_dense = false;
   int tb = 0;          // MFMA kernel: trajectories per workgroup
@@ -606,7 +608,7 @@ int step_geometry(Ctx* c, size_t B, Geometry& geo) {
         nn_supported(c->p.nx, c->p.ny, c->precision, c->vary) &&
         nn_pays(c->p.nx, c->p.ny, c->precision, c->vary, B, cus)) {
       int per_cu_nn = 0;
-      HIPCHK(c, nn_occupancy(c->p.nx, c->p.ny, c->precision, c->vary, c->u_is_real, &per_cu_nn));
+      HIPCHK(c, nn_occupancy(c->p.nx, c->p.ny, c->precision, c->vary, c->u_is_real, &per_cu_nn, &geo.step));
       if (per_cu_nn < 1) return fail(c, TWMC_ERR_UNSUPPORTED, "step kernel does not fit on a CU");
       geo.nn = true;
       geo.grid_nn = (int)std::min<size_t>(B, (size_t)per_cu_nn * cus);
@@ -624,6 +626,16 @@ int step_geometry(Ctx* c, size_t B, Geometry& geo) {
     geo.grid = balanced_wave_grid(B, per_cu, cus);
   else
     geo.grid = (int)std::min<size_t>(units, (size_t)per_cu * cus);
+  if (geo.ahead)
+    geo.step = ahead_shape(c->n, c->ell_m, c->precision, B);
+  else if (geo.nn)
+    geo.step.grid = geo.grid_nn;
+  else if (c->ell_m > 0)
+    geo.step = geo.sparse.step;
+  else if (geo.grid_nn > 0)
+    geo.step = {geo.grid_nn, generic_nn_block(c->precision, c->n, site_uniform(c)), geo.lds_nn};
+  else
+    geo.step = {geo.grid, geo.block, geo.lds};
   return TWMC_OK;
 }
 
@@ -1193,6 +1205,7 @@ int twmc_batch_begin(twmc_ctx* ctx, const twmc_batch_desc* d) {
     c->nn = geo.nn;
     c->grid_nn = geo.grid_nn;
     c->lds_nn = geo.lds_nn;
+    c->step = geo.step;
   }
   if (c->kernel == TWMC_KERNEL_STACK) {
     // steps on the sweep kernel; frames stay with the LDS kernel (geometry above).
@@ -1209,6 +1222,7 @@ int twmc_batch_begin(twmc_ctx* ctx, const twmc_batch_desc* d) {
     }
     HIPCHK(c, stack_prepare(c->stack, c->p.nx, c->p.ny, (int)B, rsl, c->base[1].data(), c->base[2].data(), c->dt4,
                             -2.0 * c->p.J));
+    c->step = c->stack.step;
   }
 
   size_t sets = c->noisy_params ? B : 1;
@@ -1508,9 +1522,9 @@ int twmc_query(twmc_ctx* ctx, twmc_stats* st) {
   }
   c->ev_red.clear();
   c->stats.kernel = c->kernel;
-  c->stats.grid = c->grid;
-  c->stats.block = c->block;
-  c->stats.lds_bytes = (int)c->lds;
+  c->stats.grid = c->step.grid;
+  c->stats.block = c->step.block;
+  c->stats.lds_bytes = (int)c->step.lds;
   *st = c->stats;
   return TWMC_OK;
 }

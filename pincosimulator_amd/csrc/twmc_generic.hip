@@ -983,6 +983,14 @@ const void* generic_nn_ptr(int precision, int ppt, bool unif, int lay, int block
               : generic_nn_ptr_u<float, false>(ppt, lay, block, tpb);
 }
 
+// trajectories per workgroup of a nearest-neighbour step launch (TPB)
+int nn_tpb(int n) {
+  const int np = (n + 1) / 2;
+  return np <= 16 ? 4 : np <= 32 ? 2 : 1;
+}
+
+}  // namespace
+
 // threads per workgroup of a nearest-neighbour step launch: one or two waves
 // for lattices of up to 128 or 256 sites (a pair per thread, every wave busy),
 // 1024 for FP64 site-uniform lattices of 2049 to 4096 sites (with even rows and
@@ -993,14 +1001,6 @@ int generic_nn_block(int precision, int n, bool unif) {
   if (np <= 128) return 128;
   return (precision == 64 && unif && generic_pairs_per_thread(n, 1024) == 2) ? 1024 : kBlock;
 }
-
-// trajectories per workgroup of a nearest-neighbour step launch (TPB)
-int nn_tpb(int n) {
-  const int np = (n + 1) / 2;
-  return np <= 16 ? 4 : np <= 32 ? 2 : 1;
-}
-
-}  // namespace
 
 // LDS of a nearest-neighbour step launch: the per-wave sums, one copy of the
 // state per trajectory of the workgroup (two for the double-buffered

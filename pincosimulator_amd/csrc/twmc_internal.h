@@ -201,6 +201,7 @@ size_t generic_nn_lds_bytes(int nx, int ny, int precision, bool site_uniform);
 // trajectories per workgroup of the nearest-neighbour step launch (1, 2 or 4):
 // its grid covers ceil(B / that) workgroups
 int generic_nn_traj_per_block(int n);
+int generic_nn_block(int precision, int n, bool site_uniform);  // its threads per workgroup
 hipError_t generic_nn_occupancy(int precision, int nx, int ny, size_t lds, bool site_uniform,
                                 int* blocks_per_cu);
 hipError_t launch_generic_nn(const StepArgs& a, int precision, int grid, size_t lds, hipStream_t s);
@@ -224,13 +225,20 @@ size_t mfma_lds_bytes(int np, int tb);
 int mfma_tb(int np, size_t n_traj, int cus);  // trajectories per workgroup
 hipError_t launch_mfma(const StepArgs& a, int grid, hipStream_t s);
 
+// workgroups, threads per workgroup and dynamic LDS of a step launch
+struct LaunchShape {
+  int grid = 0, block = 0;
+  size_t lds = 0;
+};
+
 // one-point batches of the main API on the sweep kernel: FP32, FFT hopping,
 // site-uniform shared parameters, no F(t)
 struct StackPlan {
   void* d_point = nullptr;
   void* d_items = nullptr;
   void* d_counter = nullptr;
-  int n_items = 0, grid = 0, tb = 1;
+  int n_items = 0, tb = 1;
+  LaunchShape step;
   bool u_real = false;  // Im U = 0
 };
 bool stack_supported(int nx, int ny);
@@ -261,7 +269,7 @@ hipError_t band_occupancy(int n, int w, int lieb, int uni, int dense, int* block
 constexpr int kVaryNone = 0, kVaryRsl = 1, kVaryF = 4;  // a bit for each of rsl, U, F
 bool nn_supported(int nx, int ny, int precision, int vary);
 bool nn_pays(int nx, int ny, int precision, int vary, size_t n_traj, int cus);
-hipError_t nn_occupancy(int nx, int ny, int precision, int vary, bool u_real, int* blocks_per_cu);
+hipError_t nn_occupancy(int nx, int ny, int precision, int vary, bool u_real, int* blocks_per_cu, LaunchShape* shape);
 hipError_t launch_nn(const StepArgs& a, int precision, int grid, hipStream_t s);
 
 // FFT hopping, up to 256 sites, static parameters: the step launch of the LDS kernel
@@ -269,6 +277,8 @@ hipError_t launch_nn(const StepArgs& a, int precision, int grid, hipStream_t s);
 bool ahead_pays(int nx, int ny, int precision, size_t n_traj, int cus);
 // matrix hopping with few nonzeros per column, up to 512 sites, static parameters: the same
 bool ahead_pays_sparse(int n, int most, int precision, size_t n_traj, int cus);
+// ell_m: StepArgs::ell_m, 0: FFT hopping
+LaunchShape ahead_shape(int n, int ell_m, int precision, size_t n_traj);
 hipError_t launch_ahead(const StepArgs& a, int precision, hipStream_t s);
 
 // matrix hopping with at most six nonzeros per column (`most`), up to 512 sites:
@@ -277,8 +287,7 @@ constexpr int kSparseMaxSites = 512;
 struct SparsePlan {
   int s = 0;  // sites per lane, 0: not planned
   bool prio = false;
-  int grid = 0;
-  size_t lds = 0;
+  LaunchShape step;
 };
 int sparse_entries(int most);  // entries per column of the kernel's table, 0: too many
 bool sparse_supported(int n, int hopping, int most);

@@ -320,8 +320,10 @@ bool nn_pays(int nx, int ny, int precision, int vary, size_t n_traj, int cus) {
   return n <= 512 ? per_cu >= 4 : n <= 2048 || n_traj > 2 * (size_t)cus;
 }
 
-hipError_t nn_occupancy(int nx, int ny, int precision, int vary, bool u_real, int* blocks_per_cu) {
+hipError_t nn_occupancy(int nx, int ny, int precision, int vary, bool u_real, int* blocks_per_cu, LaunchShape* shape) {
   const Launch l = launch_of(nx, ny, precision, vary, u_real);
+  shape->block = l.block;
+  shape->lds = l.lds;
   hipError_t e = allow_lds(l);
   if (e != hipSuccess) return e;
   return hipOccupancyMaxActiveBlocksPerMultiprocessor(blocks_per_cu, l.f, l.block, l.lds);

@@ -309,8 +309,7 @@ hipError_t sparse_plan(int n, int precision, int most, size_t n_traj, int cus, S
         best = cost;
         plan->s = s;
         plan->prio = prio;
-        plan->lds = lds;
-        plan->grid = (int)std::min(blocks, grid);
+        plan->step = {(int)std::min(blocks, grid), 64 * kWaves, lds};
       }
     }
   }
@@ -319,12 +318,12 @@ hipError_t sparse_plan(int n, int precision, int most, size_t n_traj, int cus, S
 
 hipError_t launch_sparse(const StepArgs& a, int precision, const SparsePlan& plan, hipStream_t s) {
   const void* f = kernel_for(precision, plan.s, a.ell_m, plan.prio);
-  if (plan.lds > 65536) {
-    hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)plan.lds);
+  if (plan.step.lds > 65536) {
+    hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)plan.step.lds);
     if (e != hipSuccess) return e;
   }
   void* args[] = {const_cast<StepArgs*>(&a)};
-  return hipLaunchKernel(f, dim3(plan.grid), dim3(64 * kWaves), args, plan.lds, s);
+  return hipLaunchKernel(f, dim3(plan.step.grid), dim3(plan.step.block), args, plan.step.lds, s);
 }
 
 }  // namespace twmc

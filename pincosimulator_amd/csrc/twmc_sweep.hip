@@ -694,7 +694,7 @@ hipError_t stack_prepare(StackPlan& sp, int nx, int ny, int n_traj, const double
   for (int t0 = 0; t0 < n_traj; t0 += P.tb) items.push_back(SweepItemDev{0, t0});
   sp.n_items = (int)items.size();
   sp.tb = P.tb;
-  sp.grid = std::min(sp.n_items, slots);
+  sp.step = {std::min(sp.n_items, slots), kStepBlock, sweep_lds_bytes(false)};
   if (e == hipSuccess) e = hipMalloc(&sp.d_point, sizeof(SweepPointDev));
   if (e == hipSuccess) e = hipMalloc(&sp.d_items, items.size() * sizeof(SweepItemDev));
   if (e == hipSuccess) e = hipMalloc(&sp.d_counter, 2 * sizeof(unsigned int));
@@ -719,7 +719,7 @@ hipError_t stack_launch(const StackPlan& sp, const StepArgs& a, hipStream_t s) {
   g.n_steps = a.n_steps;
   g.traj_ids = a.traj_ids;
   hipLaunchKernelGGL(sweep_reset_kernel, dim3(1), dim3(64), 0, s, (unsigned int*)sp.d_counter);
-  return launch_step(g, sp.u_real, sp.grid, s);
+  return launch_step(g, sp.u_real, sp.step.grid, s);
 }
 
 void stack_release(StackPlan& sp) {

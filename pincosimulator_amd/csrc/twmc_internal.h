@@ -84,7 +84,7 @@ struct StepArgs {
   const void* a_lo;
   int np;                    // n padded to a multiple of 128
   int tb;                    // MFMA kernel: trajectories per workgroup
-  unsigned int* queue;       // 64x64 stencil and nn kernels: work queue of the launch (one word)
+  unsigned int* queue;       // 64x64 stencil and nn kernels: work queue of the launch (one word), null: fixed shares
   // several frames in one launch (ahead kernel, capture-only launch of the LDS kernel):
   // frame0 + k, k < group, lies at frames[trajectory][frames_stride][n]; the steps
   // store it after k group_steps steps
@@ -230,6 +230,18 @@ struct LaunchShape {
   int grid = 0, block = 0;
   size_t lds = 0;
 };
+
+// Whether a step launch of the 64x64 stencil and nn kernels takes its trajectories from
+// the queue, or each workgroup a fixed share.  The queue evens out the workgroups of a
+// CU, which do not advance alike, but hands out one trajectory after the other, about 12
+// ns each, so the steps of one (FP32 1e12 site-steps/s, FP64 a third) have to take
+// longer.  us of a launch, queue / share: 8192 trajectories of 17x21, 1 step 105 / 17, 30
+// steps 132 / 136, 100 steps 379 / 429; 20000 of 5x13, 30 steps 248 / 95, 300 steps 854 /
+// 859; 4096 of 32x32, 10 steps 69 / 63, 30 steps 153 / 162; 4096 of 64x64, 3 steps 82 / 81, 10
+// steps 190 / 193, 100 steps 1560 / 1683; FP64, 3000 of 40x41, 1 step 50 / 40, 10 steps 184 / 190.
+inline bool queue_pays(const StepArgs& a, int grid, int precision) {
+  return a.n_traj > grid && (uint64_t)a.n_steps * (uint64_t)a.n >= (precision == 64 ? 8192u : 20000u);
+}
 
 // one-point batches of the main API on the sweep kernel: FP32, FFT hopping,
 // site-uniform shared parameters, no F(t)

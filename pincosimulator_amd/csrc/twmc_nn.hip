@@ -4,7 +4,8 @@
 // stacked kernel does not take (rows of odd length, an energy or a drive that varies
 // from site to site or is drawn per trajectory).  One workgroup owns one trajectory:
 // a pair per thread (two for 2049 to 4096 sites), the state in registers, the
-// neighbours from one LDS copy of it; trajectories come from a work queue.
+// neighbours from one LDS copy of it; in launches of more than a few steps
+// (queue_pays) trajectories come from a work queue.
 //
 // What bounds it: VALU issue, at eight waves per SIMD.
 //  * FP64, uniform: the LDS kernel (twmc_generic.hip) keeps the Box-Muller
@@ -220,8 +221,12 @@ __global__ void __launch_bounds__(BLOCK, waves_per_simd(sizeof(T), PPT, V)) nn_s
         const int i = 2 * (threadIdx.x + BLOCK * j) + h;
         if (i < n) gb[i] = beta[2 * j + h];
       }
-    // the next trajectory, from the queue (the barriers of the steps separate this
-    // word's uses)
+    // the next trajectory: of this workgroup's share, or from the queue (the barriers of
+    // the steps separate this word's uses)
+    if (!g.queue) {
+      b += gridDim.x;
+      continue;
+    }
     if (threadIdx.x == 0) *s_next = (int)(gridDim.x + atomicAdd(g.queue, 1u));
     __syncthreads();
     b = __builtin_amdgcn_readfirstlane(*s_next);
@@ -333,8 +338,10 @@ hipError_t launch_nn(const StepArgs& a, int precision, int grid, hipStream_t s) 
   const Launch l = launch_of(a.nx, a.ny, precision, a.vary, a.u_real != 0);
   hipError_t e = allow_lds(l);
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(queue_reset_kernel, dim3(1), dim3(64), 0, s, a.queue);
-  void* args[] = {const_cast<StepArgs*>(&a)};
+  StepArgs q = a;
+  if (!queue_pays(a, grid, precision)) q.queue = nullptr;
+  else hipLaunchKernelGGL(queue_reset_kernel, dim3(1), dim3(64), 0, s, q.queue);
+  void* args[] = {&q};
   return hipLaunchKernel(l.f, dim3(grid), dim3(l.block), args, l.lds, s);
 }
 

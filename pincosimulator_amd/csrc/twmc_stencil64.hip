@@ -39,9 +39,9 @@ constexpr int kL = 64;
 // What bounds it: VALU issue, 44.5 instructions per site-step of which the four
 // transcendental ones run on their own unit beside the others when other waves
 // have work: 64 registers for eight waves per SIMD, two workgroups per CU.  The
-// two do not advance evenly (the older one is served first), so trajectories are
-// taken from a queue: dealt out by workgroup, one of the two finished early and
-// left the other to a half-filled CU.  16384 trajectories, 500-step launches:
+// two do not advance evenly (the older one is served first), so in launches of more
+// than a few steps (queue_pays) trajectories are taken from a queue: dealt out by
+// workgroup, one of the two finished early and left the other to a half-filled CU.  16384 trajectories, 500-step launches:
 // 60.9 us per step = 1.10e12 site-steps/s; dealt out 69.6; one wave per trajectory
 // with its rows in registers (128 VGPRs, four waves per SIMD), the form before
 // both, 80.2; this form at four waves per SIMD 75.8; raised priority around the
@@ -76,7 +76,7 @@ __global__ void __launch_bounds__(kBlock, 8) stencil64_step_kernel(StepArgs g) {
   const int lft = row + ((p0 - 1) & 31), rgt = row + ((p0 + 1) & 31);
   const int dn0 = (p0 - 32) & (kPairs - 1), up1 = (p0 + kBlock + 32) & (kPairs - 1);
 
-  // the first trajectory by workgroup, the next ones from the queue
+  // the first trajectory by workgroup, the next ones as the launch says
   for (int b = blockIdx.x; b < g.n_traj;) {
     const uint64_t traj = g.traj_ids[b];
     float4* gb = reinterpret_cast<float4*>(reinterpret_cast<cpx<float>*>(g.beta) + (size_t)b * kL * kL);
@@ -142,10 +142,11 @@ __global__ void __launch_bounds__(kBlock, 8) stencil64_step_kernel(StepArgs g) {
       const cpx<float> v0 = beta[2 * j], v1 = beta[2 * j + 1];
       gb[p0 + kBlock * j] = make_float4(v0.re, v0.im, v1.re, v1.im);
     }
-    // the next trajectory, through a word of copy 1 (its load writes copy 0)
+    // the next trajectory: of this workgroup's share, or from the queue; through a word of
+    // copy 1 (its load writes copy 0)
     int* next = reinterpret_cast<int*>(&st[1][0][0]);
     __syncthreads();
-    if (threadIdx.x == 0) *next = (int)(gridDim.x + atomicAdd(g.queue, 1u));
+    if (threadIdx.x == 0) *next = (int)(gridDim.x + (g.queue ? atomicAdd(g.queue, 1u) : (unsigned int)b));
     __syncthreads();
     b = __builtin_amdgcn_readfirstlane(*next);
   }
@@ -158,11 +159,13 @@ bool stencil64_supported(int nx, int ny, int hopping, int precision, int param_s
 }
 
 hipError_t launch_stencil64(const StepArgs& a, int grid, hipStream_t s) {
-  hipLaunchKernelGGL(queue_reset_kernel, dim3(1), dim3(64), 0, s, a.queue);
+  StepArgs q = a;
+  if (!queue_pays(a, grid, 32)) q.queue = nullptr;
+  else hipLaunchKernelGGL(queue_reset_kernel, dim3(1), dim3(64), 0, s, q.queue);
   if (a.u_real)
-    hipLaunchKernelGGL(stencil64_step_kernel<true>, dim3(grid), dim3(kBlock), 0, s, a);
+    hipLaunchKernelGGL(stencil64_step_kernel<true>, dim3(grid), dim3(kBlock), 0, s, q);
   else
-    hipLaunchKernelGGL(stencil64_step_kernel<false>, dim3(grid), dim3(kBlock), 0, s, a);
+    hipLaunchKernelGGL(stencil64_step_kernel<false>, dim3(grid), dim3(kBlock), 0, s, q);
   return hipGetLastError();
 }
 

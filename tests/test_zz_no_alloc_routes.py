@@ -18,7 +18,7 @@ def lieb(cells):
 
 CASES = [("stencil64", 32, base.square(64, 64, 30), 1100, 600),
          ("generic", 64, base.square(64, 64, 30), 600, 513),
-         ("generic", 32, base.square(17, 21, 30), 5000, 2500),
+         ("generic", 32, base.square(27, 41, 30), 3000, 1500),
          ("generic", 64, dict(base.square(16, 18, 30), F=1.4 * np.exp(0.01j * np.arange(288))), 4500, 300),
          ("generic", 64, lieb(24), 2100, 70),
          ("generic", 64, lieb(128), 1000, 600),

@@ -54,7 +54,7 @@ constexpr int kMaxNy = 512;    // row length (chain length or 2D row)
 struct SweepPointDev {
   int nx, ny, tb, fft_x;  // fft_x = 1: 2D point (rows are lattice rows), 0: stacked 1D trajectories
   RadixPlan px, py;
-  int tw_x, tw_y, kc_x, kc_y;  // offsets into the table pools
+  int tw_x, tw_y;  // offsets into the twiddle pool
   float rsl_re, rsl_im, u_re, u_im, f_re, f_im;
   float dt4, kscale;
   int n_traj;
@@ -75,7 +75,6 @@ struct SweepArgs {
   int n_items;
   unsigned int* counter;
   const cpx<float>* tw_pool;
-  const float* kc_pool;
   cpx<float>* beta;
   double* traj_m2;
   double* traj_m4;
@@ -495,10 +494,9 @@ struct SweepCtx {
   std::vector<int> tb;  // trajectories per work item, per point
   bool u_real = true;   // Im U = 0 in every point
   std::vector<cpx<float>> tw_pool;
-  std::vector<float> kc_pool;
   std::vector<unsigned char> bin_pool;
   uint64_t total_traj = 0, total_sites = 0;
-  void *d_points = nullptr, *d_items = nullptr, *d_counter = nullptr, *d_tw = nullptr, *d_kc = nullptr,
+  void *d_points = nullptr, *d_items = nullptr, *d_counter = nullptr, *d_tw = nullptr,
        *d_beta = nullptr, *d_m2 = nullptr, *d_m4 = nullptr, *d_binit = nullptr, *d_bins = nullptr,
        *d_ksum = nullptr;
   size_t ksum_cap = 0;
@@ -522,15 +520,14 @@ int sfail(SweepCtx* c, int code, const std::string& m) {
     if (e_ != hipSuccess) return sfail(c, TWMC_ERR_HIP, std::string(#expr ": ") + hipGetErrorString(e_)); \
   } while (0)
 
-int add_tables(SweepCtx* c, int L, int& tw_off, int& kc_off) {
-  tw_off = (int)c->tw_pool.size();
-  kc_off = (int)c->kc_pool.size();
+// the twiddle factors of length L; returns their offset
+int add_twiddles(SweepCtx* c, int L) {
+  const int off = (int)c->tw_pool.size();
   for (int m = 0; m < L; ++m) {
     long double a = -2.0L * 3.14159265358979323846264338327950288L * m / L;
     c->tw_pool.push_back(mk(float(cosl(a)), float(sinl(a))));
-    c->kc_pool.push_back(L == 1 ? 0.0f : float(cos(2.0 * M_PI / double(L) * double(m))));
   }
-  return 0;
+  return off;
 }
 
 // radial bin of every mode of an nx x ny lattice: bin 0 is k = 0; the other
@@ -626,7 +623,6 @@ SweepArgs base_args(SweepCtx* c) {
   a.n_items = c->n_items;
   a.counter = (unsigned int*)c->d_counter;
   a.tw_pool = (const cpx<float>*)c->d_tw;
-  a.kc_pool = (const float*)c->d_kc;
   a.beta = (cpx<float>*)c->d_beta;
   a.traj_m2 = (double*)c->d_m2;
   a.traj_m4 = (double*)c->d_m4;
@@ -754,15 +750,12 @@ int twmc_sweep_create(const twmc_sweep_point* pts, uint64_t n_points, double dt,
   c->frame_steps = frame_steps;
   c->seed = seed;
   c->pts.assign(pts, pts + n_points);
-  std::map<std::pair<int, int>, std::pair<int, int>> tables;  // length -> (tw, kc) offsets
-  std::map<std::pair<int, int>, int> bin_tables;                // shape -> bin table offset
-  auto table_for = [&](int L) {
-    auto it = tables.find({L, 0});
-    if (it != tables.end()) return it->second;
-    int a, b;
-    add_tables(c, L, a, b);
-    tables[{L, 0}] = {a, b};
-    return std::make_pair(a, b);
+  std::map<int, int> twiddles;                    // length -> offset
+  std::map<std::pair<int, int>, int> bin_tables;  // shape -> bin table offset
+  auto twiddles_of = [&](int L) {
+    auto it = twiddles.find(L);
+    if (it == twiddles.end()) it = twiddles.emplace(L, add_twiddles(c, L)).first;
+    return it->second;
   };
   uint64_t state_off = 0, m_off = 0;
   for (uint64_t p = 0; p < n_points; ++p) {
@@ -779,12 +772,8 @@ int twmc_sweep_create(const twmc_sweep_point* pts, uint64_t n_points, double dt,
       return sfail(nullptr, TWMC_ERR_UNSUPPORTED,
                    "sweep point " + std::to_string(p) + ": up to 4096 sites, 64 rows, rows of even length <= 512");
     }
-    auto ty = table_for(ny);
-    auto tx = table_for(nx);
-    P.tw_y = ty.first;
-    P.kc_y = ty.second;
-    P.tw_x = tx.first;
-    P.kc_x = tx.second;
+    P.tw_y = twiddles_of(ny);
+    P.tw_x = twiddles_of(nx);
     // rsl = -i omega - gamma/2 (TWMCBaseSolver.cpp:74)
     P.rsl_re = float(q.omega[1] - q.gamma / 2.0);
     P.rsl_im = float(-q.omega[0]);
@@ -818,7 +807,6 @@ int twmc_sweep_create(const twmc_sweep_point* pts, uint64_t n_points, double dt,
   if (e == hipSuccess) e = hipMalloc(&c->d_points, c->dev_pts.size() * sizeof(SweepPointDev));
   if (e == hipSuccess) e = hipMalloc(&c->d_counter, 256);
   if (e == hipSuccess) e = hipMalloc(&c->d_tw, c->tw_pool.size() * sizeof(cpx<float>));
-  if (e == hipSuccess) e = hipMalloc(&c->d_kc, c->kc_pool.size() * sizeof(float));
   if (e == hipSuccess) e = hipMalloc(&c->d_beta, state_off * sizeof(cpx<float>));
   std::vector<double> binit(4 * n_points);
   for (uint64_t p = 0; p < n_points; ++p) {
@@ -831,7 +819,6 @@ int twmc_sweep_create(const twmc_sweep_point* pts, uint64_t n_points, double dt,
   if (e == hipSuccess) e = hipMalloc(&c->d_bins, c->bin_pool.size());
   if (e == hipSuccess) e = hipMemcpy(c->d_bins, c->bin_pool.data(), c->bin_pool.size(), hipMemcpyHostToDevice);
   if (e == hipSuccess) e = hipMemcpy(c->d_tw, c->tw_pool.data(), c->tw_pool.size() * sizeof(cpx<float>), hipMemcpyHostToDevice);
-  if (e == hipSuccess) e = hipMemcpy(c->d_kc, c->kc_pool.data(), c->kc_pool.size() * sizeof(float), hipMemcpyHostToDevice);
   if (e == hipSuccess) e = hipMemcpy(c->d_binit, binit.data(), binit.size() * 8, hipMemcpyHostToDevice);
   if (e == hipSuccess) e = hipFuncSetAttribute((const void*)sweep_capture_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)sweep_lds_bytes(true));
   int per_cu = 0, per_cu_cap = 0, cus = 0;
@@ -860,7 +847,7 @@ void twmc_sweep_destroy(twmc_sweep_ctx* ctx) {
   SweepCtx* c = reinterpret_cast<SweepCtx*>(ctx);
   (void)hipSetDevice(c->device);
   if (c->stream) (void)hipStreamSynchronize(c->stream);
-  void* bufs[] = {c->d_points, c->d_items, c->d_items_cap, c->d_counter, c->d_tw, c->d_kc, c->d_beta, c->d_m2, c->d_m4, c->d_binit,
+  void* bufs[] = {c->d_points, c->d_items, c->d_items_cap, c->d_counter, c->d_tw, c->d_beta, c->d_m2, c->d_m4, c->d_binit,
                   c->d_bins, c->d_ksum};
   for (void* b : bufs)
     if (b) (void)hipFree(b);

@@ -380,7 +380,7 @@ __global__ void __launch_bounds__(64 * kRowWaves) mlp_rows_kernel(NetArgs g) {
   }
 }
 
-size_t rows_lds_bytes(int hidden_layers, bool train) {
+constexpr size_t rows_lds_bytes(int hidden_layers, bool train) {
   return sizeof(float) * (kRowWaves * kRowsBlock * kMaxNarrow + kRowsBlock * kActLd +
                           (train ? hidden_layers * kRowsBlock * kMaxNarrow : 0));
 }
@@ -655,13 +655,15 @@ hipError_t launch_wgrad(const MlpCtx* c, const GradArgs& a, bool adam) {
   return hipGetLastError();
 }
 
-// the fused path: every width at most kMaxNarrow, and the hidden layers'
-// pre-activations (4 KB each) beside the 69 KB of partial sums and activations
-// in the 160 KB of LDS.  Wider networks take the layer-by-layer products.
+// the fused path: every width at most kMaxNarrow.  Wider networks take the
+// layer-by-layer products.
 bool is_narrow(const MlpCtx* c) {
+  // the pre-activations of all hidden layers (4 KB each) lie beside the 69 KB of partial
+  // sums and activations in the LDS
+  static_assert(rows_lds_bytes(kMaxLayers - 1, true) + 1024 <= 160 * 1024, "a network of kMaxLayers does not fit");
   for (int l = 0; l <= c->n_layers; ++l)
     if (c->width[l] > kMaxNarrow) return false;
-  return rows_lds_bytes(c->n_layers - 1, true) + 1024 <= 160 * 1024;
+  return true;
 }
 
 // Inference on the fused kernel: every four samples read all weights, so from some

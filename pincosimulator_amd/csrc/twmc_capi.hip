@@ -598,7 +598,7 @@ int step_geometry(Ctx* c, size_t B, Geometry& geo) {
     geo.lds = generic_lds_bytes(c->p.nx, c->p.ny, c->precision);
     HIPCHK(c, generic_occupancy(c->precision, c->n, geo.block, geo.lds, &per_cu));
     if (c->ell_m > 0) {
-      HIPCHK(c, sparse_plan(c->n, c->precision, c->ell_m, B, cus, &geo.sparse));
+      HIPCHK(c, sparse_plan(c->n, c->precision, c->ell_m, c->ft_n > 0, B, cus, &geo.sparse));
       geo.ahead = c->ft_n == 0 && ahead_pays_sparse(c->n, c->ell_m, c->precision, B, cus);
     }
     if (c->kernel == TWMC_KERNEL_GENERIC && c->p.hopping == TWMC_HOP_FFT && c->ft_n == 0 &&

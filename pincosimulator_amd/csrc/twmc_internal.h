@@ -303,7 +303,7 @@ struct SparsePlan {
 };
 int sparse_entries(int most);  // entries per column of the kernel's table, 0: too many
 bool sparse_supported(int n, int hopping, int most);
-hipError_t sparse_plan(int n, int precision, int most, size_t n_traj, int cus, SparsePlan* plan);
+hipError_t sparse_plan(int n, int precision, int most, bool ft, size_t n_traj, int cus, SparsePlan* plan);
 hipError_t launch_sparse(const StepArgs& a, int precision, const SparsePlan& plan, hipStream_t s);
 
 hipError_t mfma_occupancy(int n, int tb, int* blocks_per_cu);

@@ -18,11 +18,11 @@
 // else VALU issue (about 95 instructions per FP64 site-step).  The noise does
 // not depend on the state, so with two sites per lane the next step's draw is
 // formed beside this step's LDS round trip and update.
-// Measured, per step of the whole batch, against the LDS kernel's product (256
+// Measured, us per step of the whole batch, against the LDS kernel's product (256
 // threads per trajectory, columns through global index tables): FP64 Lieb chain
-// of 72 sites x 1000 trajectories 3.47 -> 0.57 us, x 16384 37.8 -> 5.5 us, 384
-// sites x 4096 16.8 -> 6.5 us (2.4e11 site-steps/s); FP32 with drawn energies, 384
-// sites x 4096 10.1 -> 2.5 us (6.4e11).
+// of 72 sites x 2500 trajectories 6.85 -> 1.09, x 16384 37.9 -> 5.3, 384 sites x 4096
+// 16.2 -> 6.2 (2.6e11 site-steps/s); FP32 with drawn energies, 384 sites x 4096 9.8 ->
+// 2.25 (7.0e11).
 #include <algorithm>
 #include <cmath>
 
@@ -79,7 +79,12 @@ __device__ __forceinline__ void wave_sync() {
 // PRIO (FP32, more than two waves per SIMD): a wave forming its Box-Muller samples
 // goes first, so that the waves do not bunch up before the transcendental unit
 // (384 sites x 4096 2.42 -> 2.22 us per step; 72 x 1000, one wave, 0.33 -> 0.37).
-template <typename T, int S, int M, bool PRIO>
+// FT: the drive is F(t), read per step instead of held: after the hopping sums, whose
+// neighbours' registers are free by then, and under the draw (400 sites of six
+// neighbours, FP64, 64 trajectories: 3.80 -> 3.44 us per step, the LDS kernel's product
+// 3.61; three neighbours 3.23 -> 2.92, 3.04).  The eight-site form of six neighbours
+// still spills five registers.
+template <typename T, int S, int M, bool PRIO, bool FT>
 __global__ void __launch_bounds__(64 * kWaves, S == 2 ? 2 : 1) sparse_step_kernel(StepArgs g) {
   extern __shared__ __align__(16) unsigned char smem[];
   const int n = g.n, lp = (n + S - 1) / S, tpw = 64 / lp;
@@ -130,7 +135,8 @@ __global__ void __launch_bounds__(64 * kWaves, S == 2 ? 2 : 1) sparse_step_kerne
     cpx<T>* gb = reinterpret_cast<cpx<T>*>(g.beta) + (size_t)b * n;
     const size_t poff = (size_t)(g.param_stride ? b : 0) * n;
     // c (rsl + i U (|b|^2 - 1)) = (A0 - Ui |b|^2) + i (B0 + Ur |b|^2), c i F = (fr, fi), c = cdt
-    T zr[S], zi[S], A0[S], B0[S], Ur[S], Ui[S], fr[S], fi[S];
+    constexpr int SF = FT ? 1 : S, SG = FT ? S : 1;
+    T zr[S], zi[S], A0[S], B0[S], Ur[S], Ui[S], fr[SF], fi[SF];
 #pragma unroll
     for (int s = 0; s < S; ++s) {
       const int j = q * S + s;
@@ -146,8 +152,10 @@ __global__ void __launch_bounds__(64 * kWaves, S == 2 ? 2 : 1) sparse_step_kerne
       B0[s] = cdt * (r.im - u.re);
       Ur[s] = cdt * u.re;
       Ui[s] = cdt * u.im;
-      fr[s] = -cdt * f.im;
-      fi[s] = cdt * f.re;
+      if constexpr (!FT) {
+        fr[s] = -cdt * f.im;
+        fi[s] = cdt * f.re;
+      }
     }
     T wr[S], wi[S];
     auto draw = [&](uint32_t step) __attribute__((always_inline)) {
@@ -168,7 +176,10 @@ __global__ void __launch_bounds__(64 * kWaves, S == 2 ? 2 : 1) sparse_step_kerne
     };
     constexpr bool kAhead = S == 2;  // the next step's noise beside this step's update
     if constexpr (kAhead) draw(uint32_t(g.step0));
+    // F(t): the interval of the step before and its ends, so that a step reads only the drive
     int ft_id = 0;
+    const double ft0 = FT ? g.ft_times[0] : 0.0;
+    double ft_lo = ft0, ft_hi = FT && g.ft_n > 1 ? g.ft_times[1] : HUGE_VAL;
     for (int st = 0; st < g.n_steps; ++st) {
       if (act) {
 #pragma unroll
@@ -182,24 +193,31 @@ __global__ void __launch_bounds__(64 * kWaves, S == 2 ? 2 : 1) sparse_step_kerne
         for (int m = 0; m < M; ++m) v[s][m] = ring[at[s][m]];
       wave_sync();
       T dr[S], di[S];
-      if (g.ft_n > 0) {
-        // F(t) before this step (TWMCLiebSolver.cpp:252-256), as c i F
-        const T fdt = T(drive_interval(g.ft_times, g.ft_n, g.t0 + double(st) * g.dt, ft_id));
+      // F(t) before this step (TWMCLiebSolver.cpp:252-256), as c i F
+      T gr[SG], gi[SG];
+      auto drive = [&]() __attribute__((always_inline)) {
+        const double t = g.t0 + double(st) * g.dt;
+        while (ft_hi < t) {
+          ++ft_id;
+          ft_lo = ft_hi;
+          ft_hi = ft_id + 1 < g.ft_n ? g.ft_times[ft_id + 1] : HUGE_VAL;
+        }
+        const T fdt = T(t <= ft0 ? 0.0 : t - ft_lo);
         const cpx<T>* fv = reinterpret_cast<const cpx<T>*>(g.ft_vals) + (size_t)ft_id * n;
         const cpx<T>* fs = reinterpret_cast<const cpx<T>*>(g.ft_slopes) + (size_t)ft_id * n;
 #pragma unroll
         for (int s = 0; s < S; ++s) {
           const int j = min(q * S + s, n - 1);
-          dr[s] = -cdt * fma(fdt, fs[j].im, fv[j].im);
-          di[s] = cdt * fma(fdt, fs[j].re, fv[j].re);
+          gr[s] = -cdt * fma(fdt, fs[j].im, fv[j].im);
+          gi[s] = cdt * fma(fdt, fs[j].re, fv[j].re);
         }
-      } else {
+      };
 #pragma unroll
-        for (int s = 0; s < S; ++s) {
-          dr[s] = fr[s];
-          di[s] = fi[s];
-        }
+      for (int s = 0; s < S; ++s) {
+        dr[s] = FT ? T(0) : fr[FT ? 0 : s];
+        di[s] = FT ? T(0) : fi[FT ? 0 : s];
       }
+      if constexpr (FT && kAhead) drive();
       T nr[S], ni[S];  // this step's noise
       if constexpr (kAhead) {
 #pragma unroll
@@ -217,6 +235,8 @@ __global__ void __launch_bounds__(64 * kWaves, S == 2 ? 2 : 1) sparse_step_kerne
           dr[s] = fma(cf[s][m], v[s][m].im, dr[s]);
           di[s] = fma(-cf[s][m], v[s][m].re, di[s]);
         }
+      // read here, beside the draw: the neighbours' registers are free by now
+      if constexpr (FT && !kAhead) drive();
       if constexpr (!kAhead) {
         draw(uint32_t(g.step0 + (uint64_t)st));
 #pragma unroll
@@ -229,6 +249,10 @@ __global__ void __launch_bounds__(64 * kWaves, S == 2 ? 2 : 1) sparse_step_kerne
       for (int s = 0; s < S; ++s) {
         const T x = zr[s], y = zi[s], mq = fma(y, y, x * x);
         const T cr = fma(-Ui[s], mq, A0[s]), ci = fma(Ur[s], mq, B0[s]);
+        if constexpr (FT) {
+          dr[s] += gr[s];
+          di[s] += gi[s];
+        }
         // increment = noise + dt iF + dt h + drift, all small, added to beta once
         const T ur = fma(-ci, y, fma(cr, x, dr[s])), ui = fma(ci, x, fma(cr, y, di[s]));
         zr[s] = x + (kScaled ? nr[s] + ur : fma(dt, ur, nr[s]));
@@ -243,21 +267,28 @@ __global__ void __launch_bounds__(64 * kWaves, S == 2 ? 2 : 1) sparse_step_kerne
   }
 }
 
-template <typename T, int S, bool PRIO>
+template <typename T, int S, bool PRIO, bool FT>
 const void* kernel_m(int m) {
-  return m <= 3 ? (const void*)sparse_step_kernel<T, S, 3, PRIO> : (const void*)sparse_step_kernel<T, S, 6, PRIO>;
+  return m <= 3 ? (const void*)sparse_step_kernel<T, S, 3, PRIO, FT> : (const void*)sparse_step_kernel<T, S, 6, PRIO, FT>;
 }
 
-template <typename T, bool PRIO>
+template <typename T, bool PRIO, bool FT>
 const void* kernel_s(int s, int m) {
-  return s == 2   ? kernel_m<T, 2, PRIO>(m)
-         : s == 4 ? kernel_m<T, 4, PRIO>(m)
-         : s == 6 ? kernel_m<T, 6, PRIO>(m)
-                  : kernel_m<T, 8, PRIO>(m);
+  return s == 2   ? kernel_m<T, 2, PRIO, FT>(m)
+         : s == 4 ? kernel_m<T, 4, PRIO, FT>(m)
+         : s == 6 ? kernel_m<T, 6, PRIO, FT>(m)
+                  : kernel_m<T, 8, PRIO, FT>(m);
 }
 
-const void* kernel_for(int precision, int s, int m, bool prio) {
-  return precision == 64 ? kernel_s<double, false>(s, m) : prio ? kernel_s<float, true>(s, m) : kernel_s<float, false>(s, m);
+template <bool FT>
+const void* kernel_ft(int precision, int s, int m, bool prio) {
+  return precision == 64 ? kernel_s<double, false, FT>(s, m)
+         : prio          ? kernel_s<float, true, FT>(s, m)
+                         : kernel_s<float, false, FT>(s, m);
+}
+
+const void* kernel_for(int precision, int s, int m, bool prio, bool ft) {
+  return ft ? kernel_ft<true>(precision, s, m, prio) : kernel_ft<false>(precision, s, m, prio);
 }
 
 size_t lds_bytes(int n, int precision, int s) {
@@ -280,7 +311,7 @@ bool sparse_supported(int n, int hopping, int most) {
 // of issue, a chain of 0.48 us; FP32 0.20 us, 0.08 + 0.23 us.  Few trajectories
 // give two sites per lane (the shortest chain), many the S that leaves the
 // fewest lanes and SIMDs without work.
-hipError_t sparse_plan(int n, int precision, int most, size_t n_traj, int cus, SparsePlan* plan) {
+hipError_t sparse_plan(int n, int precision, int most, bool ft, size_t n_traj, int cus, SparsePlan* plan) {
   double best = 0.0;
   plan->s = 0;
   for (int s : {2, 4, 6, 8}) {
@@ -289,7 +320,7 @@ hipError_t sparse_plan(int n, int precision, int most, size_t n_traj, int cus, S
     const size_t per_block = (size_t)kWaves * (64 / lp);
     const size_t blocks = (n_traj + per_block - 1) / per_block;
     const bool prio = blocks > 2 * (size_t)cus;
-    const void* f = kernel_for(precision, s, most, prio);
+    const void* f = kernel_for(precision, s, most, prio, ft);
     const size_t lds = lds_bytes(n, precision, s);
     if (lds > 65536) {
       hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
@@ -317,7 +348,7 @@ hipError_t sparse_plan(int n, int precision, int most, size_t n_traj, int cus, S
 }
 
 hipError_t launch_sparse(const StepArgs& a, int precision, const SparsePlan& plan, hipStream_t s) {
-  const void* f = kernel_for(precision, plan.s, a.ell_m, plan.prio);
+  const void* f = kernel_for(precision, plan.s, a.ell_m, plan.prio, a.ft_n > 0);
   if (plan.step.lds > 65536) {
     hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)plan.step.lds);
     if (e != hipSuccess) return e;

@@ -91,10 +91,13 @@ __global__ void __launch_bounds__(64 * kWaves, S == 2 ? 2 : 1) sparse_step_kerne
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const double* ltab = reinterpret_cast<const double*>(smem);
   constexpr int kTab = sizeof(T) == 8 ? f64::kTabSize * (int)sizeof(double) : 0;
-  if constexpr (sizeof(T) == 8) {
-    for (int i = threadIdx.x; i < f64::kTabSize; i += 64 * kWaves) reinterpret_cast<double*>(smem)[i] = kF64TabDev[i];
-    __syncthreads();
-  }
+  // the tables' loads run beside those of the coefficients below
+  constexpr int kTabLoads = f64::kTabSize / (64 * kWaves);
+  static_assert(kTabLoads * 64 * kWaves == f64::kTabSize, "whole rounds of the workgroup");
+  double tab[kTabLoads];
+  if constexpr (sizeof(T) == 8)
+#pragma unroll
+    for (int k = 0; k < kTabLoads; ++k) tab[k] = kF64TabDev[threadIdx.x + 64 * kWaves * k];
   f64::Series bmk = f64::kSeries;
   if constexpr (sizeof(T) == 8) f64::pin(bmk);
 
@@ -120,11 +123,18 @@ __global__ void __launch_bounds__(64 * kWaves, S == 2 ? 2 : 1) sparse_step_kerne
   for (int s = 0; s < S; ++s)
 #pragma unroll
     for (int m = 0; m < M; ++m) {
-      const int j = q * S + s;
-      const int i = j < n ? g.ell_row[j * M + m] : -1;
-      cf[s][m] = i >= 0 ? coef[j * M + m] : T(0);
-      at[s][m] = i >= 0 ? (i % S) * lp + i / S : S * lp;
+      const int j = q * S + s, e = min(j, n - 1) * M + m;
+      const int row = g.ell_row[e];
+      const T c = coef[e];
+      const bool bond = j < n && row >= 0;
+      cf[s][m] = bond ? c : T(0);
+      at[s][m] = bond ? (row % S) * lp + row / S : S * lp;
     }
+  if constexpr (sizeof(T) == 8) {
+#pragma unroll
+    for (int k = 0; k < kTabLoads; ++k) reinterpret_cast<double*>(smem)[threadIdx.x + 64 * kWaves * k] = tab[k];
+    __syncthreads();
+  }
 
   const int n_waves = gridDim.x * kWaves;
   for (int b0 = (blockIdx.x * kWaves + wave) * tpw; b0 < g.n_traj; b0 += n_waves * tpw) {

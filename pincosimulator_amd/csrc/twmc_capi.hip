@@ -144,7 +144,7 @@ struct Ctx {
   SparsePlan sparse;  // LDS kernel, matrix hopping: its steps on the sparse kernel
   bool band_dense = false;  // banded kernel: the batch's form (band_dense)
   int tb = 0;               // MFMA kernel: trajectories per workgroup
-  int group = 1;            // ahead kernel: most frames in one launch
+  int group = 1;            // ahead and sparse kernels: most frames in one launch
   int vary = 0;              // scan_vary and scan_u_real: the parameters are fixed
   bool u_is_real = false;
   bool ahead = false;       // LDS kernel: its steps on the ahead kernel
@@ -791,7 +791,7 @@ int read_states(Ctx* c, const void* src, size_t count, double* dst) {
   return TWMC_OK;
 }
 
-// Most frames that a launch of the ahead kernel takes: it stores the states of
+// Most frames that a launch of the ahead or sparse kernel takes: it stores the states of
 // several (into the trajectory output if it was asked for), whose sums one capture
 // and one reduction launch then form.  A frame of a small lattice is otherwise three
 // launches of which the steps are a small part (256 trajectories of 64 sites, FP64, 21
@@ -801,14 +801,15 @@ int read_states(Ctx* c, const void* src, size_t count, double* dst) {
 // within 64 MiB, its steps within 16384 (a few ms).
 void plan_group(Ctx* c, size_t B) {
   c->group = 1;
-  if (!c->ahead || !generic_capture_overwrites(c->n)) return;
+  // (F(t) is evaluated at the launch's first time plus the steps since: one launch a frame)
+  if (!(c->ahead || c->ell_m > 0) || c->ft_n > 0 || !generic_capture_overwrites(c->n)) return;
   const size_t state = B * c->n * c->es, sums = (size_t)c->grid * kQ * c->n * sizeof(double);
   const size_t most = std::min<size_t>({(size_t)c->n_frames, 64, 16384 / (size_t)c->p.frame_steps,
                                         (16u << 20) / state, (64u << 20) / sums});
   c->group = std::max<int>(1, (int)most);
 }
 
-// segments from k on that one launch of the ahead kernel can take: each stores a
+// segments from k on that one launch can take: each stores a
 // frame first, all but the last have the same number of steps
 int group_size(const Ctx* c, size_t k, uint64_t most) {
   if (c->group < 2) return 1;
@@ -837,7 +838,10 @@ int advance_group(Ctx* c, StepArgs a, int m, hipStream_t s) {
   a.capture = 0;
   hipEvent_t e0 = nullptr, r0 = nullptr;
   HIPCHK(c, timed(c, c->ev_step, s, true, e0));
-  HIPCHK(c, launch_ahead(a, c->precision, s));
+  if (c->ahead)
+    HIPCHK(c, launch_ahead(a, c->precision, s));
+  else
+    HIPCHK(c, launch_sparse(a, c->precision, c->sparse, s));
   HIPCHK(c, timed(c, c->ev_step, s, false, e0));
   c->stats.site_steps += (uint64_t)a.n_steps * (uint64_t)c->n * c->n_traj;
   HIPCHK(c, timed(c, c->ev_red, s, true, r0));

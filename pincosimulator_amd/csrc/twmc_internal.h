@@ -85,7 +85,7 @@ struct StepArgs {
   int np;                    // n padded to a multiple of 128
   int tb;                    // MFMA kernel: trajectories per workgroup
   unsigned int* queue;       // 64x64 stencil and nn kernels: work queue of the launch (one word), null: fixed shares
-  // several frames in one launch (ahead kernel, capture-only launch of the LDS kernel):
+  // several frames in one launch (ahead and sparse kernels, capture-only launch of the LDS kernel):
   // frame0 + k, k < group, lies at frames[trajectory][frames_stride][n]; the steps
   // store it after k group_steps steps
   void* frames;

@@ -190,7 +190,22 @@ __global__ void __launch_bounds__(64 * kWaves, S == 2 ? 2 : 1) sparse_step_kerne
     int ft_id = 0;
     const double ft0 = FT ? g.ft_times[0] : 0.0;
     double ft_lo = ft0, ft_hi = FT && g.ft_n > 1 ? g.ft_times[1] : HUGE_VAL;
+    int due = 0, frame = 0;  // steps to the next stored frame, frames stored
+    auto store_frame = [&] {
+      cpx<T>* out = reinterpret_cast<cpx<T>*>(g.frames) + ((size_t)b * g.frames_stride + g.frame0 + frame) * n;
+#pragma unroll
+      for (int s = 0; s < S; ++s) {
+        const int j = q * S + s;
+        if (live && j < n) out[j] = mk(zr[s], zi[s]);
+      }
+      ++frame;
+      due = g.group_steps;
+    };
     for (int st = 0; st < g.n_steps; ++st) {
+      if (due-- == 0 && frame < g.group) {
+        store_frame();
+        --due;
+      }
       if (act) {
 #pragma unroll
         for (int s = 0; s < S; ++s) ring[s * lp + q] = mk(zr[s], zi[s]);
@@ -269,6 +284,7 @@ __global__ void __launch_bounds__(64 * kWaves, S == 2 ? 2 : 1) sparse_step_kerne
         zi[s] = y + (kScaled ? ni[s] + ui : fma(dt, ui, ni[s]));
       }
     }
+    if (frame < g.group) store_frame();  // the state after the last step
 #pragma unroll
     for (int s = 0; s < S; ++s) {
       const int j = q * S + s;

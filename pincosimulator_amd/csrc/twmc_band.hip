@@ -228,7 +228,7 @@ __global__ void __launch_bounds__(64, UNI ? uni_waves(S, W, LIEB) : 1) band_step
 #pragma unroll
       for (int p = 0; p < S / 2; ++p) {
         const u32x4 ctr = make_counter(traj, TAG_WIENER, step, pbase + (uint32_t)p);
-        const u32x4 w = LIEB && !DENSE ? philox4x32_10(ctr, g.key0, g.key1) : philox4x32_10_wave(ctr, g.key0, g.key1);
+        const u32x4 w = DENSE || UNI ? philox4x32_10_wave(ctr, g.key0, g.key1) : philox4x32_10(ctr, g.key0, g.key1);
         float rn[2], cs[2], sn[2];
         if constexpr (PRIO) __builtin_amdgcn_s_setprio(2);
         box_muller_f32_scaled(w.x, w.y, nl, rn[0], cs[0], sn[0]);
@@ -264,7 +264,9 @@ __global__ void __launch_bounds__(64, UNI ? uni_waves(S, W, LIEB) : 1) band_step
 }
 
 // Bound by latency the uniform form gains where it saves most registers, four and more
-// sites per lane without padding (512 sites, W = 2, x 1000: 0.91 -> 0.88 us per step); for
+// sites per lane without padding (512 sites, W = 2, x 1000: 0.91 -> 0.88 us per step, the
+// Philox rounds with the trajectory's words in scalar registers; with parameters per site
+// those lengthen the chain, 384 x 64 0.60 -> 0.63); for
 // the Lieb chain and with padding to reset it loses (384 x 1500 0.98 / 1.05, 210 x 64
 // 0.42 / 0.45, 495 x 1000 0.90 / 0.94): those take the parameters per site.
 template <int S, int W, bool LIEB>

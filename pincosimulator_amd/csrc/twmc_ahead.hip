@@ -281,6 +281,18 @@ Launch launch_of(int precision, int n, int m, bool unif, bool xn) {
 
 }  // namespace
 
+// The lines below are those of long launches.  A workgroup first fills its tables and a
+// chunk of noise, one trajectory each, so where several share a CU a launch of few steps
+// costs more than the LDS and sparse kernels' (us of a launch, those kernels / this one:
+// FP64, 1x64, 2048 trajectories, 4 steps 9.7 / 12.4, 32 steps 23.4 / 22.8; FP32, 4096, 8
+// steps 9.5 / 14.3; FP64, 16x16, 512, 4 steps 10.3 / 13.4, 256 9.8 / 10.4, 16 steps 16.0 /
+// 13.9): half the batch below 64 steps, a quarter below 8.
+namespace {
+size_t batch_limit(int per_cu, uint64_t n_steps, int cus) {
+  return (size_t)per_cu * cus / (n_steps < 8 ? 4 : n_steps < 64 ? 2 : 1);
+}
+}  // namespace
+
 // A step costs the same for any batch until the CUs hold several workgroups; from
 // then on the LDS and nn kernels, whose waves are full, overtake it.  Measured, us per
 // step, those kernels against this one:
@@ -291,10 +303,10 @@ Launch launch_of(int precision, int n, int m, bool unif, bool xn) {
 //   FP32, 1x128, drawn F   256 trajectories 0.47 / 0.19, 4000 1.00 / 0.84
 //   FP64, 16x16  256 trajectories 0.67 / 0.42, 512 1.00 / 0.81, 1000 1.13 / 1.58
 //   FP32, 9x21   256 trajectories 0.50 / 0.36, 512 0.57 / 0.43, 2000 0.96 / 1.04
-bool ahead_pays(int nx, int ny, int precision, size_t n_traj, int cus) {
+bool ahead_pays(int nx, int ny, int precision, size_t n_traj, uint64_t n_steps, int cus) {
   const int n = nx * ny;
   const int per_cu = n > 128 ? 2 : precision == 32 ? 16 : n > 64 ? 4 : 8;
-  return ny > 1 && n <= 256 && n_traj <= (size_t)per_cu * cus;
+  return ny > 1 && n <= 256 && n_traj <= batch_limit(per_cu, n_steps, cus);
 }
 
 // The sparse kernel against this one, us per step, Lieb chains with drawn energies:
@@ -304,9 +316,9 @@ bool ahead_pays(int nx, int ny, int precision, size_t n_traj, int cus) {
 //   FP32, 72 sites   256 trajectories 0.33 / 0.18, 2000 0.47 / 0.35
 //   FP32, 144 sites  256 trajectories 0.54 / 0.31, 512 0.55 / 0.37, 1000 0.58 / 0.69
 //   FP32, 384 sites  256 trajectories 0.79 / 0.52, 512 0.80 / 1.00
-bool ahead_pays_sparse(int n, int most, int precision, size_t n_traj, int cus) {
+bool ahead_pays_sparse(int n, int most, int precision, size_t n_traj, uint64_t n_steps, int cus) {
   const int per_cu = n <= 128 ? 8 : n <= 256 || precision == 64 ? 2 : 1;
-  return (n <= 256 || (n <= 512 && most <= 3)) && n_traj <= (size_t)per_cu * cus;
+  return (n <= 256 || (n <= 512 && most <= 3)) && n_traj <= batch_limit(per_cu, n_steps, cus);
 }
 
 LaunchShape ahead_shape(int n, int ell_m, int precision, size_t n_traj) {

@@ -565,7 +565,8 @@ struct Geometry {
   bool nn = false;     // LDS kernel with FFT hopping: the step launch on the nn kernel
 };
 
-int step_geometry(Ctx* c, size_t B, Geometry& geo) {
+// n_steps: of a launch (of several frames, if it takes them).
+int step_geometry(Ctx* c, size_t B, uint64_t n_steps, Geometry& geo) {
   int cus = 0;
   HIPCHK(c, hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device));
   int per_cu = 1;
@@ -599,10 +600,10 @@ int step_geometry(Ctx* c, size_t B, Geometry& geo) {
     HIPCHK(c, generic_occupancy(c->precision, c->n, geo.block, geo.lds, &per_cu));
     if (c->ell_m > 0) {
       HIPCHK(c, sparse_plan(c->n, c->precision, c->ell_m, c->ft_n > 0, B, cus, &geo.sparse));
-      geo.ahead = c->ft_n == 0 && ahead_pays_sparse(c->n, c->ell_m, c->precision, B, cus);
+      geo.ahead = c->ft_n == 0 && ahead_pays_sparse(c->n, c->ell_m, c->precision, B, n_steps, cus);
     }
     if (c->kernel == TWMC_KERNEL_GENERIC && c->p.hopping == TWMC_HOP_FFT && c->ft_n == 0 &&
-        ahead_pays(c->p.nx, c->p.ny, c->precision, B, cus)) {
+        ahead_pays(c->p.nx, c->p.ny, c->precision, B, n_steps, cus)) {
       geo.ahead = true;
     } else if (c->p.hopping == TWMC_HOP_FFT && c->ft_n == 0 &&
         nn_supported(c->p.nx, c->p.ny, c->precision, c->vary) &&
@@ -1196,7 +1197,7 @@ int twmc_batch_begin(twmc_ctx* ctx, const twmc_batch_desc* d) {
   HIPCHK(c, hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device));
   {
     Geometry geo;
-    int rc = step_geometry(c, B, geo);
+    int rc = step_geometry(c, B, c->n_steps, geo);
     if (rc != TWMC_OK) return rc;
     c->grid = geo.grid;
     c->block = geo.block;
@@ -1578,7 +1579,7 @@ int twmc_advance_noalloc(twmc_ctx* ctx, const uint64_t* d_traj_ids, uint64_t n_t
   const int max_chunks =
       (int)std::min<size_t>(kSiteSumChunks, ((size_t)TWMC_NOALLOC_SCRATCH_BYTES - params) / per_chunk);
   Geometry geo;
-  int rc = step_geometry(c, n_traj, geo);
+  int rc = step_geometry(c, n_traj, n_steps, geo);
   if (rc != TWMC_OK) return rc;
   hipStream_t s = stream ? static_cast<hipStream_t>(stream) : c->stream;
   void* rsl = base;

@@ -285,10 +285,11 @@ hipError_t nn_occupancy(int nx, int ny, int precision, int vary, bool u_real, in
 hipError_t launch_nn(const StepArgs& a, int precision, int grid, hipStream_t s);
 
 // FFT hopping, up to 256 sites, static parameters: the step launch of the LDS kernel
-// (TWMC_KERNEL_GENERIC) for small batches, one workgroup per trajectory
-bool ahead_pays(int nx, int ny, int precision, size_t n_traj, int cus);
+// (TWMC_KERNEL_GENERIC) for small batches, one workgroup per trajectory; n_steps: of
+// the launch
+bool ahead_pays(int nx, int ny, int precision, size_t n_traj, uint64_t n_steps, int cus);
 // matrix hopping with few nonzeros per column, up to 512 sites, static parameters: the same
-bool ahead_pays_sparse(int n, int most, int precision, size_t n_traj, int cus);
+bool ahead_pays_sparse(int n, int most, int precision, size_t n_traj, uint64_t n_steps, int cus);
 // ell_m: StepArgs::ell_m, 0: FFT hopping
 LaunchShape ahead_shape(int n, int ell_m, int precision, size_t n_traj);
 hipError_t launch_ahead(const StepArgs& a, int precision, hipStream_t s);

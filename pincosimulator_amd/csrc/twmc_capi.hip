@@ -565,7 +565,8 @@ struct Geometry {
   bool nn = false;     // LDS kernel with FFT hopping: the step launch on the nn kernel
 };
 
-// n_steps: of a launch (of several frames, if it takes them).
+// n_steps: of the launch; of a batch that stores frames UINT64_MAX, as the ahead kernel
+// takes several in a launch.
 int step_geometry(Ctx* c, size_t B, uint64_t n_steps, Geometry& geo) {
   int cus = 0;
   HIPCHK(c, hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device));
@@ -1197,7 +1198,7 @@ int twmc_batch_begin(twmc_ctx* ctx, const twmc_batch_desc* d) {
   HIPCHK(c, hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device));
   {
     Geometry geo;
-    int rc = step_geometry(c, B, c->n_steps, geo);
+    int rc = step_geometry(c, B, UINT64_MAX, geo);
     if (rc != TWMC_OK) return rc;
     c->grid = geo.grid;
     c->block = geo.block;

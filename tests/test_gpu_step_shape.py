@@ -33,12 +33,10 @@ def drawn(**kw):
 
 @pytest.mark.parametrize("precision,nx,ny,per_cu", [(64, 4, 4, 8), (64, 5, 13, 4), (64, 16, 16, 2), (32, 1, 64, 16),
                                                     (32, 9, 21, 2)])
-@pytest.mark.parametrize("steps,part", [(64, 1), (63, 2), (8, 2), (7, 4), (1, 4)])
-def test_ahead_line(precision, nx, ny, per_cu, steps, part):
-    line = per_cu * torch.cuda.get_device_properties(0).multi_processor_count // part
-    print(f"{nx}x{ny}, FP{precision}, {steps} steps", flush=True)
-    spec = lattice(nx, ny, frame_steps=steps, t_end=0.005 * (steps + 0.25))
-    few, many = (shape(spec, b, precision) for b in (line, line + 1))
+def test_ahead_line(precision, nx, ny, per_cu):
+    line = per_cu * torch.cuda.get_device_properties(0).multi_processor_count
+    print(f"{nx}x{ny}, FP{precision}", flush=True)
+    few, many = (shape(lattice(nx, ny), b, precision) for b in (line, line + 1))
     n = nx * ny
     assert few[:2] == (line, 256 if n <= 128 else 512)
     assert many[1] == (64 if n <= 128 else 128)
@@ -68,7 +66,7 @@ def test_nn_fp32(nx, ny, kw, block):
 
 def test_matrix_and_stacked():
     cus = torch.cuda.get_device_properties(0).multi_processor_count
-    spec = spec_of(sparse_matrix(72, 3, 5), frame_steps=64, t_end=0.005 * 64.25)
+    spec = spec_of(sparse_matrix(72, 3, 5), frame_steps=3, t_end=0.005 * 3.25)
     assert shape(spec, 8 * cus, 64)[:2] == (8 * cus, 256)
     sparse = shape(spec, 8 * cus + 1, 64)
     assert sparse[0] <= (8 * cus + 4) // 4 and sparse[1] == 256

@@ -166,9 +166,9 @@ typedef struct twmc_stats {
   double reduce_kernel_ms;
   uint64_t reduce_launches;
   int32_t kernel;            /* kernel used by the last batch */
-  int32_t grid;              /* workgroups of the step kernel */
-  int32_t block;             /* threads per workgroup */
-  int32_t lds_bytes;         /* dynamic LDS per workgroup */
+  int32_t grid;              /* workgroups of the step launch, on whichever kernel the batch steps */
+  int32_t block;             /* threads per workgroup of it */
+  int32_t lds_bytes;         /* dynamic LDS per workgroup of it */
 } twmc_stats;
 
 int twmc_abi_version(void);
@@ -188,8 +188,9 @@ int twmc_set_timing(twmc_ctx* ctx, int enable);   /* HIP events around step laun
 int twmc_query(twmc_ctx* ctx, twmc_stats* st);
 int twmc_reset_stats(twmc_ctx* ctx);
 /* fraction of the current batch's steps the device has completed (an event
- * after each segment, polled without blocking); any thread may call it while
- * the owning thread advances or reads the batch */
+ * after each segment, polled without blocking; where one launch takes several
+ * frames of a small batch, up to 64 and 16384 steps, they complete together);
+ * any thread may call it while the owning thread advances or reads the batch */
 float twmc_progress(const twmc_ctx* ctx);
 
 /* ---- allocation-free stepping --------------------------------------------
@@ -209,7 +210,7 @@ float twmc_progress(const twmc_ctx* ctx);
  * Asynchronous; no host synchronisation.  Site-shared parameters and a static
  * drive only, on the context's kernel (the stacked kernel excepted: create
  * such a context with TWMC_KERNEL_GENERIC).  Its own device memory -- the
- * parameter tables and the partial sums -- is one fixed array of
+ * parameter tables, a work queue and the partial sums -- is one fixed array of
  * TWMC_NOALLOC_SCRATCH_BYTES held by every GPU the library runs on until the
  * process ends; a lattice whose tables and one partial slot exceed it is
  * rejected.  Every call on one GPU shares that array, so calls that overlap

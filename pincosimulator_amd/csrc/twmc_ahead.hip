@@ -2,7 +2,7 @@
 // up to 256 sites, the hopping in its nearest-neighbour form (the exact real-space form
 // of the reference's FFT product, TWMCBaseSolver.cpp:80-88, :235-242), and matrix
 // hopping with few nonzeros per column (TWMCLiebSolver.cpp:259-267), up to 256 sites with
-// six, 512 with three.
+// six, 512 with three (above 256, FP64, 16 values spill).
 //
 // What bounds it: the latency of one step after the other; the chip is mostly idle.
 // In the LDS kernel (twmc_generic.hip) and the sparse kernel (twmc_sparse.hip) a wave's

@@ -73,7 +73,8 @@ __host__ __device__ constexpr bool lieb_bond(int r, int d) {
 // of a step: DPP and no priority (384 sites x 1000: 0.57 against 0.68 us).
 // Before, 99 registers and the latency form for all: 384 sites x 8192 3.69, x
 // 16384 7.16 us per step (8.8e11 -> 1.03e12 site-steps/s).
-// waves per SIMD that the uniform form's registers allow without spills
+// waves per SIMD that the uniform form's registers allow with at most three spilled (six
+// sites per lane and DENSE: two in the Lieb form and W = 1, three in W = 3)
 constexpr int uni_waves(int s, int w, bool lieb) {
   return s == 2 || lieb ? 8 : s == 4 ? (w <= 2 ? 7 : 6) : s == 6 ? (w == 1 ? 7 : 5) : w == 1 ? 5 : 4;
 }

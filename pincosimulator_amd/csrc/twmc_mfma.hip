@@ -64,7 +64,10 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 // 2 QG TPW site pairs per step, one for every 2 / QG k blocks, whose MFMAs carry that
 // pair's Philox draw, Box-Muller and drift/drive terms (fenced pieces); after
 // the GEMM only dt h is added.  A wave whose rows all lie past the lattice only keeps
-// the barriers; k blocks past it are left out, if there are any (FULL: none).
+// the barriers; k blocks past it are left out, if there are any.  FULL: no such test, for
+// lattices whose k blocks fill np, and for np = 512, where 385 to 480 sites step their
+// zeros along.  Two of the forms at np = 384 spill with 32 trajectories: FULL one value,
+// the other (257 to 352 sites) 13.
 template <int TPW, int QG, bool FULL, bool CAPTURE_ONLY>
 __global__ void __launch_bounds__(512, 1) mfma_step_kernel(StepArgs g) {
   extern __shared__ __align__(16) unsigned char smem[];

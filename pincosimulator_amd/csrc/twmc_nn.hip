@@ -19,7 +19,8 @@
 //    per pair, and conflict about threefold in the LDS banks (up to 2048 sites a copy of
 //    the kernel reading one row was 11% faster).
 //  * Odd rows: the LDS kernel forms each site's neighbour places, a division among
-//    them, in every step; here they are formed once and held.  8192 trajectories, FP32
+//    them, in every step; here they are formed once and held (uniform, FP64, above 2048
+//    sites, eleven values spill).  8192 trajectories, FP32
 //    40x41 35.3 -> 19.6, 63x63 73.9 -> 42.7; FP64 40x41 75.0 -> 50.3, 63x63 136 -> 103.
 //  * A varying parameter: the LDS kernel reads rsl, U and F of every site from memory
 //    in every step (64x64, FP32: 98 KB a step and trajectory, 7.4 TB/s); here the one

@@ -38,7 +38,8 @@ constexpr int kL = 64;
 //
 // What bounds it: VALU issue, 44.5 instructions per site-step of which the four
 // transcendental ones run on their own unit beside the others when other waves
-// have work: 64 registers for eight waves per SIMD, two workgroups per CU.  The
+// have work: 64 registers for eight waves per SIMD (two values spill with a real U),
+// two workgroups per CU.  The
 // two do not advance evenly (the older one is served first), so in launches of more
 // than a few steps (queue_pays) trajectories are taken from a queue: dealt out by
 // workgroup, one of the two finished early and left the other to a half-filled CU.  16384 trajectories, 500-step launches:

@@ -235,7 +235,8 @@ __device__ __forceinline__ void step_item(const SweepArgs& g, const SweepPointDe
 
 // The step launch: 1024-thread workgroups, up to two site pairs per thread, 64
 // registers for eight waves per SIMD (the transcendental instructions then run
-// beside the others, as in the 64x64 kernel).
+// beside the others, as in the 64x64 kernel); ten values spill, thirteen with a
+// complex U.
 // Bound by VALU issue: 45.6 instructions per site-step (2D; chains 43.5), four of
 // them transcendental.  A 512-point sweep frame 35.8 -> 32.3 ms against 256-thread
 // workgroups of up to eight pairs per thread (168 registers, three waves per
